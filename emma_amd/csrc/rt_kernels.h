@@ -264,6 +264,41 @@ struct TileLds {
   int item_nei[kTileWaves][kHaloCap];
 };
 
+// LDS of one tile of the cell kernel: one photon group's state and closure of
+// the tile's cells, then the halo slots of each wave (component-major, so that
+// a wave's accesses are consecutive)
+template <typename R>
+struct CellLds {
+  static constexpr int kHaloCap = 64;
+  static constexpr int kSlots = kTileCells + kTileWaves * kHaloCap;
+  R v[9][kSlots];  // e, fx, fy, fz, the closure's diag, arg, n
+  unsigned char cancel[kSlots];  // 1: the flux from this neighbour is dropped
+  unsigned char item[kTileWaves][kHaloCap];  // listed halo: slot -> lane*4 + direction
+  int item_nei[kTileWaves][kHaloCap];        // and the face's nei_oct entry
+  __device__ __forceinline__ void put(int i, R e, R fx, R fy, R fz, const Closure<R>& q) {
+    v[0][i] = e;
+    v[1][i] = fx;
+    v[2][i] = fy;
+    v[3][i] = fz;
+    v[4][i] = q.diag;
+    v[5][i] = q.arg;
+    v[6][i] = q.n[0];
+    v[7][i] = q.n[1];
+    v[8][i] = q.n[2];
+  }
+  __device__ __forceinline__ void get(int i, R& e, R& fx, R& fy, R& fz, Closure<R>& q) const {
+    e = v[0][i];
+    fx = v[1][i];
+    fy = v[2][i];
+    fz = v[3][i];
+    q.diag = v[4][i];
+    q.arg = v[5][i];
+    q.n[0] = v[6][i];
+    q.n[1] = v[7][i];
+    q.n[2] = v[8][i];
+  }
+};
+
 // one level step of the schedule: its arguments, FillRad's block before it
 // and the hydro injection after it (fill / hydro: 0 = skip)
 template <typename R>

@@ -140,9 +140,12 @@ __device__ __forceinline__ T gld_in(const T* base, int i) {
     return gld(base, i);
 }
 
-template <typename T>
-__device__ __forceinline__ T sel(int i, T a, T b, T c) {
-  return i == 0 ? a : (i == 1 ? b : c);
+template <typename R, bool Fast>
+__device__ __forceinline__ Closure<R> closure_of(R fx, R fy, R fz, R ee, R c) {
+  if constexpr (Fast)
+    return closure_fast(fx, fy, fz, ee, c);
+  else
+    return closure<R>(fx, fy, fz, ee, c);
 }
 
 // The level-step kernels take (LevelArgs, ChemConst) by value but read them
@@ -237,73 +240,78 @@ __device__ __forceinline__ void reflux(const LevelArgs<R>& a, int p, int q, int 
   atomicAdd(acc + 3 * GA + g, F[3] * dts * w * R(0.125));
 }
 
-// leaf cell after its fluxes: base state (+ refluxes from the finer level),
-// update, N<0/NaN guard, chemistry, write of the next state.  Returns the
-// accepted chemistry sub-steps.
-// The chemistry inputs (src, x n_H, eint, n_H) come from memory, or from
-// `pre` when the caller loaded them early (pre_src[GA], pre[3]).
-template <typename R, int G, bool Fast, int Sub, bool NT = false>
-__device__ __forceinline__ int finish_leaf(const LevelArgs<R>& a, const ChemConst& K, int cell, int ch, int ng,
-                                           R* Ue, R* Ux, R* Uy, R* Uz, const R* De, const R* Dx, const R* Dy,
-                                           const R* Dz, const R* pre_src = nullptr, const double* pre = nullptr) {
-  constexpr int GA = G > 0 ? G : kMaxGrp;
-  const int n = a.ncell;
-  if (ch <= -2) {  // the refluxes of the finer octs behind its faces, in pair order
-    const int code = -2 - ch;
-    R* acc = a.racc + (size_t)(code >> 3) * Sub * 4 * GA;
-    const int m = (code & 7) * Sub;
-    // all loads before the clearing stores.  A leaf has at most six pairs:
-    // the tiled kernel's loop unrolls, and its loads (an accumulator's 4G
-    // values are contiguous), clamped to the leaf's last accumulator, go out
-    // together instead of one pair after another
-    constexpr int kMaxSub = 6 * Sub;
-    R s[GA][4];
+// the refluxes of the finer octs behind a leaf's faces, added to its base
+// state in pair order; their accumulators are cleared.  Sub: accumulators per
+// pair, GA: groups an accumulator holds, groups [g0, g0 + NG) are taken.
+template <typename R, int GA, int NG, int Sub>
+__device__ __forceinline__ void fold_reflux(const LevelArgs<R>& a, int ch, int g0, int ng, R* Ue, R* Ux, R* Uy, R* Uz) {
+  const int code = -2 - ch;
+  R* acc = a.racc + (size_t)(code >> 3) * Sub * 4 * GA + g0;
+  const int m = (code & 7) * Sub;
+  // all loads before the clearing stores.  A leaf has at most six pairs:
+  // the tiled kernel's loop unrolls, and its loads (an accumulator's 4G
+  // values are contiguous), clamped to the leaf's last accumulator, go out
+  // together instead of one pair after another
+  constexpr int kMaxSub = 6 * Sub;
+  R s[NG][4];
 #pragma unroll
-    for (int g = 0; g < GA; g++) s[g][0] = s[g][1] = s[g][2] = s[g][3] = R(0);
+  for (int g = 0; g < NG; g++) s[g][0] = s[g][1] = s[g][2] = s[g][3] = R(0);
 #pragma unroll(Sub == 1 ? kMaxSub : 1)
-    for (int i = 0; i < (Sub == 1 ? kMaxSub : m); i++) {
-      const R* p = acc + (size_t)min(i, m - 1) * 4 * GA;
+  for (int i = 0; i < (Sub == 1 ? kMaxSub : m); i++) {
+    const R* p = acc + (size_t)min(i, m - 1) * 4 * GA;
 #pragma unroll
-      for (int v = 0; v < 4; v++) {
+    for (int v = 0; v < 4; v++) {
 #pragma unroll
-        for (int g = 0; g < GA; g++) {
-          if (g < ng) {
-            const R x = p[v * GA + g];
-            s[g][v] += i < m ? x : R(0);
-          }
+      for (int g = 0; g < NG; g++) {
+        if (g < ng) {
+          const R x = p[v * GA + g];
+          s[g][v] += i < m ? x : R(0);
         }
-      }
-    }
-#pragma unroll(Sub == 1 ? kMaxSub : 1)
-    for (int i = 0; i < kMaxSub; i++) {
-      if (i < m) {
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-#pragma unroll
-          for (int g = 0; g < GA; g++)
-            if (g < ng) acc[(size_t)i * 4 * GA + v * GA + g] = R(0);
-        }
-      }
-    }
-#pragma unroll
-    for (int g = 0; g < GA; g++) {
-      if (g < ng) {
-        Ue[g] += s[g][0];
-        Ux[g] += s[g][1];
-        Uy[g] += s[g][2];
-        Uz[g] += s[g][3];
       }
     }
   }
+#pragma unroll(Sub == 1 ? kMaxSub : 1)
+  for (int i = 0; i < kMaxSub; i++) {
+    if (i < m) {
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+#pragma unroll
+        for (int g = 0; g < NG; g++)
+          if (g < ng) acc[(size_t)i * 4 * GA + v * GA + g] = R(0);
+      }
+    }
+  }
+#pragma unroll
+  for (int g = 0; g < NG; g++) {
+    if (g < ng) {
+      Ue[g] += s[g][0];
+      Ux[g] += s[g][1];
+      Uy[g] += s[g][2];
+      Uz[g] += s[g][3];
+    }
+  }
+}
+
+// leaf cell after its transport (T: the updated state): N<0/NaN guard,
+// chemistry, write of the next state.  Returns the accepted chemistry
+// sub-steps.
+// The chemistry inputs (src, x n_H, eint, n_H) come from memory, or from
+// `pre` when the caller loaded them early (pre_src[GA], pre[3]).
+template <typename R, int G, bool Fast, int Sub, bool NT = false>
+__device__ __forceinline__ int finish_leaf(const LevelArgs<R>& a, const ChemConst& K, int cell, int ng, const R* Te,
+                                           const R* Tx, const R* Ty, const R* Tz, const R* pre_src = nullptr,
+                                           const double* pre = nullptr) {
+  constexpr int GA = G > 0 ? G : kMaxGrp;
+  const int n = a.ncell;
   double e[GA], src[GA];
   R fx[GA], fy[GA], fz[GA];  // fluxes after transport, in the storage type
 #pragma unroll
   for (int g = 0; g < GA; g++) {
     if (g < ng) {
-      e[g] = (double)(R)(Ue[g] + De[g]);
-      fx[g] = Ux[g] + Dx[g];
-      fy[g] = Uy[g] + Dy[g];
-      fz[g] = Uz[g] + Dz[g];
+      e[g] = (double)Te[g];
+      fx[g] = Tx[g];
+      fy[g] = Ty[g];
+      fz[g] = Tz[g];
       src[g] = (double)(pre_src != nullptr ? pre_src[g] : gld(a.src + g * n, cell));
     }
   }
@@ -397,21 +405,20 @@ __device__ __forceinline__ int finish_leaf(const LevelArgs<R>& a, const ChemCons
 // state (updatefieldrad without the split test, rad_utils.c:1548-1552) and
 // keeps x, eint, T (chemrad skips it)
 template <typename R, int GA>
-__device__ __forceinline__ void transport_split_cell(const LevelArgs<R>& a, int cell, int ng, const R* Ue, const R* Ux,
-                                                     const R* Uy, const R* Uz, const R* De, const R* Dx, const R* Dy,
-                                                     const R* Dz) {
+__device__ __forceinline__ void transport_split_cell(const LevelArgs<R>& a, int cell, int ng, const R* Te, const R* Tx,
+                                                     const R* Ty, const R* Tz) {
   const int n = a.ncell;
 #pragma unroll
   for (int g = 0; g < GA; g++) {
     if (g < ng) {
-      gst(a.eo + g * n, cell, Ue[g] + De[g]);
-      gst(a.fxo + g * n, cell, Ux[g] + Dx[g]);
-      gst(a.fyo + g * n, cell, Uy[g] + Dy[g]);
-      gst(a.fzo + g * n, cell, Uz[g] + Dz[g]);
+      gst(a.eo + g * n, cell, Te[g]);
+      gst(a.fxo + g * n, cell, Tx[g]);
+      gst(a.fyo + g * n, cell, Ty[g]);
+      gst(a.fzo + g * n, cell, Tz[g]);
     }
   }
-  const double e0 = (double)(R)(Ue[0] + De[0]);
-  const double e1 = ng > 1 ? (double)(R)(Ue[1 < GA ? 1 : 0] + De[1 < GA ? 1 : 0]) : (double)(R)(Ux[0] + Dx[0]);
+  const double e0 = (double)Te[0];
+  const double e1 = ng > 1 ? (double)Te[1 < GA ? 1 : 0] : (double)Tx[0];
   if (e0 < 0 || isnan(e0) || isnan(e1)) raise_status(a.status, -3, a.level, cell);
   gst(a.nhpluso, cell, gld(a.nhplus, cell));
   gst(a.einto, cell, gld(a.eint, cell));
@@ -451,8 +458,9 @@ __device__ __forceinline__ void block_counters(unsigned long long* counters, uns
 
 // ------------------------------------------------------------------ level step
 // One thread per cell; neighbours straight from global memory.  Fast selects
-// the mixed-precision physics (rt_physics_fast.h); the FP64 kernel
-// (Fast = false) keeps the reference's operation order.
+// the mixed-precision physics (rt_physics_fast.h); FP64 (Fast = false) keeps
+// the reference's operation order.  The persistent kernel's per-cell items;
+// the per-level launches run cell_step_lds below.
 // The cells of block `block` (256 consecutive cells, 32 octs).
 template <typename R, int G, bool Fast>
 __device__ __forceinline__ void cell_step(const LevelArgs<R>& a, const ChemConst& K, int block, int lc) {
@@ -555,22 +563,253 @@ __device__ __forceinline__ void cell_step(const LevelArgs<R>& a, const ChemConst
           }
         }
       }
+      if (ch <= -2) fold_reflux<R, GA, GA, kRefluxCell>(a, ch, 0, ng, Ue, Ux, Uy, Uz);
+#pragma unroll
+      for (int g = 0; g < GA; g++) {
+        if (g < ng) {
+          Ue[g] += De[g];
+          Ux[g] += Dx[g];
+          Uy[g] += Dy[g];
+          Uz[g] += Dz[g];
+        }
+      }
       if (ch >= 0) {
-        transport_split_cell<R, GA>(a, cell, ng, Ue, Ux, Uy, Uz, De, Dx, Dy, Dz);
+        transport_split_cell<R, GA>(a, cell, ng, Ue, Ux, Uy, Uz);
       } else {
         leaf = 1;
-        nit_acc =
-            (unsigned)finish_leaf<R, G, Fast, kRefluxCell>(a, K, cell, ch, ng, Ue, Ux, Uy, Uz, De, Dx, Dy, Dz);
+        nit_acc = (unsigned)finish_leaf<R, G, Fast, kRefluxCell>(a, K, cell, ng, Ue, Ux, Uy, Uz);
       }
     }
   }
   if (a.counters != nullptr) block_counters<4>(a.counters, nit_acc, leaf);
 }
 
+// The same step with every closure computed once.  FP64 with any group count
+// and mixed precision with other than 1 or 3 groups; the operations and their
+// order are those of cell_step, so the results are the same bit for bit.
+//
+// cell_step is bound by its FP64 instructions: seven closures per cell and
+// group (its own and six neighbours', five divisions and two square roots
+// each) where two are enough.  Here a 256-thread work-group owns 32
+// consecutive octs, one cell per thread, and takes one photon group at a time:
+// each cell's state and closure go to LDS once, neighbours in the tile are read
+// from there, and only the halo (a third to a half of the leaving faces on a
+// complete level) is evaluated again: on complete levels (variant kListed) one
+// listed halo face per lane in one round, on sparse ones each lane its own
+// leaving face in each direction pass.  One group at a time keeps the LDS at
+// 37 KB (FP64; 18 KB FP32) whatever the group count, and only the transported
+// state of the other groups live across the passes.
+template <typename R>
+__device__ __forceinline__ CellLds<R>* cell_lds() {
+  __shared__ CellLds<R> lds;
+  return &lds;
+}
+
 template <typename R, int G, bool Fast>
-__global__ __launch_bounds__(256) void level_step_kernel(LevelArgs<R> a_by_value, ChemConst K_by_value) {
+__device__ __forceinline__ void cell_step_lds(const LevelArgs<R>& a, const ChemConst& K, int tile, int lc,
+                                              CellLds<R>& lds) {
+  constexpr int GA = (G == 1 || G == 3) ? G : kMaxGrp;  // groups of a reflux accumulator
+  const int n = a.ncell;
+  const int wv = lc >> 6, lane = lc & 63;
+  const int cell = tile * kTileCells + lc;
+  const int oct0 = tile * kTileOcts;
+  const int oct = cell >> 3, ic = cell & 7;
+  const bool valid = cell < n;
+  const bool transport = a.transport != 0;
+  const bool listed = a.variant == kListed;
+  const R c = a.c, hc = a.hc, dts = a.dtsurdx;
+  int ch = -1;
+  int noD[3] = {0, 0, 0};  // nei_oct entry of the face that leaves the oct, per direction
+  if (valid) {
+    ch = gld(a.child, cell);
+    if (transport) {
+#pragma unroll
+      for (int d = 0; d < 3; d++) noD[d] = gld(a.nei, oct * 6 + 2 * d + ((ic >> d) & 1));
+    }
+  }
+  const bool restricted = ch >= 0 && !a.update_split;  // takes its children's mean, no transport
+  const bool moves = valid && transport && !restricted;
+  auto in_tile = [&](int no) { return no >= oct0 && no < oct0 + kTileOcts; };
+  int hbase[3] = {0, 0, 0}, nhalo = 0;
+  unsigned long long hball[3] = {0ull, 0ull, 0ull};
+  if (transport) {
+    lds.cancel[lc] = (unsigned char)(ch >= 0 && !a.keep_split_flux);
+    if (listed) {
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        const bool out = moves && !in_tile(noD[d]);
+        hball[d] = __ballot(out);
+        hbase[d] = nhalo;
+        nhalo += __popcll(hball[d]);
+        if (out) {
+          const int slot = hbase[d] + lanes_below_mask(hball[d]);  // < kHaloCap (variant chosen from the topology)
+          lds.item[wv][slot] = (unsigned char)(lane * 4 + d);
+          lds.item_nei[wv][slot] = noD[d];
+        }
+      }
+      // the list is written and read by lanes of the same wave
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+  }
+  // the halo face in direction d of cell hcell, nei_oct entry no: where its
+  // neighbour's state lies
+  struct Halo {
+    int j, d;
+    bool on, coarse, refl;
+  };
+  auto halo_of = [&](bool on, int hcell, int d, int no) {
+    Halo h;
+    const int hic = hcell & 7, side = (hic >> d) & 1;
+    const bool bound = on && no <= kNeiReflective;  // domain face (rad_utils.c:1106-1213, 1376-1407)
+    h.on = on;
+    h.d = d;
+    h.coarse = on && no < 0 && !bound;
+    h.refl = bound && no == kNeiReflective;
+    h.j = !on ? 0
+              : bound ? (hcell & ~7) + trans_source(2 * d + side, hic)
+                      : h.coarse ? -1 - no : no * 8 + (hic ^ (1 << d));
+    return h;
+  };
+  // its cancel flag (the flux from a split neighbour is dropped, RADSTEP)
+  auto halo_cancel = [&](const Halo& h) {
+    return h.on && !h.coarse && !a.keep_split_flux && gld(a.child, h.j) >= 0;
+  };
+  // group g of its state into LDS slot i, with its closure
+  auto halo_put = [&](const Halo& h, int g, int i) {
+    if (!h.on) return;
+    const size_t o = (size_t)g * (size_t)(h.coarse ? a.ncoarse : n) + (size_t)h.j;
+    const R ve = (h.coarse ? a.ce : a.e)[o];
+    R vx = (h.coarse ? a.cfx : a.fx)[o], vy = (h.coarse ? a.cfy : a.fy)[o], vz = (h.coarse ? a.cfz : a.fz)[o];
+    if (h.refl) {
+      if (h.d == 0) vx = -vx;
+      if (h.d == 1) vy = -vy;
+      if (h.d == 2) vz = -vz;
+    }
+    lds.put(i, ve, vx, vy, vz, closure_of<R, Fast>(vx, vy, vz, ve, c));
+  };
+  const int hslot0 = kTileCells + wv * CellLds<R>::kHaloCap;
+  Halo hl;  // listed: this lane's entry of the wave's list
+  if (transport && listed) {
+    const int it = lds.item[wv][lane];
+    hl = halo_of(lane < nhalo, (cell & ~63) + (it >> 2), it & 3, lds.item_nei[wv][lane]);
+    lds.cancel[hslot0 + lane] = (unsigned char)halo_cancel(hl);
+  }
+  R Te[G], Tx[G], Ty[G], Tz[G];  // the transported state
+#pragma unroll
+  for (int g = 0; g < G; g++) {
+    if (valid) {
+      Te[g] = gld(a.e + (size_t)g * n, cell);
+      Tx[g] = gld(a.fx + (size_t)g * n, cell);
+      Ty[g] = gld(a.fy + (size_t)g * n, cell);
+      Tz[g] = gld(a.fz + (size_t)g * n, cell);
+    }
+  }
+  if (transport) {
+    // the flux from a neighbour is multiplied by 0 or 1 (rad_utils.c:518-526)
+    R keepm[3], keepp[3];
+    int pairD[3] = {-1, -1, -1};  // reflux pair of a leaving face with a coarse leaf behind it
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+      const R ue = Te[g], ux = Tx[g], uy = Ty[g], uz = Tz[g];
+      Closure<R> Q;
+      if (valid) {
+        Q = closure_of<R, Fast>(ux, uy, uz, ue, c);
+        lds.put(lc, ue, ux, uy, uz, Q);
+      }
+      if (listed) halo_put(hl, g, hslot0 + lane);
+      __syncthreads();
+      if (moves) {
+        R De = R(0), Dx = R(0), Dy = R(0), Dz = R(0);
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+          // one face in d lies inside the oct and one leaves it; bit says
+          // which is which (bit 1: the minus face is the inside one)
+          const int bit = (ic >> d) & 1, jin = lc ^ (1 << d);
+          const bool inT = in_tile(noD[d]);
+          const int jl = (int)(((unsigned)noD[d] - (unsigned)oct0) * 8u + (unsigned)(ic ^ (1 << d)));
+          const int slot = listed ? hbase[d] + lanes_below_mask(hball[d]) : lane;
+          const int jout = inT ? jl : hslot0 + slot;
+          if (!listed && !inT) {  // this lane's own slot: written and read by it alone
+            const Halo h = halo_of(true, cell, d, noD[d]);
+            if (g == 0) lds.cancel[jout] = (unsigned char)halo_cancel(h);
+            halo_put(h, g, jout);
+          }
+          if (g == 0) {
+            const bool cin = lds.cancel[jin] != 0, cout = lds.cancel[jout] != 0;
+            keepm[d] = (bit ? cin : cout) ? R(0) : R(1);
+            keepp[d] = (bit ? cout : cin) ? R(0) : R(1);
+            if (!inT && noD[d] < 0 && noD[d] > kNeiReflective) pairD[d] = gld(a.rpair, oct * 6 + 2 * d + bit);
+          }
+          const int jm = bit ? jin : jout, jp = bit ? jout : jin;
+          R Fm[4], Fp[4], ve, vx, vy, vz;
+          Closure<R> qv;
+          lds.get(jm, ve, vx, vy, vz, qv);
+          lf_flux<R>(d, 0, ue, ux, uy, uz, Q, ve, vx, vy, vz, qv, hc, Fm);
+          lds.get(jp, ve, vx, vy, vz, qv);
+          lf_flux<R>(d, 1, ue, ux, uy, uz, Q, ve, vx, vy, vz, qv, hc, Fp);
+#pragma unroll
+          for (int v = 0; v < 4; v++) {
+            Fm[v] *= keepm[d];
+            Fp[v] *= keepp[d];
+          }
+          // the minus face first, as the six faces are numbered
+          De += Fm[0] * dts;
+          Dx += Fm[1] * dts;
+          Dy += Fm[2] * dts;
+          Dz += Fm[3] * dts;
+          De -= Fp[0] * dts;
+          Dx -= Fp[1] * dts;
+          Dy -= Fp[2] * dts;
+          Dz -= Fp[3] * dts;
+          if (pairD[d] >= 0) {
+            // the cell's place in the oct face: its two coordinates across d
+            const int q = ((ic >> ((d + 1) % 3)) & 1) | (((ic >> ((d + 2) % 3)) & 1) << 1);
+            R F[4];
+#pragma unroll
+            for (int v = 0; v < 4; v++) F[v] = bit ? Fp[v] : Fm[v];
+            reflux<R, GA>(a, pairD[d], q, 2 * d + bit, g, F, dts);
+          }
+        }
+        if (ch <= -2) fold_reflux<R, GA, 1, kRefluxCell>(a, ch, g, 1, &Te[g], &Tx[g], &Ty[g], &Tz[g]);
+        Te[g] += De;
+        Tx[g] += Dx;
+        Ty[g] += Dy;
+        Tz[g] += Dz;
+      }
+      if (g + 1 < G) __syncthreads();  // the next group overwrites the tile's state
+    }
+  }
+  unsigned int nit_acc = 0, leaf = 0;
+  if (valid) {
+    if (a.t_first != nullptr) xion_times(a, cell);
+    if (restricted) {
+      restrict_cell(a, cell, ch, G);
+    } else if (ch >= 0) {
+      transport_split_cell<R, G>(a, cell, G, Te, Tx, Ty, Tz);
+    } else {
+      if (!transport && ch <= -2) {
+#pragma unroll
+        for (int g = 0; g < G; g++)
+          fold_reflux<R, GA, 1, kRefluxCell>(a, ch, g, 1, &Te[g], &Tx[g], &Ty[g], &Tz[g]);
+      }
+      leaf = 1;
+      nit_acc = (unsigned)finish_leaf<R, G, Fast, kRefluxCell>(a, K, cell, G, Te, Tx, Ty, Tz);
+    }
+  }
+  if (a.counters != nullptr) block_counters<kTileWaves>(a.counters, nit_acc, leaf);
+}
+
+// Waves per SIMD the register allocation aims at: FP64 with one group fits
+// four (64^3 cells 22.2 -> 20.1 us), with two or three groups three (64^3
+// cells 69 -> 64 us); more groups would spill.
+constexpr int cell_step_waves(size_t rb, int g) { return rb != 8 ? 1 : g == 1 ? 4 : g <= 3 ? 3 : 1; }
+template <typename R, int G, bool Fast>
+__global__ __launch_bounds__(kTileCells) __attribute__((amdgpu_waves_per_eu(cell_step_waves(sizeof(R), G)))) void
+level_step_kernel(LevelArgs<R> a_by_value, ChemConst K_by_value) {
   const KernArgs<R> args = kernargs<R>();
-  cell_step<R, G, Fast>(args.a, args.K, xcd_block(args.a.nblocks), (int)threadIdx.x);
+  cell_step_lds<R, G, Fast>(args.a, args.K, xcd_block(args.a.nblocks), (int)threadIdx.x, *cell_lds<R>());
 }
 
 // ------------------------------------------------------------------ tiled level step
@@ -820,7 +1059,7 @@ __device__ __forceinline__ void tiled_step(const LevelArgs<float>& a, const Chem
   Closure<float> Q[G];
   if (valid) {
 #pragma unroll
-    for (int g = 0; g < G; g++) Q[g] = closure_fast(Ux[g], Uy[g], Uz[g], Ue[g], c);
+    for (int g = 0; g < G; g++) Q[g] = closure_fast<true>(Ux[g], Uy[g], Uz[g], Ue[g], c);
   }
   if constexpr (!PerDir) store_item(hf[0], lane);
 
@@ -988,12 +1227,22 @@ __device__ __forceinline__ void tiled_step(const LevelArgs<float>& a, const Chem
     if (a.t_first != nullptr) xion_times(a, cell);
     if (ch >= 0 && !a.update_split) {
       restrict_cell(a, cell, ch, G);
-    } else if (ch >= 0) {
-      transport_split_cell<float, G>(a, cell, G, Ue, Ux, Uy, Uz, De, Dx, Dy, Dz);
     } else {
-      leaf = 1;
-      nit_acc = (unsigned)finish_leaf<float, G, true, kRefluxTiled, NT>(a, K, cell, ch, G, Ue, Ux, Uy, Uz, De, Dx, Dy, Dz,
-                                                                    Src, pre);
+      if (ch <= -2) fold_reflux<float, G, G, kRefluxTiled>(a, ch, 0, G, Ue, Ux, Uy, Uz);
+#pragma unroll
+      for (int g = 0; g < G; g++) {
+        Ue[g] += De[g];
+        Ux[g] += Dx[g];
+        Uy[g] += Dy[g];
+        Uz[g] += Dz[g];
+      }
+      if (ch >= 0) {
+        transport_split_cell<float, G>(a, cell, G, Ue, Ux, Uy, Uz);
+      } else {
+        leaf = 1;
+        nit_acc =
+            (unsigned)finish_leaf<float, G, true, kRefluxTiled, NT>(a, K, cell, G, Ue, Ux, Uy, Uz, Src, pre);
+      }
     }
   }
   if (a.counters != nullptr) block_counters<kTileWaves>(a.counters, nit_acc, leaf);
@@ -1391,12 +1640,29 @@ hipError_t launch_level_step(const LevelArgs<R>& a0, const ChemConst& K, hipStre
   int nb = (a.ncell + 255) / 256;
   nb = (nb + 7) & ~7;
   a.nblocks = nb;
-  const dim3 grid(nb), block(256);
+  const dim3 grid(nb), block(kTileCells);
   constexpr bool fast = sizeof(R) == 4;
   switch (a.ng) {
-    case 1: hipLaunchKernelGGL((level_step_kernel<R, 1, fast>), grid, block, 0, s, a, K); break;
-    case 3: hipLaunchKernelGGL((level_step_kernel<R, 3, fast>), grid, block, 0, s, a, K); break;
-    default: hipLaunchKernelGGL((level_step_kernel<R, 0, fast>), grid, block, 0, s, a, K); break;
+#define EMMA_STEP(g) \
+  case g: hipLaunchKernelGGL((level_step_kernel<R, g, fast>), grid, block, 0, s, a, K); break
+    EMMA_STEP(2);
+    EMMA_STEP(4);
+    EMMA_STEP(5);
+    EMMA_STEP(6);
+    EMMA_STEP(7);
+    EMMA_STEP(8);
+    EMMA_STEP(9);
+    default:
+      if constexpr (fast) {
+        return hipErrorInvalidValue;  // 1 and 3 groups took the tiled kernel
+      } else {
+        switch (a.ng) {
+          EMMA_STEP(1);
+          EMMA_STEP(3);
+          default: return hipErrorInvalidValue;
+        }
+      }
+#undef EMMA_STEP
   }
   return hipGetLastError();
 }

@@ -41,12 +41,18 @@ __device__ __forceinline__ double fdiv64(double a, double b) {
 // 25 - 4 (4 - 3 f^2) = 3 (3 + 4 f^2)), so (1 - chi)/2 = (s - 1)/3 and
 // (3 chi - 1)/2 = 2 - s need no division.  Beyond f^2 = 4/3 the reference
 // clamps the root to 0 and chi = (3 + 4 f^2) / 5.
+// |F|^2 is written out as fused multiply-adds: left to contraction, the
+// compiler picks the order of the squares by call site, and the same cell's
+// closure would round differently in two kernels.  X2First: the x term is the
+// one rounded by itself (a tile's own cells in the tiled kernel); otherwise
+// the y term (its halo cells, and the per-cell kernels).
+template <bool X2First = false>
 __device__ __forceinline__ Closure<float> closure_fast(float fx, float fy, float fz, float ee, float c) {
 #pragma clang fp contract(fast)
   // branch-free: the isotropic case (E <= 0 or F = 0: n = 0, f = 0) by selects
   Closure<float> q;
   const float c2e = ee * c * c;
-  const float f2 = fx * fx + fy * fy + fz * fz;
+  const float f2 = X2First ? fmaf(fz, fz, fmaf(fy, fy, fx * fx)) : fmaf(fz, fz, fmaf(fx, fx, fy * fy));
   const bool aniso = (ee > 0.f) & (f2 > 1e-36f);
   const float ri = aniso ? __builtin_amdgcn_rsqf(f2) : 0.f;
   q.n[0] = fx * ri;
