@@ -295,6 +295,17 @@ static ChemConst make_chem(const emma_rt_params& p, double dtnew, double aexp) {
   K.ki_e = K.pa3 / p.unit_N;
   K.ki_f = K.pa4 / p.unit_l * p.unit_t / p.unit_N;
   K.ki_eint = K.pa5 / (p.unit_n * p.unit_d * K.pv2);
+  K.r_a2 = 1. / K.a2;
+  K.r_a3 = 1. / K.a3;
+  K.r_pa3 = 1. / K.pa3;
+  K.r_pa4 = 1. / K.pa4;
+  K.r_pa5 = 1. / K.pa5;
+  K.r_unit_N = 1. / p.unit_N;
+  K.r_unit_l = 1. / p.unit_l;
+  K.r_unit_t = 1. / p.unit_t;
+  K.r_unit_n = 1. / p.unit_n;
+  K.r_unit_d = 1. / p.unit_d;
+  K.r_pv2 = 1. / K.pv2;
   for (int g = 0; g < p.ngrp; g++) {
     K.heat[g] = p.alphae[g] * p.hnu[g] - p.alphai[g] * kHnu0;
     K.alphai[g] = p.alphai[g];

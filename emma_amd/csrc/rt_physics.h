@@ -9,6 +9,8 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
+#include "rt_math64.h"
+
 namespace emma {
 
 constexpr int kMaxGrp = 9;
@@ -56,6 +58,8 @@ struct ChemConst {
   double ki_e;     // a^3/unit_N
   double ki_f;     // a^4/unit_l*unit_t/unit_N
   double ki_eint;  // a^5/(unit_n*unit_d*unit_v^2)
+  // reciprocals of the FP64 path's uniform divisors (div64)
+  double r_a2, r_a3, r_pa3, r_pa4, r_pa5, r_unit_N, r_unit_l, r_unit_t, r_unit_n, r_unit_d, r_pv2;
 };
 
 // ---------------------------------------------------------------- Eddington
@@ -78,17 +82,33 @@ __device__ __forceinline__ Closure<R> closure(R fx, R fy, R fz, R ee, R c) {
   q.n[0] = R(0);
   q.n[1] = R(0);
   q.n[2] = R(0);
-  if (ee > R(0)) {
-    ff = sqrt(fx * fx + fy * fy + fz * fz);
-    if (ff > R(0)) {
-      q.n[0] = fx / ff;
-      q.n[1] = fy / ff;
-      q.n[2] = fz / ff;
+  R arg, chi;
+  if constexpr (sizeof(R) == 8) {  // the three n_i share |F|'s reciprocal
+    if (ee > R(0)) {
+      ff = sqrt(fx * fx + fy * fy + fz * fz);
+      if (ff > R(0)) {
+        const R r = rcp64(ff);
+        q.n[0] = div64(fx, ff, r);
+        q.n[1] = div64(fy, ff, r);
+        q.n[2] = div64(fz, ff, r);
+      }
+      ff = div64(ff, c * ee);
     }
-    ff = ff / (c * ee);
+    arg = fmax(R(4) - R(3) * ff * ff, R(0));
+    chi = div64(R(3) + R(4) * ff * ff, R(5) + R(2) * sqrt(arg));
+  } else {
+    if (ee > R(0)) {
+      ff = sqrt(fx * fx + fy * fy + fz * fz);
+      if (ff > R(0)) {
+        q.n[0] = fx / ff;
+        q.n[1] = fy / ff;
+        q.n[2] = fz / ff;
+      }
+      ff = ff / (c * ee);
+    }
+    arg = fmax(R(4) - R(3) * ff * ff, R(0));
+    chi = (R(3) + R(4) * ff * ff) / (R(5) + R(2) * sqrt(arg));
   }
-  R arg = fmax(R(4) - R(3) * ff * ff, R(0));
-  R chi = (R(3) + R(4) * ff * ff) / (R(5) + R(2) * sqrt(arg));
   q.diag = (R(1) - chi) / R(2) * c2e;
   q.arg = (R(3) * chi - R(1)) / R(2) * c2e;
   return q;
@@ -141,16 +161,23 @@ struct Rates {
 __device__ __forceinline__ Rates rates_of(double temp) {
   Rates r;
   const double sT = sqrt(temp);
-  const double sT5 = sqrt(temp / 1e5);
-  const double lam = 2e0 * 157807e0 / temp;
-  r.A1 = exp(-157809.1e0 / temp) * 2.54e-21 * sT / (1. + sT5);
-  r.A6 = 3.435e-30 * temp * pow(lam, 1.970e0) / pow(1. + (pow(lam / 2.250e0, 0.376e0)), 3.720e0);
-  r.A3 = exp(-118348e0 / temp) * 7.5e-19 / (1 + sT5);
+  const double sT5 = sqrt(div64(temp, 1e5, 1e-5));
+  const double rT = rcp64(temp);
+  const double g = 1. + sT5, rg = rcp64(g);
+  r.A1 = div64(exp64(div64(-157809.1e0, temp, rT)) * 2.54e-21 * sT, g, rg);
+  r.A3 = div64(exp64(div64(-118348e0, temp, rT)) * 7.5e-19, g, rg);
   r.A4 = 1.42e-27 * 1.5e0 * sT;
-  double ab = 2.753e-14 * pow(lam, 1.5) / pow(1e0 + pow(lam / 2.740, 0.407), 2.242);
-  r.alphab = ab * 1e-6 * 1.;
-  double b = 1.17e-10 * sT / (1 + sT5) * exp(-(157809e0 / temp));
+  const double b = div64(1.17e-10 * sT, g, rg) * exp64(-div64(157809e0, temp, rT));
   r.beta = b * 1e-6 * 1.;
+  // lam^1.970 / (1 + (lam/2.250)^0.376)^3.720 and
+  // lam^1.5 / (1 + (lam/2.740)^0.407)^2.242, lam = 2 x 157807 / T
+  const Dd L = log_dd(div64(2e0 * 157807e0, temp, rT));
+  const Dd ln225 = {0x1.9f323ecbf984cp-1, -0x1.a92e513217f5cp-58}, ln274 = {0x1.020987bfdcb15p+0, 0x1.953b86e09d8b0p-55};
+  const Dd W6 = log_dd(1. + exp_of(dd_scale(0.376e0, dd_sub(L, ln225))));
+  r.A6 = 3.435e-30 * temp * exp_of(dd_sub(dd_scale(1.970e0, L), dd_scale(3.720e0, W6)));
+  const Dd Wb = log_dd(1. + exp_of(dd_scale(0.407, dd_sub(L, ln274))));
+  const double ab = 2.753e-14 * exp_of(dd_sub(dd_scale(1.5, L), dd_scale(2.242, Wb)));
+  r.alphab = ab * 1e-6 * 1.;
   return r;
 }
 
@@ -176,23 +203,22 @@ __device__ int chem_cell(const ChemConst& K, int ng, double* e, double* fx, doub
                          const double* src, double& nhplus, double& eint_code, double nh, double& temp,
                          int chemonly, int& nit) {
   constexpr int GA = G > 0 ? G : kMaxGrp;
-  double egy[GA], fl0[GA], fl1[GA], fl2[GA], srcl[GA], et[GA], p[GA];
+  double egy[GA], fl0[GA], fl1[GA], fl2[GA], srcl[GA], et[GA], p[GA], rp[GA];
   const double aexporg = K.aexp;
-  const double a3 = K.a3;
   const double notchem = (double)(!chemonly);
 #pragma unroll
   for (int g = 0; g < GA; g++) {
     if (g < ng) {
-      egy[g] = e[g] / a3 * K.unit_N;
-      fl0[g] = fx[g] / K.pa4 * K.unit_l / K.unit_t * K.unit_N;
-      fl1[g] = fy[g] / K.pa4 * K.unit_l / K.unit_t * K.unit_N;
-      fl2[g] = fz[g] / K.pa4 * K.unit_l / K.unit_t * K.unit_N;
-      srcl[g] = (src[g] * K.unit_N / K.unit_t / K.a2) / K.pa3;
+      egy[g] = div64(e[g], K.a3, K.r_a3) * K.unit_N;
+      fl0[g] = div64(div64(fx[g], K.pa4, K.r_pa4) * K.unit_l, K.unit_t, K.r_unit_t) * K.unit_N;
+      fl1[g] = div64(div64(fy[g], K.pa4, K.r_pa4) * K.unit_l, K.unit_t, K.r_unit_t) * K.unit_N;
+      fl2[g] = div64(div64(fz[g], K.pa4, K.r_pa4) * K.unit_l, K.unit_t, K.r_unit_t) * K.unit_N;
+      srcl[g] = div64(div64(div64(src[g] * K.unit_N, K.unit_t, K.r_unit_t), K.a2, K.r_a2), K.pa3, K.r_pa3);
     }
   }
-  double x0 = nhplus / nh;
-  const double nH = nh / a3 * K.unit_N;
-  double eint = eint_code / K.pa5 * K.unit_n * K.unit_d * K.pv2;
+  double x0 = div64(nhplus, nh);
+  const double nH = div64(nh, K.a3, K.r_a3) * K.unit_N;
+  double eint = div64(eint_code, K.pa5, K.r_pa5) * K.unit_n * K.unit_d * K.pv2;
   const double emin = K.emin;
   nit = 0;
   if (egy[0] < kEmin) return -4;
@@ -202,14 +228,14 @@ __device__ int chem_cell(const ChemConst& K, int ng, double* e, double* fx, doub
   double tcur = 0.;
   const double dt = K.dt;
   double tcached = -1.;
-  Rates r = rates_of(1e4);
+  Rates r = {};  // evaluated on the first pass (tloc != tcached)
   int tries = 0;
   while (tcur < dt) {
     // the reference loops until t >= dt; a try budget keeps every wave finite
     // on pathological input (reported as non-convergence)
     if (++tries > kMaxTries) return -5;
     const double Nfree = (1. + x0) * nH;
-    const double tloc = eint / (1.5 * Nfree * kKboltz);
+    const double tloc = div64(eint, 1.5 * Nfree * kKboltz);
     if (!(tloc == tcached)) {  // rates depend on T only, which changes only after an accepted sub-step
       r = rates_of(tloc);
       tcached = tloc;
@@ -220,6 +246,7 @@ __device__ int chem_cell(const ChemConst& K, int ng, double* e, double* fx, doub
 #pragma unroll
     for (int g = 0; g < GA; g++)
       if (g < ng) ai += K.heat[g] * egy[g] * nH * (1.0 - x0);
+    // (a zero rate has to give an infinite cooling time: plain division)
     const double tcool = fabs(eint / (ai * notchem - Cool0));
     const double dtcool = fmin(fudgecool * tcool, dt - tcur);
     const double alpha = r.alphab;  // OTSA (chem_utils.c:497-500)
@@ -228,14 +255,16 @@ __device__ int chem_cell(const ChemConst& K, int ng, double* e, double* fx, doub
     for (int g = 0; g < GA; g++) {
       if (g < ng) {
         const double aig = K.alphai[g] * (1. - x0);
+        // one reciprocal for the density's and (below) the flux's quotients
+        p[g] = (1. + (aig * nH) * dtcool);
+        rp[g] = rcp64(p[g]);
         if (chemonly) {
           et[g] = egy[g];
         } else {
-          et[g] = ((alpha - r.alphab) * x0 * x0 * nH * nH * dtcool * 0. + egy[g] + srcl[g] * dtcool * K.factgrp[g]) /
-                  (1. + dtcool * (aig * nH));
+          et[g] = div64((alpha - r.alphab) * x0 * x0 * nH * nH * dtcool * 0. + egy[g] + srcl[g] * dtcool * K.factgrp[g],
+                        p[g], rp[g]);
         }
         if ((et[g] < 0) || isnan(et[g])) test = 1;
-        p[g] = (1. + (aig * nH) * dtcool);
       }
     }
     if (test) {
@@ -247,7 +276,7 @@ __device__ int chem_cell(const ChemConst& K, int ng, double* e, double* fx, doub
     for (int g = 0; g < GA; g++)
       if (g < ng) ai += K.alphai[g] * et[g] * notchem;
     const double RECT = alpha * x0 * x0 * nH * dtcool;
-    const double xt = 1. - (RECT + (1.0 - x0)) / (1. + dtcool * (r.beta * x0 * nH + ai));
+    const double xt = 1. - div64(RECT + (1.0 - x0), 1. + dtcool * (r.beta * x0 * nH + ai));
     if (((xt > 1.) || (xt < 0.)) || isnan(xt)) {
       fudgecool /= 10.;
       continue;
@@ -262,7 +291,7 @@ __device__ int chem_cell(const ChemConst& K, int ng, double* e, double* fx, doub
       fudgecool = fudgecool / 10.;
       continue;
     }
-    const double deltaE = fabs(eintt / eint - 1.);
+    const double deltaE = fabs(div64(eintt, eint) - 1.);
     if (deltaE > kFracVar) {
       fudgecool = fudgecool / 10.;
       continue;
@@ -274,9 +303,9 @@ __device__ int chem_cell(const ChemConst& K, int ng, double* e, double* fx, doub
         if (g < ng) {
           egy[g] = et[g];
           if (!chemonly) {
-            fl0[g] = fl0[g] / p[g];
-            fl1[g] = fl1[g] / p[g];
-            fl2[g] = fl2[g] / p[g];
+            fl0[g] = div64(fl0[g], p[g], rp[g]);
+            fl1[g] = div64(fl1[g], p[g], rp[g]);
+            fl2[g] = div64(fl2[g], p[g], rp[g]);
           }
         }
       }
@@ -292,9 +321,9 @@ __device__ int chem_cell(const ChemConst& K, int ng, double* e, double* fx, doub
         if (g < ng) {
           egy[g] = et[g] * r3;
           if (!chemonly) {
-            fl0[g] = fl0[g] / p[g] * r4;
-            fl1[g] = fl1[g] / p[g] * r4;
-            fl2[g] = fl2[g] / p[g] * r4;
+            fl0[g] = div64(fl0[g], p[g], rp[g]) * r4;
+            fl1[g] = div64(fl1[g], p[g], rp[g]) * r4;
+            fl2[g] = div64(fl2[g], p[g], rp[g]) * r4;
           }
         }
       }
@@ -307,34 +336,39 @@ __device__ int chem_cell(const ChemConst& K, int ng, double* e, double* fx, doub
     if ((nit == K.ncvgcool) && (K.ncvgcool != 0)) break;
   }
   // back to code units (chem_utils.c:775-791) and E2T (21-32)
-  double pa3f, pa4f, pa5f;
+  double pa3f, pa4f, pa5f, r_pa3f, r_pa5f;
   if (K.static_cosmo) {
     pa3f = K.pa3;
     pa4f = K.pa4;
     pa5f = K.pa5;
+    r_pa3f = K.r_pa3;
+    r_pa5f = K.r_pa5;
   } else {
     pa3f = pow(aexp, 3);
     pa4f = pow(aexp, 4);
     pa5f = pow(aexp, 5);
+    r_pa3f = rcp64(pa3f);
+    r_pa5f = rcp64(pa5f);
   }
   if (!chemonly) {
+    const double ul = K.unit_l, rul = K.r_unit_l, uN = K.unit_N, ruN = K.r_unit_N;
 #pragma unroll
     for (int g = 0; g < GA; g++) {
       if (g < ng) {
-        e[g] = fmax(egy[g] * pa3f / K.unit_N, K.emin_grp[g]);
-        fx[g] = fl0[g] * pa4f / K.unit_l * K.unit_t / K.unit_N;
-        fy[g] = fl1[g] * pa4f / K.unit_l * K.unit_t / K.unit_N;
-        fz[g] = fl2[g] * pa4f / K.unit_l * K.unit_t / K.unit_N;
+        e[g] = fmax(div64(egy[g] * pa3f, uN, ruN), K.emin_grp[g]);
+        fx[g] = div64(div64(fl0[g] * pa4f, ul, rul) * K.unit_t, uN, ruN);
+        fy[g] = div64(div64(fl1[g] * pa4f, ul, rul) * K.unit_t, uN, ruN);
+        fz[g] = div64(div64(fl2[g] * pa4f, ul, rul) * K.unit_t, uN, ruN);
       }
     }
   }
   nhplus = x0 * nh;
-  eint_code = eint * pa5f / K.unit_n / K.unit_d / K.pv2;
+  eint_code = div64(div64(div64(eint * pa5f, K.unit_n, K.r_unit_n), K.unit_d, K.r_unit_d), K.pv2, K.r_pv2);
   {
-    const double x = nhplus / nh;
-    const double nHe = nh / pa3f * K.unit_N;
-    const double ee = eint_code / pa5f * K.pstar;
-    temp = ee / (1.5 * nHe * kKboltz * (1. + x) * (1. + kyHe));
+    const double x = div64(nhplus, nh);
+    const double nHe = div64(nh, pa3f, r_pa3f) * K.unit_N;
+    const double ee = div64(eint_code, pa5f, r_pa5f) * K.pstar;
+    temp = div64(ee, 1.5 * nHe * kKboltz * (1. + x) * (1. + kyHe));
   }
   return 0;
 }
