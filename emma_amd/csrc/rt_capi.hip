@@ -18,6 +18,7 @@
 #include "rt_kernels.h"
 #include "rt_sched.h"
 #include "rt_stencil.h"
+#include "rt_xfer.h"
 
 using namespace emma;
 
@@ -409,6 +410,7 @@ extern "C" int emma_rt_create(const emma_rt_params* p, emma_rt_ctx** out) {
   int n = 0;
   if (hipGetDeviceCount(&n) != hipSuccess || n == 0) return EMMA_RT_ERR_NODEVICE;
   emma_rt_ctx* c = new emma_rt_ctx();
+  xfer_retain();
   c->p = *p;
   memset(&c->stats, 0, sizeof(c->stats));
   memset(c->level_ms, 0, sizeof(c->level_ms));
@@ -463,6 +465,7 @@ extern "C" int emma_rt_destroy(emma_rt_ctx* c) {
   if (c->h_status) (void)hipHostFree(c->h_status);
   if (c->h_counters) (void)hipHostFree(c->h_counters);
   if (c->stream) (void)hipStreamDestroy(c->stream);
+  xfer_release();
   delete c;
   return EMMA_RT_OK;
 }
@@ -664,53 +667,25 @@ static DevLevel* level_of(emma_rt_ctx* c, int level) {
   return &c->lev[level - c->lmin];
 }
 
-// floor (photon densities, FP32 storage): a value at or above the group's
-// floor must not round below it (ncell values per group)
-template <typename R>
-static int upload_r(void* dst, const double* src, size_t n, hipStream_t s, const emma_rt_params* floor = nullptr,
-                    size_t ncell = 0) {
-  if (sizeof(R) == sizeof(double)) {
-    HIPCHK(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyHostToDevice, s));
-    HIPCHK(hipStreamSynchronize(s));
-    return EMMA_RT_OK;
+// the group fields and cell fields of one level as transfer parts; host
+// pointers in emma_rt_set_level's order, null ones left out
+static int level_parts(emma_rt_ctx* c, DevLevel& L, double* const host[9], XferPart* p) {
+  const int G = c->p.ngrp, b = L.cur, f32 = c->rbytes == 4;
+  const size_t n = L.ncell;
+  void* const rad[5] = {L.e[b], L.fx[b], L.fy[b], L.fz[b], L.src};
+  double* const cell[4] = {L.nhplus[b], L.eint[b], L.nh, L.temp[b]};
+  int np = 0;
+  for (int g = 0; host[0] && g < G; g++) {  // the photon densities group by group: each has its floor
+    const double f = f32 ? emin_floor(c->p, g) : 0.;
+    p[np++] = {(char*)rad[0] + g * n * c->rbytes, host[0] + g * n, n, f32, f32 ? emin_floor_up(f) : 0.f, f};
   }
-  std::vector<R> tmp(n);
-  for (size_t i = 0; i < n; i++) tmp[i] = (R)src[i];
-  if (floor != nullptr) {
-    for (size_t i = 0; i < n; i++) {
-      const int g = (int)(i / ncell);
-      const double f = emin_floor(*floor, g);
-      if (src[i] >= f && (double)tmp[i] < f) tmp[i] = (R)emin_floor_up(f);
-    }
-  }
-  HIPCHK(hipMemcpyAsync(dst, tmp.data(), n * sizeof(R), hipMemcpyHostToDevice, s));
-  HIPCHK(hipStreamSynchronize(s));
-  return EMMA_RT_OK;
+  for (int k = 1; k < 5; k++)
+    if (host[k]) p[np++] = {rad[k], host[k], (size_t)G * n, f32, 0.f, 0.};
+  for (int k = 0; k < 4; k++)
+    if (host[5 + k]) p[np++] = {cell[k], host[5 + k], n, 0, 0.f, 0.};
+  return np;
 }
-
-template <typename R>
-static int download_r(double* dst, const void* src, size_t n, hipStream_t s) {
-  if (sizeof(R) == sizeof(double)) {
-    HIPCHK(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
-    return EMMA_RT_OK;
-  }
-  std::vector<R> tmp(n);
-  HIPCHK(hipMemcpyAsync(tmp.data(), src, n * sizeof(R), hipMemcpyDeviceToHost, s));
-  HIPCHK(hipStreamSynchronize(s));
-  for (size_t i = 0; i < n; i++) dst[i] = (double)tmp[i];
-  return EMMA_RT_OK;
-}
-
-static int upload_rf(emma_rt_ctx* c, void* dst, const double* src, size_t n, bool photon_floor = false,
-                     size_t ncell = 0) {
-  const emma_rt_params* fl = photon_floor ? &c->p : nullptr;
-  return c->rbytes == 8 ? upload_r<double>(dst, src, n, c->stream) : upload_r<float>(dst, src, n, c->stream, fl, ncell);
-}
-
-static int download_rf(emma_rt_ctx* c, double* dst, const void* src, size_t n) {
-  return c->rbytes == 8 ? download_r<double>(dst, src, n, c->stream) : download_r<float>(dst, src, n, c->stream);
-}
+static_assert(EMMA_RT_MAX_GRP + 8 <= kMaxXferParts, "a level's arrays fit one transfer");
 
 extern "C" int emma_rt_set_level(emma_rt_ctx* c, int level, const double* e, const double* fx, const double* fy,
                                  const double* fz, const double* src, const double* nhplus, const double* eint,
@@ -718,17 +693,12 @@ extern "C" int emma_rt_set_level(emma_rt_ctx* c, int level, const double* e, con
   DevLevel* L = level_of(c, level);
   if (L == nullptr) return EMMA_RT_ERR_STATE;
   if (!e || !fx || !fy || !fz || !src || !nhplus || !eint || !nh || !temp) return EMMA_RT_ERR_ARG;
-  const size_t gn = (size_t)c->p.ngrp * L->ncell;
-  const int b = L->cur;
-  int st;
-  if ((st = upload_rf(c, L->e[b], e, gn, true, L->ncell)) || (st = upload_rf(c, L->fx[b], fx, gn)) ||
-      (st = upload_rf(c, L->fy[b], fy, gn)) || (st = upload_rf(c, L->fz[b], fz, gn)) ||
-      (st = upload_rf(c, L->src, src, gn)))
-    return st;
-  HIPCHK(hipMemcpy(L->nhplus[b], nhplus, L->ncell * sizeof(double), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(L->eint[b], eint, L->ncell * sizeof(double), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(L->temp[b], temp, L->ncell * sizeof(double), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(L->nh, nh, L->ncell * sizeof(double), hipMemcpyHostToDevice));
+  double* const host[9] = {const_cast<double*>(e),      const_cast<double*>(fx),   const_cast<double*>(fy),
+                           const_cast<double*>(fz),     const_cast<double*>(src),  const_cast<double*>(nhplus),
+                           const_cast<double*>(eint),   const_cast<double*>(nh),   const_cast<double*>(temp)};
+  XferPart p[kMaxXferParts];
+  const int np = level_parts(c, *L, host, p);
+  HIPCHK(xfer_to_device(c->device, c->stream, p, np));
   return EMMA_RT_OK;
 }
 
@@ -736,19 +706,10 @@ extern "C" int emma_rt_get_level(emma_rt_ctx* c, int level, double* e, double* f
                                  double* src, double* nhplus, double* eint, double* nh, double* temp) {
   DevLevel* L = level_of(c, level);
   if (L == nullptr) return EMMA_RT_ERR_STATE;
-  HIPCHK(hipStreamSynchronize(c->stream));
-  const size_t gn = (size_t)c->p.ngrp * L->ncell;
-  const int b = L->cur;
-  int st;
-  if (e && (st = download_rf(c, e, L->e[b], gn))) return st;
-  if (fx && (st = download_rf(c, fx, L->fx[b], gn))) return st;
-  if (fy && (st = download_rf(c, fy, L->fy[b], gn))) return st;
-  if (fz && (st = download_rf(c, fz, L->fz[b], gn))) return st;
-  if (src && (st = download_rf(c, src, L->src, gn))) return st;
-  if (nhplus) HIPCHK(hipMemcpy(nhplus, L->nhplus[b], L->ncell * sizeof(double), hipMemcpyDeviceToHost));
-  if (eint) HIPCHK(hipMemcpy(eint, L->eint[b], L->ncell * sizeof(double), hipMemcpyDeviceToHost));
-  if (nh) HIPCHK(hipMemcpy(nh, L->nh, L->ncell * sizeof(double), hipMemcpyDeviceToHost));
-  if (temp) HIPCHK(hipMemcpy(temp, L->temp[b], L->ncell * sizeof(double), hipMemcpyDeviceToHost));
+  double* const host[9] = {e, fx, fy, fz, src, nhplus, eint, nh, temp};
+  XferPart p[kMaxXferParts];
+  const int np = level_parts(c, *L, host, p);
+  HIPCHK(xfer_to_host(c->device, c->stream, p, np));
   return EMMA_RT_OK;
 }
 
@@ -1247,9 +1208,10 @@ extern "C" int emma_rt_set_hydro(emma_rt_ctx* c, int level, const double* d, con
   for (int k = 0; k < 7; k++)
     if (L->hyd[k] == nullptr) HIPCHK(hipMalloc((void**)&L->hyd[k], nb));
   const double* in[6] = {d, u, v, w, p, dX};
-  for (int k = 0; k < 6; k++) HIPCHK(hipMemcpy(L->hyd[k], in[k], nb, hipMemcpyHostToDevice));
   HIPCHK(launch_fill((unsigned int*)L->hyd[6], 2 * L->ncell, 0u, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  XferPart x[6];
+  for (int k = 0; k < 6; k++) x[k] = {L->hyd[k], const_cast<double*>(in[k]), (size_t)L->ncell, 0, 0.f, 0.};
+  HIPCHK(xfer_to_device(c->device, c->stream, x, 6));
   return EMMA_RT_OK;
 }
 
@@ -1258,11 +1220,10 @@ extern "C" int emma_rt_get_hydro(emma_rt_ctx* c, int level, double* p, double* d
   if (L == nullptr) return EMMA_RT_ERR_STATE;
   if (L->ncell == 0) return EMMA_RT_OK;
   if (L->hyd[0] == nullptr) return EMMA_RT_ERR_STATE;
-  const size_t nb = (size_t)L->ncell * sizeof(double);
-  HIPCHK(hipStreamSynchronize(c->stream));
-  if (p) HIPCHK(hipMemcpy(p, L->hyd[4], nb, hipMemcpyDeviceToHost));
-  if (dX) HIPCHK(hipMemcpy(dX, L->hyd[5], nb, hipMemcpyDeviceToHost));
-  if (E) HIPCHK(hipMemcpy(E, L->hyd[6], nb, hipMemcpyDeviceToHost));
+  double* const out[3] = {p, dX, E};
+  XferPart x[3];
+  for (int k = 0; k < 3; k++) x[k] = {L->hyd[4 + k], out[k], out[k] ? (size_t)L->ncell : 0, 0, 0.f, 0.};
+  HIPCHK(xfer_to_host(c->device, c->stream, x, 3));
   return EMMA_RT_OK;
 }
 

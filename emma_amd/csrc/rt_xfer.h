@@ -1,0 +1,33 @@
+// rt_xfer.h -- host arrays of doubles to and from device arrays of double or
+// float (the state of a level, emma_rt_set_level / emma_rt_get_level).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <stddef.h>
+
+namespace emma {
+
+// one array: n values, device storage float (f32) or double.  floor > 0 (to
+// the device, f32): a value at or above it that rounds below it becomes
+// floor_up, the smallest float at or above it.
+struct XferPart {
+  void* dev;
+  void* host;
+  size_t n;
+  int f32;
+  float floor_up;
+  double floor;
+};
+constexpr int kMaxXferParts = 24;
+
+// Both wait for the work queued on the stream before and return with the copy
+// done.  Callable from several threads; the staging memory is shared by all
+// callers, bounded, and released with the last xfer_release().
+hipError_t xfer_to_host(int device, hipStream_t s, const XferPart* parts, int np);
+hipError_t xfer_to_device(int device, hipStream_t s, const XferPart* parts, int np);
+// a user of the staging memory comes (a context is made) and goes
+void xfer_retain();
+void xfer_release();
+
+}  // namespace emma

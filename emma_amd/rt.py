@@ -342,12 +342,12 @@ class RadGPU:
     def set(self, level: int, which: int, F: Fields):
         if which != 0:
             raise ValueError("the device holds one state per level (rfield); rfieldnew is internal")
-        F = F.copy()
-        self._check(self.lib.emma_rt_set_level(self.h, level, *[_d(getattr(F, k)) for k in Fields.NAMES]))
+        a = [np.ascontiguousarray(getattr(F, k), dtype=np.float64) for k in Fields.NAMES]
+        self._check(self.lib.emma_rt_set_level(self.h, level, *[_d(x) for x in a]))
 
     def get(self, level: int, which: int = 0) -> Fields:
         n = self.tree.level(level).ncell
-        F = Fields.zeros(self.params.ngrp, n)
+        F = Fields.empty(self.params.ngrp, n)
         self._check(self.lib.emma_rt_get_level(self.h, level, *[_d(getattr(F, k)) for k in Fields.NAMES]))
         return F
 

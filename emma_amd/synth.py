@@ -49,6 +49,12 @@ class Fields:
         s = lambda: np.zeros(ncell)
         return cls(g(), g(), g(), g(), g(), s(), s(), s(), s())
 
+    @classmethod
+    def empty(cls, ngrp: int, ncell: int) -> "Fields":
+        g = lambda: np.empty((ngrp, ncell))
+        s = lambda: np.empty(ncell)
+        return cls(g(), g(), g(), g(), g(), s(), s(), s(), s())
+
     def xion(self) -> np.ndarray:
         return self.nhplus / self.nh
 
