@@ -9,6 +9,7 @@
 #include <sys/stat.h>
 
 #include <algorithm>
+#include <chrono>
 #include <map>
 #include <mutex>
 #include <string>
@@ -154,10 +155,8 @@ struct emma_rt_ctx {
   std::vector<DevLevel> lev;  // index level - lmin
   int* d_status = nullptr;
   unsigned long long* d_counters = nullptr;
-  // page-locked copies of the status word and the counters, read back by
-  // end_call with asynchronous copies behind the call's work and one wait
-  int* h_status = nullptr;
-  unsigned long long* h_counters = nullptr;
+  CallRecord* h_call = nullptr;  // page-locked: what the call's last kernel reports
+  bool words_dirty = false;      // a call began and did not reach its end
   void* scratch = nullptr;  // this device's no-alloc staging area (emma_rt_advance_stencil_noalloc)
   double* d_photons = nullptr;
   // straggler list of the tiled mixed kernel (capacity: the largest level's
@@ -419,9 +418,7 @@ extern "C" int emma_rt_create(const emma_rt_params* p, emma_rt_ctx** out) {
       hipMalloc((void**)&c->d_status, 4 * sizeof(int)) != hipSuccess ||
       hipMalloc((void**)&c->d_counters, kCounterSlots * kCounterStride * sizeof(unsigned long long)) != hipSuccess ||
       hipMalloc((void**)&c->d_photons, sizeof(double)) != hipSuccess ||
-      hipHostMalloc((void**)&c->h_status, 4 * sizeof(int)) != hipSuccess ||
-      hipHostMalloc((void**)&c->h_counters, kCounterSlots * kCounterStride * sizeof(unsigned long long)) !=
-          hipSuccess) {
+      hipHostMalloc((void**)&c->h_call, sizeof(CallRecord)) != hipSuccess) {
     emma_rt_destroy(c);
     return EMMA_RT_ERR_HIP;
   }
@@ -462,8 +459,7 @@ extern "C" int emma_rt_destroy(emma_rt_ctx* c) {
   (void)hipFree(c->d_status);
   (void)hipFree(c->d_counters);
   (void)hipFree(c->d_photons);
-  if (c->h_status) (void)hipHostFree(c->h_status);
-  if (c->h_counters) (void)hipHostFree(c->h_counters);
+  if (c->h_call) (void)hipHostFree(c->h_call);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   xfer_release();
   delete c;
@@ -933,6 +929,7 @@ static int ensure_defer_slots(emma_rt_ctx* c, long long n) {
   const int m = (int)((n + 255) & ~255LL);
   HIPCHK(dalloc(&c->d_defer_ctl, (size_t)m));
   c->defer_slots = m;
+  c->words_dirty = true;
   return EMMA_RT_OK;
 }
 
@@ -944,22 +941,27 @@ static long long steps_per_call(emma_rt_ctx* c, int ncoarse) {
   return steps;
 }
 
-// the device words a call starts from: status, straggler list lengths,
-// counters (fill kernels, so that a coarse step can capture them at the
-// head of its graph)
+// Call words: the status word, the straggler list lengths and the counters.
+// A call finds them zero: its last kernel (call_end_kernel) reports the status
+// and the summed counters into a page-locked record and clears the words for
+// the next call, in place of three fill launches before the call's work and two
+// copies behind it (a level step of 16^3 cells from the host: 41 us a call
+// with them, 23 us now, 6 us of it the level step).  A call that ended early left them dirty: the
+// next one clears them.
 static int clear_call_words(emma_rt_ctx* c) {
   HIPCHK(launch_fill((unsigned int*)c->d_status, 4, 0u, c->stream));
   if (c->defer_slots > 0) HIPCHK(launch_fill((unsigned int*)c->d_defer_ctl, c->defer_slots, 0u, c->stream));
-  if (c->counters) HIPCHK(launch_fill((unsigned int*)c->d_counters, 2 * kCounterSlots * kCounterStride, 0u, c->stream));
+  HIPCHK(launch_fill((unsigned int*)c->d_counters, 2 * kCounterSlots * kCounterStride, 0u, c->stream));
   return EMMA_RT_OK;
 }
 
-// clear_device = false: the caller runs clear_call_words inside its graph
-static int begin_call(emma_rt_ctx* c, bool clear_device = true) {
-  if (clear_device) {
+static int begin_call(emma_rt_ctx* c) {
+  if (c->words_dirty) {
     int st = clear_call_words(c);
     if (st) return st;
   }
+  c->words_dirty = true;
+  c->h_call->flag = 0;
   c->defer_seq = 0;
   memset(&c->stats, 0, sizeof(c->stats));
   c->ev_used = 0;
@@ -967,24 +969,38 @@ static int begin_call(emma_rt_ctx* c, bool clear_device = true) {
   return EMMA_RT_OK;
 }
 
-static int end_call(emma_rt_ctx* c) {
-  // the status word (and the counters) copied behind the call's work, one wait
-  const bool counted = c->counters != 0;
-  HIPCHK(hipMemcpyAsync(c->h_status, c->d_status, 4 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  if (counted)
-    HIPCHK(hipMemcpyAsync(c->h_counters, c->d_counters, kCounterSlots * kCounterStride * sizeof(unsigned long long),
-                          hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
-  const int* status = c->h_status;
-  const unsigned long long* slots = c->h_counters;
-  unsigned long long cnt[3] = {0ull, 0ull, 0ull};
-  if (counted) {
-    for (int i = 0; i < kCounterSlots; i++) {
-      cnt[0] += slots[(size_t)i * kCounterStride + 0];
-      cnt[1] += slots[(size_t)i * kCounterStride + 1];
-      cnt[2] += slots[(size_t)i * kCounterStride + 2];
+// the call's last kernel (captured at the tail of a coarse step's graph)
+static hipError_t queue_call_end(emma_rt_ctx* c) {
+  return launch_call_end(c->d_status, c->counters ? c->d_counters : nullptr, c->d_defer_ctl, c->defer_slots, c->h_call,
+                         c->stream);
+}
+
+// Wait for the call's record.  Its flag arrives with the record, some
+// microseconds before the runtime reports the stream idle; past a short wait
+// (long calls, or a failed one) the runtime's own wait takes over.
+static int wait_call(emma_rt_ctx* c) {
+  if (!c->timing) {
+    const auto t0 = std::chrono::steady_clock::now();
+    for (;;) {
+      for (int i = 0; i < 64; i++) {
+        if (__atomic_load_n(&c->h_call->flag, __ATOMIC_ACQUIRE) != 0) return EMMA_RT_OK;
+        __builtin_ia32_pause();
+      }
+      if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) break;
     }
   }
+  HIPCHK(hipStreamSynchronize(c->stream));
+  return __atomic_load_n(&c->h_call->flag, __ATOMIC_ACQUIRE) != 0 ? EMMA_RT_OK : EMMA_RT_ERR_HIP;
+}
+
+static int end_call(emma_rt_ctx* c, bool queued = false) {
+  if (!queued) HIPCHK(queue_call_end(c));
+  int st = wait_call(c);
+  if (st) return st;
+  c->words_dirty = false;
+  const bool counted = c->counters != 0;
+  const int* status = c->h_call->status;
+  const unsigned long long* cnt = c->h_call->counts;
   c->stats.status = status[0];
   c->stats.bad_level = status[1];
   c->stats.bad_cell = status[2];
@@ -1586,10 +1602,8 @@ extern "C" int emma_rt_coarse_step(emma_rt_ctx* c, double aexp, int ncoarse) {
   if (st) return st;
   st = ensure_defer_slots(c, steps_per_call(c, ncoarse));
   if (st) return st;
-  // replays of the captured coarse step clear the call's device words at
-  // the head of the graph; eager launches (TIMING_LAUNCH) clear them here
-  const bool eager = c->timing == 1;
-  st = begin_call(c, eager);
+  const bool eager = c->timing == 1;  // launches with their own events
+  st = begin_call(c);
   if (st) return st;
   if (eager && c->sched == EMMA_RT_SCHED_GRAPH) {  // eager launches with per-kernel events
     for (int i = 0; i < ncoarse; i++) {
@@ -1621,8 +1635,8 @@ extern "C" int emma_rt_coarse_step(emma_rt_ctx* c, double aexp, int ncoarse) {
         free_cached(e);
         HIPCHK(be);
       }
-      rs = clear_call_words(c);
-      if (rs == EMMA_RT_OK) rs = run_cached(c, e, false);
+      rs = run_cached(c, e, false);
+      if (rs == EMMA_RT_OK && queue_call_end(c) != hipSuccess) rs = EMMA_RT_ERR_HIP;
       hipError_t ce = hipStreamEndCapture(c->stream, &g);
       if (rs || ce != hipSuccess) {
         if (ce == hipSuccess) (void)hipGraphDestroy(g);
@@ -1632,10 +1646,11 @@ extern "C" int emma_rt_coarse_step(emma_rt_ctx* c, double aexp, int ncoarse) {
       }
     } else {
       HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-      int rs = clear_call_words(c);
+      int rs = EMMA_RT_OK;
       const int timing = c->timing;
       c->timing = 0;  // no event records inside the graph
       for (int i = 0; i < ncoarse && rs == EMMA_RT_OK; i++) rs = recurse(c, 0, aexp);
+      if (rs == EMMA_RT_OK && queue_call_end(c) != hipSuccess) rs = EMMA_RT_ERR_HIP;
       c->timing = timing;
       hipError_t ce = hipStreamEndCapture(c->stream, &g);
       for (auto& L : c->lev) e.endpar.push_back(L.cur);
@@ -1675,7 +1690,7 @@ extern "C" int emma_rt_coarse_step(emma_rt_ctx* c, double aexp, int ncoarse) {
   }
   for (size_t k = 0; k < c->lev.size(); k++) c->lev[k].cur = it->second.endpar[k];
   c->stats.level_steps = steps_per_call(c, ncoarse);
-  return end_call(c);
+  return end_call(c, !eager);
 }
 
 extern "C" int emma_rt_set_schedule(emma_rt_ctx* c, int sched) {

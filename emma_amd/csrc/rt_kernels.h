@@ -353,4 +353,15 @@ hipError_t launch_photon_sum(const R* e, const int* child, int ncell, int ng, do
 
 hipError_t launch_fill(unsigned int* p, int n, unsigned int v, hipStream_t s);
 
+// what a call's last kernel reports into page-locked memory: the status words,
+// the summed counters (sub-steps, leaf updates, deferred leaves), then the flag
+struct CallRecord {
+  int status[3];
+  int flag;
+  unsigned long long counts[3];
+};
+// reports and clears the call words; counters null: not counted
+hipError_t launch_call_end(int* status, unsigned long long* counters, int* defer_ctl, int ndefer, CallRecord* rec,
+                           hipStream_t s);
+
 }  // namespace emma

@@ -1446,6 +1446,41 @@ __global__ void fill_kernel(unsigned int* p, int n, unsigned int v) {
   if (i < n) p[i] = v;
 }
 
+// The end of a call: one work-group sums the counter slots (a slot per thread),
+// reports them with the status words to the host and clears all call words for
+// the next call.  The flag is stored last, at system scope.
+__global__ __launch_bounds__(kCounterSlots) void call_end_kernel(int* status, unsigned long long* counters,
+                                                                 int* defer_ctl, int ndefer, CallRecord* rec) {
+  __shared__ unsigned long long red[3][kCounterSlots / 64];
+  const int t = (int)threadIdx.x;
+  if (counters != nullptr) {
+    unsigned long long* slot = counters + (size_t)t * kCounterStride;
+    unsigned long long v[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) v[k] = slot[k];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      slot[k] = 0ull;
+      for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o, 64);
+      if ((t & 63) == 0) red[k][t >> 6] = v[k];
+    }
+  }
+  for (int i = t; i < ndefer; i += kCounterSlots) defer_ctl[i] = 0;
+  __syncthreads();
+  if (t == 0) {
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      unsigned long long sum = 0ull;
+      if (counters != nullptr)
+        for (int w = 0; w < kCounterSlots / 64; w++) sum += red[k][w];
+      rec->counts[k] = sum;
+      rec->status[k] = status[k];
+      status[k] = 0;
+    }
+    __hip_atomic_store(&rec->flag, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
 // ------------------------------------------------------------------ persistent coarse step
 // The schedule's read-only tables are read through the constant address
 // space: at a wave-uniform index the loads are scalar loads, and the level
@@ -1722,6 +1757,12 @@ hipError_t launch_photon_sum(const R* e, const int* child, int ncell, int ng, do
 
 hipError_t launch_fill(unsigned int* p, int n, unsigned int v, hipStream_t s) {
   hipLaunchKernelGGL(fill_kernel, dim3((n + 255) / 256), dim3(256), 0, s, p, n, v);
+  return hipGetLastError();
+}
+
+hipError_t launch_call_end(int* status, unsigned long long* counters, int* defer_ctl, int ndefer, CallRecord* rec,
+                           hipStream_t s) {
+  hipLaunchKernelGGL(call_end_kernel, dim3(1), dim3(kCounterSlots), 0, s, status, counters, defer_ctl, ndefer, rec);
   return hipGetLastError();
 }
 
