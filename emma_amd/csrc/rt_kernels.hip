@@ -12,6 +12,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "rt_fill.h"
 #include "rt_kernels.h"
@@ -176,28 +177,32 @@ __device__ __forceinline__ void xion_times(const LevelArgs<R>& a, int cell) {
   if ((xion >= 0.5) && (a.t_first[cell] == -1)) a.t_first[cell] = a.tphy;
 }
 
-// split cell: its next state is the mean of its 8 children (rad_utils.c:1955-2006)
+// split cell: its next state is the mean of its 8 children (rad_utils.c:1955-2006);
+// group g's fields, and the cell fields
 template <typename R>
-__device__ __forceinline__ void restrict_cell(const LevelArgs<R>& a, int cell, int ch, int ng) {
+__device__ __forceinline__ void restrict_group(const LevelArgs<R>& a, int cell, int ch, int g) {
   const int n = a.ncell, nf = a.nfine, j0 = ch * 8;
-  for (int g = 0; g < ng; g++) {
-    R se = R(0), sx = R(0), sy = R(0), sz = R(0), ss = R(0);
+  R se = R(0), sx = R(0), sy = R(0), sz = R(0), ss = R(0);
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-      // plain indexing: the eight children's values merge into wide loads
-      const int j = g * nf + j0 + k;
-      se += a.fe[j] * R(0.125);
-      sx += a.ffx[j] * R(0.125);
-      sy += a.ffy[j] * R(0.125);
-      sz += a.ffz[j] * R(0.125);
-      ss += a.fsrc[j] * R(0.125);
-    }
-    gst(a.eo + g * n, cell, se);
-    gst(a.fxo + g * n, cell, sx);
-    gst(a.fyo + g * n, cell, sy);
-    gst(a.fzo + g * n, cell, sz);
-    gst(a.src + g * n, cell, ss);
+  for (int k = 0; k < 8; k++) {
+    // plain indexing: the eight children's values merge into wide loads
+    const int j = g * nf + j0 + k;
+    se += a.fe[j] * R(0.125);
+    sx += a.ffx[j] * R(0.125);
+    sy += a.ffy[j] * R(0.125);
+    sz += a.ffz[j] * R(0.125);
+    ss += a.fsrc[j] * R(0.125);
   }
+  gst(a.eo + g * n, cell, se);
+  gst(a.fxo + g * n, cell, sx);
+  gst(a.fyo + g * n, cell, sy);
+  gst(a.fzo + g * n, cell, sz);
+  gst(a.src + g * n, cell, ss);
+}
+
+template <typename R>
+__device__ __forceinline__ void restrict_scalars(const LevelArgs<R>& a, int cell, int ch) {
+  const int j0 = ch * 8;
   // (no branch inside the loop: the 32 loads go out together)
   double snp = 0., sei = 0., stp = 0., snh = 0.;
 #pragma unroll
@@ -222,6 +227,12 @@ __device__ __forceinline__ void restrict_cell(const LevelArgs<R>& a, int cell, i
     a.t_first[cell] = stf;
     a.t_last[cell] = stl;
   }
+}
+
+template <typename R>
+__device__ __forceinline__ void restrict_cell(const LevelArgs<R>& a, int cell, int ch, int ng) {
+  for (int g = 0; g < ng; g++) restrict_group(a, cell, ch, g);
+  restrict_scalars(a, cell, ch);
 }
 
 // reflux of one face flux into the coarse leaf behind it (scatterstencilrad,
@@ -292,6 +303,31 @@ __device__ __forceinline__ void fold_reflux(const LevelArgs<R>& a, int ch, int g
   }
 }
 
+// A leaf whose chemistry budget is spent (st == 1): the transported N, F are
+// stored unscaled (fscale = 1) and the cell goes on the straggler list, one
+// atomic per wave.  Returns whether it was put off.
+template <typename R>
+__device__ __forceinline__ bool defer_leaf(const LevelArgs<R>& a, int cell, int& st, int& nit) {
+  const bool deferred = st == 1;
+  const unsigned long long dm = __ballot(deferred);
+  if (dm != 0ull) {
+    const int leader = __ffsll((long long)dm) - 1;
+    int base = 0;
+    if ((int)__lane_id() == leader) base = atomicAdd(a.defer_ctl, __popcll(dm));
+    base = __shfl(base, leader);
+    if (deferred) {
+      const int slot = base + lanes_below_mask(dm);
+      if (slot < a.defer_cap)
+        a.defer_list[slot] = cell;
+      else
+        raise_status(a.status, -1, a.level, cell);  // list smaller than the level (host sizes it)
+      st = 0;
+      nit = 0;
+    }
+  }
+  return deferred;
+}
+
 // leaf cell after its transport (T: the updated state): N<0/NaN guard,
 // chemistry, write of the next state.  Returns the accepted chemistry
 // sub-steps.
@@ -330,25 +366,7 @@ __device__ __forceinline__ int finish_leaf(const LevelArgs<R>& a, const ChemCons
     st = chem_cell_fast<G>(K, ng, e, fscale, src, nhplus, eint, nh, temp, a.chemonly, nit,
                            Sub == kRefluxTiled && a.chem_budget > 0 ? a.chem_budget : -1, (double)a.chem_keep);
     if constexpr (Sub == kRefluxTiled) {
-      // budget spent: the transported N, F are stored unscaled (fscale = 1)
-      // and the cell goes on the straggler list, one atomic per wave
-      deferred = st == 1;
-      const unsigned long long dm = __ballot(deferred);
-      if (dm != 0ull) {
-        const int leader = __ffsll((long long)dm) - 1;
-        int base = 0;
-        if ((int)__lane_id() == leader) base = atomicAdd(a.defer_ctl, __popcll(dm));
-        base = __shfl(base, leader);
-        if (deferred) {
-          const int slot = base + lanes_below_mask(dm);
-          if (slot < a.defer_cap)
-            a.defer_list[slot] = cell;
-          else
-            raise_status(a.status, -1, a.level, cell);  // list smaller than the level (host sizes it)
-          st = 0;
-          nit = 0;
-        }
-      }
+      deferred = defer_leaf(a, cell, st, nit);
     }
 #pragma unroll
     for (int g = 0; g < GA; g++) {
@@ -1041,11 +1059,7 @@ __device__ __forceinline__ void tiled_step(const LevelArgs<float>& a, const Chem
   // Straight-line code (every lane loads, lanes without a halo face from
   // cell 0): a load under a divergent branch makes the wait before the
   // closures below cover it as well.
-  HaloFace<G> hf[V == kLatency ? 3 : 1];
-  if constexpr (V == kLatency) {
-#pragma unroll
-    for (int d = 0; d < 3; d++) load_face(hf[d], d);
-  }
+  HaloFace<G> hf[1];
   if constexpr (!PerDir) load_item(hf[0], lane);
   // the reflux pairs of the cell's leaving faces that have a coarse leaf
   // behind them, loaded now for the refluxing in the direction passes
@@ -1084,7 +1098,7 @@ __device__ __forceinline__ void tiled_step(const LevelArgs<float>& a, const Chem
           sShare[(g * 2 + 1) * kTileCells + lc] = make_float4(X[0], X[1], X[2], X[3]);
         }
       }
-      if constexpr (PerDir) store_item(hf[V == kLatency ? d : 0], lane);  // own slot: written and read by this lane only
+      if constexpr (PerDir) store_item(hf[0], lane);  // own slot: written and read by this lane only
       __syncthreads();
       float Rf[G][4];  // flux through a coarse face (refluxing), 0 elsewhere
       int rj = -1;     // the coarse leaf on that face
@@ -1263,12 +1277,294 @@ __global__ __launch_bounds__(kTileCells) __attribute__((amdgpu_waves_per_eu(4)))
     tiled_step<G, kListed>(args.a, args.K, tile, lds, (int)threadIdx.x);
 }
 
+// ------------------------------------------------------------------ small levels
+// A level too small to fill the GPU takes as long as one wave's chain of
+// instructions: with one cell per lane and three groups, 1,800 vector
+// instructions and two memory round trips took 13.9 us, one wave per SIMD.
+// Here a work-group owns 64 cells (8 octs) and wave g takes photon group g of
+// them, so the transport chain is a third as long and needs no barrier (a
+// wave reads only its own shares); then wave 0 runs the chemistry of the 64
+// cells while the others wait, and each wave scales and stores its group's
+// flux.  All loads go out first: topology, then the state, the leaving faces'
+// neighbours and the chemistry inputs.  The arithmetic is tiled_step's per-direction
+// form, for a neighbour in the same 32-oct tile with the rounding its own share
+// has there (own_share), for others with that of the halo (lf_share_lane), so
+// the results are the same bit for bit.
+constexpr int kSplitCells = 64;
+constexpr int kSplitOcts = kSplitCells / 8;
+
+// the share of a neighbour's state through a face normal to D: own, as
+// lf_share of a closure with X2First, otherwise as lf_share_lane
+template <int D>
+__device__ __forceinline__ void neighbour_share(bool own, float side, const float v[4], float c, float X[4]) {
+  // the two kinds of closure differ in which square of |F|^2 rounds by itself
+  const float ve = v[0], vx = v[1], vy = v[2], vz = v[3];
+  const float p = own ? vy : vx, q = own ? vx : vy;
+  const Closure<float> Q = closure_fast_f2(vx, vy, vz, ve, c, fmaf(vz, vz, fmaf(p, p, q * q)));
+  const float sc = side * c, w = Q.arg * Q.n[D];
+  X[0] = fmaf(sc, ve, v[1 + D]);
+#pragma unroll
+  for (int i = 0; i < 3; i++) {
+    float h = w * Q.n[i];
+    if (i == D) {
+      const float apart = Q.diag + h, fused = fmaf(w, Q.n[i], Q.diag);
+      h = own ? fused : apart;
+    }
+    X[1 + i] = fmaf(sc, v[1 + i], h);
+  }
+}
+
 template <int G>
-__global__ __launch_bounds__(kTileCells) __attribute__((amdgpu_waves_per_eu(2))) void level_step_tiled_latency(
-    LevelArgs<float> a_by_value, ChemConst K_by_value) {
+struct SplitLds {
+  float4 share[G][3][2][kSplitCells];  // [group][direction][A or B][cell]
+  float e[G][kSplitCells];             // transported densities
+  float fscale[G][kSplitCells];        // the chemistry's flux factors
+};
+
+template <int G>
+__global__ __launch_bounds__(64 * G) void level_step_split(LevelArgs<float> a_by_value, ChemConst K_by_value) {
   const KernArgs<float> args = kernargs<float>();
-  __shared__ TileLds<G> lds;
-  tiled_step<G, kLatency>(args.a, args.K, xcd_block(args.a.nblocks), lds, (int)threadIdx.x);
+  const LevelArgs<float>& a = args.a;
+  const ChemConst& K = args.K;
+  __shared__ SplitLds<G> lds;
+  const int g = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
+  const int tile = xcd_block(a.nblocks);
+  const int n = a.ncell;
+  const int cell = tile * kSplitCells + lane;
+  const int oct = cell >> 3, ic = cell & 7;
+  const int oct0 = tile * kSplitOcts, oct32 = oct0 & ~(kTileOcts - 1);
+  const bool valid = cell < n;
+  const bool transport = a.transport != 0;
+  const float c = a.c, dts = a.dtsurdx;
+  int ch = -1;
+  int noD[3] = {0, 0, 0};  // nei_oct entry of the face that leaves the oct, per direction
+  int pairD[3] = {-1, -1, -1};
+  float U[4] = {0.f, 0.f, 0.f, 0.f};
+  float Src[G];
+  double pre[3] = {0., 0., 1.};  // x n_H, eint, n_H
+  if (valid) {
+    ch = gld(a.child, cell);
+    if (transport) {
+#pragma unroll
+      for (int d = 0; d < 3; d++) noD[d] = gld(a.nei, oct * 6 + 2 * d + ((ic >> d) & 1));
+    }
+    U[0] = gld(a.e + g * n, cell);
+    U[1] = gld(a.fx + g * n, cell);
+    U[2] = gld(a.fy + g * n, cell);
+    U[3] = gld(a.fz + g * n, cell);
+    if (g == 0) {
+#pragma unroll
+      for (int q = 0; q < G; q++) Src[q] = gld(a.src + q * n, cell);
+      pre[0] = gld(a.nhplus, cell);
+      pre[1] = gld(a.eint, cell);
+      pre[2] = gld(a.nh, cell);
+    }
+  }
+  const bool restricted = ch >= 0 && !a.update_split;
+  if (transport) {
+    const bool moves = valid && !restricted;
+    const unsigned long long cancels = __ballot(ch >= 0 && !a.keep_split_flux);
+    auto in_wave = [&](int no) { return no >= oct0 && no < oct0 + kSplitOcts; };
+    // the leaving faces' neighbours outside the 64 cells, every load at once
+    // (lanes without one read cell 0)
+    float hv[3][4];
+    int hchild[3];
+    bool hon[3], hcoarse[3], hrefl[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      const int side = (ic >> d) & 1, no = noD[d];
+      const bool on = moves && !in_wave(no);
+      const bool bound = on && no <= kNeiReflective;  // domain face
+      const bool coarse = on && no < 0 && !bound;
+      hon[d] = on;
+      hcoarse[d] = coarse;
+      hrefl[d] = bound && no == kNeiReflective;
+      const int js = bound ? (cell & ~7) + trans_source(2 * d + side, ic)
+                           : (on && !coarse ? no * 8 + (ic ^ (1 << d)) : 0);
+      hchild[d] = gld(a.child, js);
+      if (__ballot(coarse) == 0ull) {
+        hv[d][0] = gld(a.e + g * n, js);
+        hv[d][1] = gld(a.fx + g * n, js);
+        hv[d][2] = gld(a.fy + g * n, js);
+        hv[d][3] = gld(a.fz + g * n, js);
+      } else {
+        // injected coarse leaves: the lane's array is this level's plus a
+        // per-lane distance (0, or the coarse array's address minus this
+        // level's), both bases read by scalar loads
+        const size_t o = (size_t)(coarse ? -1 - no : js) * sizeof(float);
+        auto lane_load = [&](const float* own, const float* coarser) {
+          const float* const ob = own + (size_t)g * n;
+          const float* const cb = coarser + (size_t)g * a.ncoarse;
+          const unsigned long long dist = (unsigned long long)cb - (unsigned long long)ob;
+          return *(const EMMA_GLOBAL float*)(uniform_base(ob) + (coarse ? dist : 0ull) + o);
+        };
+        hv[d][0] = lane_load(a.e, a.ce);
+        hv[d][1] = lane_load(a.fx, a.cfx);
+        hv[d][2] = lane_load(a.fy, a.cfy);
+        hv[d][3] = lane_load(a.fz, a.cfz);
+      }
+    }
+    if (valid && a.ncoarse > 0) {
+#pragma unroll
+      for (int d = 0; d < 3; d++)
+        if (noD[d] < 0) pairD[d] = gld(a.rpair, oct * 6 + 2 * d + ((ic >> d) & 1));
+    }
+    // this cell's shares of the three directions
+    const Closure<float> Q = closure_fast<true>(U[1], U[2], U[3], U[0], c);
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      float X[4];
+      lf_share_unrolled(d, 1.f, U[0], U[1], U[2], U[3], Q, c, X);
+      lds.share[g][d][0][lane] = make_float4(X[0], X[1], X[2], X[3]);
+      lf_share_unrolled(d, -1.f, U[0], U[1], U[2], U[3], Q, c, X);
+      lds.share[g][d][1][lane] = make_float4(X[0], X[1], X[2], X[3]);
+    }
+    // written and read by lanes of the same wave
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    float D[4] = {0.f, 0.f, 0.f, 0.f};
+    auto direction = [&](auto dd) {
+      constexpr int d = decltype(dd)::value;
+      const int bit = (ic >> d) & 1, jin = lane ^ (1 << d), no = noD[d];
+      const bool inW = in_wave(no);
+      const int jl = (int)(((unsigned)no - (unsigned)oct0) * 8u + (unsigned)(ic ^ (1 << d))) & (kSplitCells - 1);
+      float Rf[4] = {0.f, 0.f, 0.f, 0.f};
+      int rj = -1;
+      // the neighbour's share across the leaving face: a neighbour on the
+      // plus side contributes B, on the minus side A
+      const float4 sin = lds.share[g][d][1 - bit][jin], sout = lds.share[g][d][bit][jl];
+      if (hrefl[d]) hv[d][1 + d] = -hv[d][1 + d];
+      float X[4];
+      neighbour_share<d>(no >= oct32 && no < oct32 + kTileOcts, bit ? -1.f : 1.f, hv[d], c, X);
+      if (moves) {
+        const float Xin[4] = {sin.x, sin.y, sin.z, sin.w};
+        const float Xout[4] = {inW ? sout.x : X[0], inW ? sout.y : X[1], inW ? sout.z : X[2], inW ? sout.w : X[3]};
+        const bool cancel_in = (cancels >> jin) & 1ull;
+        const bool cancel_out = inW ? (bool)((cancels >> jl) & 1ull)
+                                    : (hon[d] && !hcoarse[d] && !a.keep_split_flux && hchild[d] >= 0);
+        const float wm = (bit ? cancel_in : cancel_out) ? 0.f : 0.5f * dts;
+        const float wp = (bit ? cancel_out : cancel_in) ? 0.f : -0.5f * dts;
+        const bool coarse_face = hcoarse[d];
+        const float4 Ag = lds.share[g][d][0][lane], Bg = lds.share[g][d][1][lane];
+        const float A[4] = {Ag.x, Ag.y, Ag.z, Ag.w}, B[4] = {Bg.x, Bg.y, Bg.z, Bg.w};
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          const float Fm = (bit ? Xin[v] : Xout[v]) + B[v];
+          const float Fp = A[v] + (bit ? Xout[v] : Xin[v]);
+          D[v] = fmaf(Fp, wp, fmaf(Fm, wm, D[v]));
+          if (coarse_face) Rf[v] = bit ? Fp : Fm;
+        }
+        if (coarse_face) rj = -1 - no;
+      }
+      // refluxing, as in tiled_step
+      const unsigned long long rmask = __ballot(rj >= 0);
+      if (rmask != 0ull) {
+        const int b1 = 1 << ((d + 1) % 3), b2 = 1 << ((d + 2) % 3);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          float x = Rf[v];
+          x += lane_xor(x, b1);
+          x += lane_xor(x, b2);
+          Rf[v] = x;
+        }
+        const int l0 = lane & ~(b1 | b2);
+        const unsigned long long grp =
+            (1ull << l0) | (1ull << (l0 | b1)) | (1ull << (l0 | b2)) | (1ull << (l0 | b1 | b2));
+        const unsigned long long mine = rmask & grp;
+        const int pr = pairD[d];
+        if (rj >= 0 && pr >= 0) {
+          float* acc = a.cracc + (size_t)pr * kRefluxTiled * 4 * G + g;
+          const float w = (bit ? 1.f : -1.f) * (0.5f * dts) * 0.125f;  // pow(-1, face+1) dt/dx / 8, shares doubled
+          if (mine == grp) {
+            const int k = __popcll(mine & ((1ull << lane) - 1ull));  // component of this lane
+            const float x = k == 0 ? Rf[0] : (k == 1 ? Rf[1] : (k == 2 ? Rf[2] : Rf[3]));
+            atomicAdd(acc + k * G, x * w);
+          } else if (lane == __builtin_ctzll(mine)) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) atomicAdd(acc + v * G, Rf[v] * w);
+          }
+        }
+      }
+    };
+    direction(std::integral_constant<int, 0>());
+    direction(std::integral_constant<int, 1>());
+    direction(std::integral_constant<int, 2>());
+    if (valid && !restricted) {
+      if (ch <= -2) fold_reflux<float, G, 1, kRefluxTiled>(a, ch, g, 1, &U[0], &U[1], &U[2], &U[3]);
+#pragma unroll
+      for (int v = 0; v < 4; v++) U[v] += D[v];
+    }
+  } else if (valid && !restricted && ch <= -2) {
+    fold_reflux<float, G, 1, kRefluxTiled>(a, ch, g, 1, &U[0], &U[1], &U[2], &U[3]);
+  }
+  const bool leaf = valid && ch < 0;
+  if (G > 1) {
+    lds.e[g][lane] = U[0];
+    __syncthreads();
+  }
+  if (g == 0) {
+    if (valid && a.t_first != nullptr) xion_times(a, cell);
+    int nit = 0;
+    if (leaf) {
+      double e[G], src[G], fscale[G];
+#pragma unroll
+      for (int q = 0; q < G; q++) {
+        e[q] = (double)(G > 1 ? lds.e[q][lane] : U[0]);
+        src[q] = (double)Src[q];
+      }
+      if (e[0] < 0 || isnan(e[0]) || isnan(G > 1 ? e[G > 1 ? 1 : 0] : (double)U[1]))
+        raise_status(a.status, -3, a.level, cell);
+      double nhplus = pre[0], eint = pre[1], temp = 0.;
+      int st = chem_cell_fast<G>(K, G, e, fscale, src, nhplus, eint, pre[2], temp, a.chemonly, nit,
+                                 a.chem_budget > 0 ? a.chem_budget : -1, (double)a.chem_keep);
+      const bool deferred = defer_leaf(a, cell, st, nit);
+      if (st != 0) raise_status(a.status, st, a.level, cell);
+#pragma unroll
+      for (int q = 0; q < G; q++) {
+        float ev = (float)e[q];
+        if (!deferred && e[q] >= K.emin_grp[q] && ev < K.emin_grp_up[q]) ev = K.emin_grp_up[q];
+        gst(a.eo + q * n, cell, ev);
+        lds.fscale[q][lane] = (float)fscale[q];
+      }
+      gst(a.nhpluso, cell, nhplus);
+      gst(a.einto, cell, eint);
+      gst(a.tempo, cell, temp);
+    } else if (valid && restricted) {
+      restrict_scalars(a, cell, ch);
+    } else if (valid) {  // COARSERAD: a split cell with its transported state
+      gst(a.nhpluso, cell, gld(a.nhplus, cell));
+      gst(a.einto, cell, gld(a.eint, cell));
+      gst(a.tempo, cell, gld(a.temp, cell));
+    }
+    if (a.counters != nullptr) {
+      const unsigned long long lb = __ballot(leaf);
+      unsigned int s0 = 0;
+#pragma unroll
+      for (int b = 0; b < 4; b++) s0 += (unsigned int)__popcll(__ballot(((unsigned)nit >> b) & 1u)) << b;
+      unsigned long long* slot = a.counters + (size_t)(blockIdx.x % kCounterSlots) * kCounterStride;
+      if (nit >= 16) atomicAdd(slot, (unsigned long long)((unsigned)nit & ~15u));
+      if (lane == 0) {
+        atomicAdd(slot + 0, (unsigned long long)s0);
+        atomicAdd(slot + 1, (unsigned long long)__popcll(lb));
+      }
+    }
+  }
+  if (valid && restricted) restrict_group(a, cell, ch, g);  // meanwhile: split cells wait for nothing
+  if (G > 1) __syncthreads();
+  if (leaf) {
+    const float fs = lds.fscale[g][lane];
+    gst(a.fxo + g * n, cell, U[1] * fs);
+    gst(a.fyo + g * n, cell, U[2] * fs);
+    gst(a.fzo + g * n, cell, U[3] * fs);
+  } else if (valid && !restricted) {
+    gst(a.eo + g * n, cell, U[0]);
+    gst(a.fxo + g * n, cell, U[1]);
+    gst(a.fyo + g * n, cell, U[2]);
+    gst(a.fzo + g * n, cell, U[3]);
+    if ((g == 0 && (U[0] < 0.f || isnan(U[0]) || (G == 1 && isnan(U[1])))) || (g == 1 && isnan(U[0])))
+      raise_status(a.status, -3, a.level, cell);
+  }
 }
 
 // ------------------------------------------------------------------ chemistry stragglers
@@ -1636,6 +1932,12 @@ __global__ __launch_bounds__(kTileCells) __attribute__((amdgpu_waves_per_eu(Tile
 }
 
 // ------------------------------------------------------------------ launchers
+template <int G>
+static void launch_split(LevelArgs<float> a, const ChemConst& K, hipStream_t s) {
+  a.nblocks = ((a.ncell + kSplitCells - 1) / kSplitCells + 7) & ~7;
+  hipLaunchKernelGGL((level_step_split<G>), dim3(a.nblocks), dim3(64 * G), 0, s, a, K);
+}
+
 template <typename R>
 hipError_t launch_level_step(const LevelArgs<R>& a0, const ChemConst& K, hipStream_t s) {
   LevelArgs<R> a = a0;
@@ -1654,7 +1956,7 @@ hipError_t launch_level_step(const LevelArgs<R>& a0, const ChemConst& K, hipStre
           sb(kStragglerThreads);
       if (a.ng == 1) {
         if (v == kLatency)
-          hipLaunchKernelGGL((level_step_tiled_latency<1>), dim3(nb), dim3(kTileCells), 0, s, a, K);
+          launch_split<1>(a, K, s);
         else if (v == kPerDir)
           hipLaunchKernelGGL((level_step_tiled<1, true>), dim3(nb), dim3(kTileCells), 0, s, a, K);
         else
@@ -1662,7 +1964,7 @@ hipError_t launch_level_step(const LevelArgs<R>& a0, const ChemConst& K, hipStre
         if (defer) hipLaunchKernelGGL((chem_straggler_kernel<1>), sg, sb, 0, s, a, K);
       } else {
         if (v == kLatency)
-          hipLaunchKernelGGL((level_step_tiled_latency<3>), dim3(nb), dim3(kTileCells), 0, s, a, K);
+          launch_split<3>(a, K, s);
         else if (v == kPerDir)
           hipLaunchKernelGGL((level_step_tiled<3, true>), dim3(nb), dim3(kTileCells), 0, s, a, K);
         else

@@ -46,13 +46,11 @@ __device__ __forceinline__ double fdiv64(double a, double b) {
 // closure would round differently in two kernels.  X2First: the x term is the
 // one rounded by itself (a tile's own cells in the tiled kernel); otherwise
 // the y term (its halo cells, and the per-cell kernels).
-template <bool X2First = false>
-__device__ __forceinline__ Closure<float> closure_fast(float fx, float fy, float fz, float ee, float c) {
+__device__ __forceinline__ Closure<float> closure_fast_f2(float fx, float fy, float fz, float ee, float c, float f2) {
 #pragma clang fp contract(fast)
   // branch-free: the isotropic case (E <= 0 or F = 0: n = 0, f = 0) by selects
   Closure<float> q;
   const float c2e = ee * c * c;
-  const float f2 = X2First ? fmaf(fz, fz, fmaf(fy, fy, fx * fx)) : fmaf(fz, fz, fmaf(fx, fx, fy * fy));
   const bool aniso = (ee > 0.f) & (f2 > 1e-36f);
   const float ri = aniso ? __builtin_amdgcn_rsqf(f2) : 0.f;
   q.n[0] = fx * ri;
@@ -65,6 +63,11 @@ __device__ __forceinline__ Closure<float> closure_fast(float fx, float fy, float
   q.diag = c2e * (clamped ? 0.2f * (1.f - 2.f * ff2) : (s - 1.f) * (1.f / 3.f));
   q.arg = c2e * (clamped ? 0.2f * (2.f + 6.f * ff2) : 2.f - s);
   return q;
+}
+template <bool X2First = false>
+__device__ __forceinline__ Closure<float> closure_fast(float fx, float fy, float fz, float ee, float c) {
+  const float f2 = X2First ? fmaf(fz, fz, fmaf(fy, fy, fx * fx)) : fmaf(fz, fz, fmaf(fx, fx, fy * fy));
+  return closure_fast_f2(fx, fy, fz, ee, c, f2);
 }
 
 // the rate fits of chem_utils.c:37-187 in FP32: pow(x, a) = exp2(a log2 x)
@@ -322,29 +325,6 @@ __device__ int chem_cell_fast(const ChemConst& K, int ng, double* e, double* fsc
   if (st != 0) return st;
   chem_fast_end<G>(K, ng, chemonly, s, e, fscale, nhplus, eint_code, temp);
   return 0;
-}
-
-// the Lax-Friedrichs face flux of lf_flux with contraction allowed (mixed path)
-__device__ __forceinline__ void lf_flux_fast(int d, int s, float Ue, float Ux, float Uy, float Uz,
-                                             const Closure<float>& qu, float Ve, float Vx, float Vy, float Vz,
-                                             const Closure<float>& qv, float hc, float F[4]) {
-#pragma clang fp contract(fast)
-  const float Me = s ? Ue : Ve, Pe = s ? Ve : Ue;
-  const float Mf[3] = {s ? Ux : Vx, s ? Uy : Vy, s ? Uz : Vz};
-  const float Pf[3] = {s ? Vx : Ux, s ? Vy : Uy, s ? Vz : Uz};
-  const Closure<float>& qm = s ? qu : qv;
-  const Closure<float>& qp = s ? qv : qu;
-  F[0] = 0.5f * (Pf[d] + Mf[d]) + hc * (Me - Pe);
-  const float wp = qp.arg * qp.n[d], wm = qm.arg * qm.n[d];
-#pragma unroll
-  for (int i = 0; i < 3; i++) {
-    float pp = wp * qp.n[i], pm = wm * qm.n[i];
-    if (i == d) {
-      pp += qp.diag;
-      pm += qm.diag;
-    }
-    F[1 + i] = 0.5f * (pp + pm) + hc * (Mf[i] - Pf[i]);
-  }
 }
 
 // Twice one side's share of the Lax-Friedrichs face flux in direction D.
