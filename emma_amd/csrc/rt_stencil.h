@@ -23,10 +23,11 @@ bool rgrid_layout(int ngrp, int real_bytes, RgridLayout* out);
 
 // coarserad: the COARSERAD build's sweeps and update (split neighbours'
 // fluxes kept, split cells updated); transport: condadvec, the sweeps and the
-// update run at all (rad_utils_gpu.cu:1058-1075)
+// update run at all (rad_utils_gpu.cu:1058-1075); direct: the records lie in
+// page-locked host memory (its device address), aligned to 16 bytes
 hipError_t launch_stencil(void* d_stencil, const RgridLayout& L, int ngrp, int real_bytes, int nread, double c,
                           double dtsurdx, int chemonly, int coarserad, int transport, const ChemConst& K,
-                          int* status, unsigned long long* counters, hipStream_t s);
+                          int* status, unsigned long long* counters, bool direct, hipStream_t s);
 
 void stencil_free(void* p);
 

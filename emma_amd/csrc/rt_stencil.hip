@@ -175,11 +175,221 @@ __global__ __launch_bounds__(256) void stencil_kernel(char* base, StencilGeo geo
   }
 }
 
+// ---- the batch read and written in place, in page-locked host memory
+// The copies of a batch into a device buffer (one for the oct slots, eight
+// strided ones for the centre cells' rfieldnew) and back (eight) ran one
+// after the other around the kernel: 8192 records with one FP64 group took
+// 1.97 ms, of which the kernel 0.2 and the wire 0.7.  PCIe is the bound, so
+// the kernel itself reads what it needs through the mapping and writes what it
+// changes, and the transfers of different work-groups overlap in both
+// directions.  A wave owns 8 octs, one cell a lane.  All host accesses are
+// consecutive over the lanes (scattered ones would each cost a bus
+// transaction): the 32 cells an oct's update reads (its own and the 24 that
+// face it; 56 are stored) and the centre cells' rfieldnew go to LDS first, and
+// the results leave through LDS the same way.  Arithmetic of stencil_kernel.
+template <typename R, int G>
+struct DirectShape {
+  static constexpr int kRtype = 5 * G + 4;        // REALs of a struct Rtype
+  static constexpr int kLight = kRtype + 1;       // of a CELLLIGHT_R (its split flag padded)
+  static constexpr int kOut = kRtype + 30 * G;    // rfieldnew, rflux: consecutive in a CELLFLUX_R
+  // an oct's REALs in LDS: the 32 cells, rfieldnew of its cells, and the
+  // fluxes of their faces inside the oct.  A facing cell has one reader, so
+  // the flux through that face takes its place.
+  static constexpr int kOct = 32 * kLight + 8 * kRtype + 8 * 15 * G;
+  // octs of a work-group: eight fill the wave; four where eight need more
+  // than half a CU's LDS
+  static constexpr int kOcts = 8 * kOct * (int)sizeof(R) <= 80 * 1024 ? 8 : 4;
+};
+
+// the cell of slot f that faces cell k (0..3) of the oct's side: its bit d is
+// the side's opposite, k gives the other two bits
+__device__ __forceinline__ int facing_cell(int f, int k) {
+  const int d = f >> 1, s = f & 1, low = k & ((1 << d) - 1);
+  return ((k >> d) << (d + 1)) | ((1 - s) << d) | low;
+}
+// and k of a cell of that slot
+__device__ __forceinline__ int facing_index(int f, int cc) {
+  const int d = f >> 1;
+  return (cc & ((1 << d) - 1)) | ((cc >> (d + 1)) << d);
+}
+
+template <typename R, int G>
+__global__ __launch_bounds__(64) void stencil_direct_kernel(char* base, StencilGeo geo, int nread, R c, R hc, R dts,
+                                                            int chemonly, StencilMode mode, ChemConst K, int* status,
+                                                            unsigned long long* counters) {
+  using S = DirectShape<R, G>;
+  __shared__ R lds[S::kOcts * S::kOct];
+  const int lane = (int)threadIdx.x;
+  const int first = (int)blockIdx.x * S::kOcts;
+  const int nocts = min(S::kOcts, nread - first);
+  char* rec0 = base + (size_t)first * geo.rgrid;
+  // cells: [oct][0..7 its own, 8 + 4 f + k facing][REAL], then rfieldnew:
+  // [oct][cell][REAL], then fluxes: [oct][cell][direction][5 G]
+  R* sCell = lds;
+  R* sNew = lds + S::kOcts * 32 * S::kLight;
+  R* sFlux = sNew + S::kOcts * 8 * S::kRtype;
+  // several loads in flight per lane: a read over the bus takes microseconds
+  auto fetch = [&](int count, R* to, auto&& from) {
+    constexpr int kFly = 8;
+    for (int i0 = lane; i0 < count; i0 += 64 * kFly) {
+      R v[kFly];
+#pragma unroll
+      for (int u = 0; u < kFly; u++)
+        if (i0 + 64 * u < count) v[u] = *from(i0 + 64 * u);
+#pragma unroll
+      for (int u = 0; u < kFly; u++)
+        if (i0 + 64 * u < count) to[i0 + 64 * u] = v[u];
+    }
+  };
+  if (mode.transport) {
+    fetch(nocts * 32 * S::kLight, sCell, [&](int i) {
+      const int o = i / (32 * S::kLight), r = i - o * (32 * S::kLight);
+      const int q = r / S::kLight, w = r - q * S::kLight;
+      const int f = (q - 8) >> 2;
+      const int slot = q < 8 ? 6 : f, cc = q < 8 ? q : facing_cell(f, (q - 8) & 3);
+      return (const R*)(rec0 + (size_t)o * geo.rgrid + geo.oct + slot * geo.octlight + cc * geo.celllight) + w;
+    });
+  } else {  // no fluxes: the centre cells' split flags only (their last REAL)
+    for (int i = lane; i < nocts * 8; i += 64) {
+      const int o = i >> 3, q = i & 7;
+      sCell[(o * 32 + q) * S::kLight + S::kRtype] =
+          ((const R*)(rec0 + (size_t)o * geo.rgrid + geo.oct + 6 * geo.octlight + q * geo.celllight))[S::kRtype];
+    }
+  }
+  fetch(nocts * 8 * S::kRtype, sNew, [&](int i) {
+    const int q = i / S::kRtype, w = i - q * S::kRtype;
+    return (const R*)(rec0 + (size_t)(q >> 3) * geo.rgrid + geo.New + (q & 7) * geo.cellflux + geo.rfieldnew) + w;
+  });
+  __syncthreads();
+  const int o = lane >> 3, ic = lane & 7;
+  const bool on = o < nocts;
+  auto split_of = [&](int q) { return *(const char*)&sCell[(o * 32 + q) * S::kLight + S::kRtype] != 0; };
+  const bool split = on && split_of(ic);
+  bool stop = !on;  // nothing more to do: no cell, or a split one that keeps its state
+  R* n = &sNew[(o * 8 + ic) * S::kRtype];
+  if (on && mode.transport) {
+    const R* C = &sCell[(o * 32 + ic) * S::kLight];
+    R De[G], Dx[G], Dy[G], Dz[G];
+    Closure<R> Q[G];
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+      Q[g] = closure<R>(C[G + g], C[2 * G + g], C[3 * G + g], C[g], c);
+      De[g] = Dx[g] = Dy[g] = Dz[g] = R(0);
+    }
+#pragma unroll
+    for (int f = 0; f < 6; f++) {
+      const int d = f >> 1, s = f & 1;
+      const int nc = ic ^ (1 << d);
+      const int q = (((ic >> d) & 1) != s) ? nc : 8 + 4 * f + facing_index(f, nc);  // getcellnei, oct.c:116-185
+      R* N = &sCell[(o * 32 + q) * S::kLight];
+      R F[G][4];
+      const R ffact = (!mode.keep_split_flux && split_of(q)) ? R(0) : R(1);
+      const R one = (f & 1) ? R(-1) : R(1);
+#pragma unroll
+      for (int g = 0; g < G; g++) {
+        const R ve = N[g], vx = N[G + g], vy = N[2 * G + g], vz = N[3 * G + g];
+        const Closure<R> qn = closure<R>(vx, vy, vz, ve, c);
+        lf_flux<R>(d, s, C[g], C[G + g], C[2 * G + g], C[3 * G + g], Q[g], ve, vx, vy, vz, qn, hc, F[g]);
+#pragma unroll
+        for (int v = 0; v < 4; v++) F[g][v] *= ffact;
+        De[g] += F[g][0] * dts * one;
+        Dx[g] += F[g][1] * dts * one;
+        Dy[g] += F[g][2] * dts * one;
+        Dz[g] += F[g][3] * dts * one;
+      }
+      R* out = q >= 8 ? N : &sFlux[((o * 8 + ic) * 3 + d) * 5 * G];
+#pragma unroll
+      for (int g = 0; g < G; g++) {
+#pragma unroll
+        for (int v = 0; v < 4; v++) out[g * 5 + v] = F[g][v];
+        out[g * 5 + 4] = R(0);
+      }
+    }
+    stop = split && !mode.update_split;  // updatefieldrad and chemrad skip split cells
+    if (!stop) {
+#pragma unroll
+      for (int g = 0; g < G; g++) {
+        n[g] += De[g];
+        n[G + g] += Dx[g];
+        n[2 * G + g] += Dy[g];
+        n[3 * G + g] += Dz[g];
+      }
+      const double e0 = (double)n[0], e1 = (double)n[1];  // e[1], or fx[0] with one group
+      if ((e0 < 0 || isnan(e0) || isnan(e1)) && atomicCAS(status, 0, -3) == 0) {
+        status[1] = -1;
+        status[2] = (first + o) * 8 + ic;
+      }
+      stop = split;  // COARSERAD: the split cell keeps its transported state, no chemistry
+    }
+  } else if (on) {
+    stop = split;
+  }
+  if (!stop) {
+    double e[G], fx[G], fy[G], fz[G], src[G];
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+      e[g] = (double)n[g];
+      fx[g] = (double)n[G + g];
+      fy[g] = (double)n[2 * G + g];
+      fz[g] = (double)n[3 * G + g];
+      src[g] = (double)n[4 * G + g];
+    }
+    double nhplus = (double)n[5 * G], eint = (double)n[5 * G + 1];
+    const double nh = (double)n[5 * G + 2];
+    double temp = 0.;
+    int nit = 0;
+    const int st = chem_cell<G>(K, G, e, fx, fy, fz, src, nhplus, eint, nh, temp, chemonly, nit);
+    if (st != 0 && atomicCAS(status, 0, st) == 0) {
+      status[1] = -1;
+      status[2] = (first + o) * 8 + ic;
+    }
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+      n[g] = (R)e[g];
+      n[G + g] = (R)fx[g];
+      n[2 * G + g] = (R)fy[g];
+      n[3 * G + g] = (R)fz[g];
+    }
+    n[5 * G] = (R)nhplus;
+    n[5 * G + 1] = (R)eint;
+    n[5 * G + 3] = (R)temp;
+    if (counters != nullptr) {
+      unsigned long long* slot = counters + (size_t)(blockIdx.x % kCounterSlots) * kCounterStride;
+      atomicAdd(slot + 0, (unsigned long long)nit);
+      atomicAdd(slot + 1, 1ull);
+    }
+  }
+  // results, consecutive over the lanes: per cell rfieldnew, then the six
+  // fluxes where they were formed
+  __syncthreads();
+  const int nout = mode.transport ? S::kOut : S::kRtype;
+  for (int i = lane; i < nocts * 8 * nout; i += 64) {
+    const int q = i / nout, w = i - q * nout;
+    const int oo = q >> 3, cc = q & 7;
+    R v;
+    if (w < S::kRtype) {
+      v = sNew[q * S::kRtype + w];
+    } else {
+      const int f = (w - S::kRtype) / (5 * G), r = w - S::kRtype - f * 5 * G;
+      const int d = f >> 1, s = f & 1;
+      v = (((cc >> d) & 1) != s) ? sFlux[(q * 3 + d) * 5 * G + r]
+                                 : sCell[(oo * 32 + 8 + 4 * f + facing_index(f, cc)) * S::kLight + r];
+    }
+    ((R*)(rec0 + (size_t)oo * geo.rgrid + geo.New + cc * geo.cellflux + geo.rfieldnew))[w] = v;
+  }
+}
+
 template <typename R, int G>
 static hipError_t launch_g(void* d, const StencilGeo& geo, int nread, double c, double dts, int chemonly,
-                           StencilMode m, const ChemConst& K, int* status, unsigned long long* counters,
+                           StencilMode m, const ChemConst& K, int* status, unsigned long long* counters, bool direct,
                            hipStream_t s) {
   const int n = nread * 8;
+  if (direct) {
+    constexpr int octs = DirectShape<R, G>::kOcts;
+    hipLaunchKernelGGL((stencil_direct_kernel<R, G>), dim3((nread + octs - 1) / octs), dim3(64), 0, s, (char*)d, geo,
+                       nread, (R)c, (R)(0.5 * c), (R)dts, chemonly, m, K, status, counters);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL((stencil_kernel<R, G>), dim3((n + 255) / 256), dim3(256), 0, s, (char*)d, geo, nread, (R)c,
                      (R)(0.5 * c), (R)dts, chemonly, m, K, status, counters);
   return hipGetLastError();
@@ -187,25 +397,25 @@ static hipError_t launch_g(void* d, const StencilGeo& geo, int nread, double c, 
 
 template <typename R>
 static hipError_t launch_r(void* d, const StencilGeo& geo, int ngrp, int nread, double c, double dts, int chemonly,
-                           StencilMode m, const ChemConst& K, int* status, unsigned long long* counters,
+                           StencilMode m, const ChemConst& K, int* status, unsigned long long* counters, bool direct,
                            hipStream_t s) {
   switch (ngrp) {
-    case 1: return launch_g<R, 1>(d, geo, nread, c, dts, chemonly, m, K, status, counters, s);
-    case 2: return launch_g<R, 2>(d, geo, nread, c, dts, chemonly, m, K, status, counters, s);
-    case 3: return launch_g<R, 3>(d, geo, nread, c, dts, chemonly, m, K, status, counters, s);
-    case 4: return launch_g<R, 4>(d, geo, nread, c, dts, chemonly, m, K, status, counters, s);
-    case 5: return launch_g<R, 5>(d, geo, nread, c, dts, chemonly, m, K, status, counters, s);
-    case 6: return launch_g<R, 6>(d, geo, nread, c, dts, chemonly, m, K, status, counters, s);
-    case 7: return launch_g<R, 7>(d, geo, nread, c, dts, chemonly, m, K, status, counters, s);
-    case 8: return launch_g<R, 8>(d, geo, nread, c, dts, chemonly, m, K, status, counters, s);
-    case 9: return launch_g<R, 9>(d, geo, nread, c, dts, chemonly, m, K, status, counters, s);
+    case 1: return launch_g<R, 1>(d, geo, nread, c, dts, chemonly, m, K, status, counters, direct, s);
+    case 2: return launch_g<R, 2>(d, geo, nread, c, dts, chemonly, m, K, status, counters, direct, s);
+    case 3: return launch_g<R, 3>(d, geo, nread, c, dts, chemonly, m, K, status, counters, direct, s);
+    case 4: return launch_g<R, 4>(d, geo, nread, c, dts, chemonly, m, K, status, counters, direct, s);
+    case 5: return launch_g<R, 5>(d, geo, nread, c, dts, chemonly, m, K, status, counters, direct, s);
+    case 6: return launch_g<R, 6>(d, geo, nread, c, dts, chemonly, m, K, status, counters, direct, s);
+    case 7: return launch_g<R, 7>(d, geo, nread, c, dts, chemonly, m, K, status, counters, direct, s);
+    case 8: return launch_g<R, 8>(d, geo, nread, c, dts, chemonly, m, K, status, counters, direct, s);
+    case 9: return launch_g<R, 9>(d, geo, nread, c, dts, chemonly, m, K, status, counters, direct, s);
     default: return hipErrorInvalidValue;
   }
 }
 
 hipError_t launch_stencil(void* d, const RgridLayout& L, int ngrp, int rb, int nread, double c, double dtsurdx,
                           int chemonly, int coarserad, int transport, const ChemConst& K, int* status,
-                          unsigned long long* counters, hipStream_t s) {
+                          unsigned long long* counters, bool direct, hipStream_t s) {
   StencilMode m;
   m.transport = transport;
   m.keep_split_flux = coarserad;
@@ -220,8 +430,8 @@ hipError_t launch_stencil(void* d, const RgridLayout& L, int ngrp, int rb, int n
   geo.cellflux = L.v[12];
   geo.rfieldnew = L.v[15];
   geo.rflux = L.v[16];
-  if (rb == 8) return launch_r<double>(d, geo, ngrp, nread, c, dtsurdx, chemonly, m, K, status, counters, s);
-  return launch_r<float>(d, geo, ngrp, nread, c, dtsurdx, chemonly, m, K, status, counters, s);
+  if (rb == 8) return launch_r<double>(d, geo, ngrp, nread, c, dtsurdx, chemonly, m, K, status, counters, direct, s);
+  return launch_r<float>(d, geo, ngrp, nread, c, dtsurdx, chemonly, m, K, status, counters, direct, s);
 }
 
 void stencil_free(void* p) {

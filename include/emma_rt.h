@@ -145,11 +145,12 @@ int emma_rt_destroy_pinned_stencil(void *stencil);
 int emma_rt_alloc_pinned(size_t bytes, void **out);
 /* rad_utils_gpu.cu:1054-1086: copy `nread` RGRIDs of `level` host->device,
    run rad_sweepX/Y/Z + updatefieldrad + chemrad semantics (CPU semantics of
-   rad_utils.c/chem_utils.c), copy back.  Only the parts the kernel reads (oct
-   slots, New.cell[*].rfieldnew) go to the device and only New.cell[*].rfieldnew
-   and rflux, the parts that change, come back.  `stencil` is host memory in
-   the reference's RGRID layout (page-locked memory from
-   emma_rt_create_pinned_stencil is fastest).  In EMMA_RT_COARSERAD mode
+   rad_utils.c/chem_utils.c), copy back.  Of the records only
+   New.cell[*].rfieldnew and rflux change.  `stencil` is host memory in the
+   reference's RGRID layout.  Page-locked records aligned to 16 bytes (from
+   emma_rt_create_pinned_stencil) are read and written in place by the kernel,
+   and only the parts it needs cross the bus; records in ordinary memory go to
+   the device buffer and back whole, at less than a third of the rate.  In EMMA_RT_COARSERAD mode
    (emma_rt_set_mode) the batch follows the COARSERAD build: the sweeps and
    the update run only when level == params.lcoarse and !chemonly (condadvec,
    rad_utils.c:1808-1812), fluxes of split neighbours are kept and split
@@ -161,8 +162,8 @@ int emma_rt_advance_stencil(emma_rt_ctx *ctx, void *stencil, int nread, int leve
 /* emma_rt_advance_stencil without the device buffer of
    emma_rt_create_radstencil: for callers that cannot allocate device memory
    (code under HIP graph capture, serving loops, harnesses that forbid
-   hipMalloc).  No counterpart in the reference.  The batch is staged in a
-   static device area of EMMA_RT_NOALLOC_STENCIL_BYTES per GPU (allocated with
+   hipMalloc).  No counterpart in the reference.  A batch in ordinary memory is
+   staged in a static device area of EMMA_RT_NOALLOC_STENCIL_BYTES per GPU (allocated with
    the library's code object, held until the process ends); the call allocates
    nothing.  nread * sizeof(struct RGRID) beyond that size (e.g. 4128 records
    at NGRP=1, 1826 at NGRP=3, REAL=double) returns EMMA_RT_ERR_ARG.  real_bytes
