@@ -614,220 +614,312 @@ __device__ __forceinline__ void cell_step(const LevelArgs<R>& a, const ChemConst
 // from there, and only the halo (a third to a half of the leaving faces on a
 // complete level) is evaluated again: on complete levels (variant kListed) one
 // listed halo face per lane in one round, on sparse ones each lane its own
-// leaving face in each direction pass.  One group at a time keeps the LDS at
-// 37 KB (FP64; 18 KB FP32) whatever the group count, and only the transported
-// state of the other groups live across the passes.
+// leaving face in each direction pass.
 template <typename R>
 __device__ __forceinline__ CellLds<R>* cell_lds() {
   __shared__ CellLds<R> lds;
   return &lds;
 }
 
-template <typename R, int G, bool Fast>
-__device__ __forceinline__ void cell_step_lds(const LevelArgs<R>& a, const ChemConst& K, int tile, int lc,
-                                              CellLds<R>& lds) {
-  constexpr int GA = (G == 1 || G == 3) ? G : kMaxGrp;  // groups of a reflux accumulator
-  const int n = a.ncell;
+// what a thread's cell needs for the transport of any group
+struct CellFaces {
+  int cell, ch;
+  int noD[3];    // nei_oct entry of the face that leaves the oct, per direction
+  int pairD[3];  // its reflux pair where a coarse leaf lies behind it, -1 elsewhere
+  bool valid, restricted, moves, listed;
+  unsigned long long hball[3];  // listed: lanes whose face in direction d is a halo face,
+  int hbase[3];                 // and the first halo slot of direction d
+};
+
+// where the neighbour across a halo face lies
+struct HaloCell {
+  int j, d;
+  bool on, coarse, refl;
+};
+
+// the halo face in direction d of cell hcell, nei_oct entry no
+__device__ __forceinline__ HaloCell halo_cell(bool on, int hcell, int d, int no) {
+  HaloCell h;
+  const int hic = hcell & 7, side = (hic >> d) & 1;
+  const bool bound = on && no <= kNeiReflective;  // domain face (rad_utils.c:1106-1213, 1376-1407)
+  h.on = on;
+  h.d = d;
+  h.coarse = on && no < 0 && !bound;
+  h.refl = bound && no == kNeiReflective;
+  h.j = !on ? 0 : bound ? (hcell & ~7) + trans_source(2 * d + side, hic) : h.coarse ? -1 - no : no * 8 + (hic ^ (1 << d));
+  return h;
+}
+
+// the flux from a split neighbour is dropped (RADSTEP)
+template <typename R>
+__device__ __forceinline__ bool halo_cancel(const LevelArgs<R>& a, const HaloCell& h) {
+  return h.on && !h.coarse && !a.keep_split_flux && gld(a.child, h.j) >= 0;
+}
+
+// group g of its state into LDS slot i, with its closure
+template <typename R, bool Fast>
+__device__ __forceinline__ void halo_put(const LevelArgs<R>& a, CellLds<R>& lds, const HaloCell& h, int g, int i) {
+  if (!h.on) return;
+  // the lane's array is this level's plus a per-lane distance (0, or the
+  // coarse array's address minus this level's), both bases scalar: a 64-bit
+  // address per lane and array would live across the group loop
+  const size_t o = byte_offset<R>(h.j);
+  auto load = [&](const R* own, const R* coarser) {
+    const R* const ob = own + (size_t)g * a.ncell;
+    const R* const cb = coarser + (size_t)g * a.ncoarse;
+    const unsigned long long dist = (unsigned long long)cb - (unsigned long long)ob;
+    return *(const EMMA_GLOBAL R*)(uniform_base(ob) + (h.coarse ? dist : 0ull) + o);
+  };
+  const R ve = load(a.e, a.ce);
+  R vx = load(a.fx, a.cfx), vy = load(a.fy, a.cfy), vz = load(a.fz, a.cfz);
+  if (h.refl) {
+    if (h.d == 0) vx = -vx;
+    if (h.d == 1) vy = -vy;
+    if (h.d == 2) vz = -vz;
+  }
+  lds.put(i, ve, vx, vy, vz, closure_of<R, Fast>(vx, vy, vz, ve, a.c));
+}
+
+__device__ __forceinline__ bool in_tile32(int no, int tile) {
+  return no >= tile * kTileOcts && no < (tile + 1) * kTileOcts;
+}
+
+// the tile's cancel flags and, on complete levels, each wave's halo list (this
+// lane's entry in hl); before the first group's transport
+template <typename R>
+__device__ __forceinline__ CellFaces cell_faces(const LevelArgs<R>& a, int tile, int lc, CellLds<R>& lds, HaloCell& hl) {
+  CellFaces c;
   const int wv = lc >> 6, lane = lc & 63;
-  const int cell = tile * kTileCells + lc;
-  const int oct0 = tile * kTileOcts;
-  const int oct = cell >> 3, ic = cell & 7;
-  const bool valid = cell < n;
+  c.cell = tile * kTileCells + lc;
+  const int oct = c.cell >> 3, ic = c.cell & 7;
+  c.valid = c.cell < a.ncell;
+  c.listed = a.variant == kListed;
+  c.ch = -1;
   const bool transport = a.transport != 0;
-  const bool listed = a.variant == kListed;
-  const R c = a.c, hc = a.hc, dts = a.dtsurdx;
-  int ch = -1;
-  int noD[3] = {0, 0, 0};  // nei_oct entry of the face that leaves the oct, per direction
-  if (valid) {
-    ch = gld(a.child, cell);
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    c.noD[d] = 0;
+    c.pairD[d] = -1;
+    c.hball[d] = 0ull;
+    c.hbase[d] = 0;
+  }
+  if (c.valid) {
+    c.ch = gld(a.child, c.cell);
     if (transport) {
 #pragma unroll
-      for (int d = 0; d < 3; d++) noD[d] = gld(a.nei, oct * 6 + 2 * d + ((ic >> d) & 1));
+      for (int d = 0; d < 3; d++) c.noD[d] = gld(a.nei, oct * 6 + 2 * d + ((ic >> d) & 1));
     }
   }
-  const bool restricted = ch >= 0 && !a.update_split;  // takes its children's mean, no transport
-  const bool moves = valid && transport && !restricted;
-  auto in_tile = [&](int no) { return no >= oct0 && no < oct0 + kTileOcts; };
-  int hbase[3] = {0, 0, 0}, nhalo = 0;
-  unsigned long long hball[3] = {0ull, 0ull, 0ull};
-  if (transport) {
-    lds.cancel[lc] = (unsigned char)(ch >= 0 && !a.keep_split_flux);
-    if (listed) {
+  c.restricted = c.ch >= 0 && !a.update_split;  // takes its children's mean, no transport
+  c.moves = c.valid && transport && !c.restricted;
+  hl.on = false;
+  if (!transport) return c;
+  lds.cancel[lc] = (unsigned char)(c.ch >= 0 && !a.keep_split_flux);
+  if (a.ncoarse > 0) {
 #pragma unroll
-      for (int d = 0; d < 3; d++) {
-        const bool out = moves && !in_tile(noD[d]);
-        hball[d] = __ballot(out);
-        hbase[d] = nhalo;
-        nhalo += __popcll(hball[d]);
-        if (out) {
-          const int slot = hbase[d] + lanes_below_mask(hball[d]);  // < kHaloCap (variant chosen from the topology)
-          lds.item[wv][slot] = (unsigned char)(lane * 4 + d);
-          lds.item_nei[wv][slot] = noD[d];
-        }
-      }
-      // the list is written and read by lanes of the same wave
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
+    for (int d = 0; d < 3; d++)
+      if (c.moves && c.noD[d] < 0 && c.noD[d] > kNeiReflective)
+        c.pairD[d] = gld(a.rpair, oct * 6 + 2 * d + ((ic >> d) & 1));
   }
-  // the halo face in direction d of cell hcell, nei_oct entry no: where its
-  // neighbour's state lies
-  struct Halo {
-    int j, d;
-    bool on, coarse, refl;
-  };
-  auto halo_of = [&](bool on, int hcell, int d, int no) {
-    Halo h;
-    const int hic = hcell & 7, side = (hic >> d) & 1;
-    const bool bound = on && no <= kNeiReflective;  // domain face (rad_utils.c:1106-1213, 1376-1407)
-    h.on = on;
-    h.d = d;
-    h.coarse = on && no < 0 && !bound;
-    h.refl = bound && no == kNeiReflective;
-    h.j = !on ? 0
-              : bound ? (hcell & ~7) + trans_source(2 * d + side, hic)
-                      : h.coarse ? -1 - no : no * 8 + (hic ^ (1 << d));
-    return h;
-  };
-  // its cancel flag (the flux from a split neighbour is dropped, RADSTEP)
-  auto halo_cancel = [&](const Halo& h) {
-    return h.on && !h.coarse && !a.keep_split_flux && gld(a.child, h.j) >= 0;
-  };
-  // group g of its state into LDS slot i, with its closure
-  auto halo_put = [&](const Halo& h, int g, int i) {
-    if (!h.on) return;
-    const size_t o = (size_t)g * (size_t)(h.coarse ? a.ncoarse : n) + (size_t)h.j;
-    const R ve = (h.coarse ? a.ce : a.e)[o];
-    R vx = (h.coarse ? a.cfx : a.fx)[o], vy = (h.coarse ? a.cfy : a.fy)[o], vz = (h.coarse ? a.cfz : a.fz)[o];
-    if (h.refl) {
-      if (h.d == 0) vx = -vx;
-      if (h.d == 1) vy = -vy;
-      if (h.d == 2) vz = -vz;
+  if (c.listed) {
+    int nhalo = 0;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      const bool out = c.moves && !in_tile32(c.noD[d], tile);
+      c.hball[d] = __ballot(out);
+      c.hbase[d] = nhalo;
+      nhalo += __popcll(c.hball[d]);
+      if (out) {
+        const int slot = c.hbase[d] + lanes_below_mask(c.hball[d]);  // < kHaloCap (variant chosen from the topology)
+        lds.item[wv][slot] = (unsigned char)(lane * 4 + d);
+        lds.item_nei[wv][slot] = c.noD[d];
+      }
     }
-    lds.put(i, ve, vx, vy, vz, closure_of<R, Fast>(vx, vy, vz, ve, c));
-  };
-  const int hslot0 = kTileCells + wv * CellLds<R>::kHaloCap;
-  Halo hl;  // listed: this lane's entry of the wave's list
-  if (transport && listed) {
+    // the list is written and read by lanes of the same wave
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const int it = lds.item[wv][lane];
-    hl = halo_of(lane < nhalo, (cell & ~63) + (it >> 2), it & 3, lds.item_nei[wv][lane]);
-    lds.cancel[hslot0 + lane] = (unsigned char)halo_cancel(hl);
-  }
-  R Te[G], Tx[G], Ty[G], Tz[G];  // the transported state
+    hl = halo_cell(lane < nhalo, (c.cell & ~63) + (it >> 2), it & 3, lds.item_nei[wv][lane]);
+    lds.cancel[kTileCells + lc] = (unsigned char)halo_cancel(a, hl);
+  } else {
+    // each lane's own slot serves one direction after the other: their flags
+    // as bits of one byte
+    unsigned flags = 0;
 #pragma unroll
-  for (int g = 0; g < G; g++) {
-    if (valid) {
-      Te[g] = gld(a.e + (size_t)g * n, cell);
-      Tx[g] = gld(a.fx + (size_t)g * n, cell);
-      Ty[g] = gld(a.fy + (size_t)g * n, cell);
-      Tz[g] = gld(a.fz + (size_t)g * n, cell);
-    }
+    for (int d = 0; d < 3; d++)
+      if (c.moves && !in_tile32(c.noD[d], tile))
+        flags |= halo_cancel(a, halo_cell(true, c.cell, d, c.noD[d])) ? 1u << d : 0u;
+    lds.cancel[kTileCells + lc] = (unsigned char)flags;
   }
-  if (transport) {
+  return c;
+}
+
+// Transport of group g of the thread's cell: its updated state in T, the
+// refluxes of the finer octs folded in.  GA: groups of a reflux accumulator.
+// All threads of the work-group; the LDS is free again after a barrier.
+template <typename R, int GA, bool Fast>
+__device__ __forceinline__ void transport_group(const LevelArgs<R>& a, const CellFaces& cf, const HaloCell& hl, int tile,
+                                                int lc, CellLds<R>& lds, int g, R T[4]) {
+  const int ic = cf.cell & 7, hslot0 = kTileCells + (lc & ~63), lane = lc & 63;
+  const R c = a.c, hc = a.hc, dts = a.dtsurdx;
+  if (cf.valid) {
+    T[0] = gld(a.e + (size_t)g * a.ncell, cf.cell);
+    T[1] = gld(a.fx + (size_t)g * a.ncell, cf.cell);
+    T[2] = gld(a.fy + (size_t)g * a.ncell, cf.cell);
+    T[3] = gld(a.fz + (size_t)g * a.ncell, cf.cell);
+  }
+  const bool fold = cf.valid && !cf.restricted && cf.ch <= -2;
+  if (!a.transport) {
+    if (fold) fold_reflux<R, GA, 1, kRefluxCell>(a, cf.ch, g, 1, &T[0], &T[1], &T[2], &T[3]);
+    return;
+  }
+  const R ue = T[0], ux = T[1], uy = T[2], uz = T[3];
+  Closure<R> Q;
+  if (cf.valid) {
+    Q = closure_of<R, Fast>(ux, uy, uz, ue, c);
+    lds.put(lc, ue, ux, uy, uz, Q);
+  }
+  if (cf.listed) halo_put<R, Fast>(a, lds, hl, g, hslot0 + lane);
+  __syncthreads();
+  if (!cf.moves) return;
+  R D[4] = {R(0), R(0), R(0), R(0)};
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    // one face in d lies inside the oct and one leaves it; bit says which is
+    // which (bit 1: the minus face is the inside one)
+    const int bit = (ic >> d) & 1, jin = lc ^ (1 << d);
+    const bool inT = in_tile32(cf.noD[d], tile);
+    const int jl = (int)(((unsigned)cf.noD[d] - (unsigned)(tile * kTileOcts)) * 8u + (unsigned)(ic ^ (1 << d)));
+    const int slot = cf.listed ? cf.hbase[d] + lanes_below_mask(cf.hball[d]) : lane;
+    const int jout = inT ? jl : hslot0 + slot;
+    // (own slot: written and read by this lane alone)
+    if (!cf.listed && !inT) halo_put<R, Fast>(a, lds, halo_cell(true, cf.cell, d, cf.noD[d]), g, jout);
+    const bool cin = lds.cancel[jin] != 0;
+    const bool cout = (cf.listed || inT) ? lds.cancel[jout] != 0 : ((lds.cancel[jout] >> d) & 1) != 0;
     // the flux from a neighbour is multiplied by 0 or 1 (rad_utils.c:518-526)
-    R keepm[3], keepp[3];
-    int pairD[3] = {-1, -1, -1};  // reflux pair of a leaving face with a coarse leaf behind it
+    const R keepm = (bit ? cin : cout) ? R(0) : R(1), keepp = (bit ? cout : cin) ? R(0) : R(1);
+    const int jm = bit ? jin : jout, jp = bit ? jout : jin;
+    R Fm[4], Fp[4], ve, vx, vy, vz;
+    Closure<R> qv;
+    lds.get(jm, ve, vx, vy, vz, qv);
+    lf_flux<R>(d, 0, ue, ux, uy, uz, Q, ve, vx, vy, vz, qv, hc, Fm);
+    lds.get(jp, ve, vx, vy, vz, qv);
+    lf_flux<R>(d, 1, ue, ux, uy, uz, Q, ve, vx, vy, vz, qv, hc, Fp);
 #pragma unroll
-    for (int g = 0; g < G; g++) {
-      const R ue = Te[g], ux = Tx[g], uy = Ty[g], uz = Tz[g];
-      Closure<R> Q;
-      if (valid) {
-        Q = closure_of<R, Fast>(ux, uy, uz, ue, c);
-        lds.put(lc, ue, ux, uy, uz, Q);
-      }
-      if (listed) halo_put(hl, g, hslot0 + lane);
-      __syncthreads();
-      if (moves) {
-        R De = R(0), Dx = R(0), Dy = R(0), Dz = R(0);
+    for (int v = 0; v < 4; v++) {
+      Fm[v] *= keepm;
+      Fp[v] *= keepp;
+      // the minus face first, as the six faces are numbered
+      D[v] += Fm[v] * dts;
+      D[v] -= Fp[v] * dts;
+    }
+    if (cf.pairD[d] >= 0) {
+      // the cell's place in the oct face: its two coordinates across d
+      const int q = ((ic >> ((d + 1) % 3)) & 1) | (((ic >> ((d + 2) % 3)) & 1) << 1);
+      R F[4];
 #pragma unroll
-        for (int d = 0; d < 3; d++) {
-          // one face in d lies inside the oct and one leaves it; bit says
-          // which is which (bit 1: the minus face is the inside one)
-          const int bit = (ic >> d) & 1, jin = lc ^ (1 << d);
-          const bool inT = in_tile(noD[d]);
-          const int jl = (int)(((unsigned)noD[d] - (unsigned)oct0) * 8u + (unsigned)(ic ^ (1 << d)));
-          const int slot = listed ? hbase[d] + lanes_below_mask(hball[d]) : lane;
-          const int jout = inT ? jl : hslot0 + slot;
-          if (!listed && !inT) {  // this lane's own slot: written and read by it alone
-            const Halo h = halo_of(true, cell, d, noD[d]);
-            if (g == 0) lds.cancel[jout] = (unsigned char)halo_cancel(h);
-            halo_put(h, g, jout);
-          }
-          if (g == 0) {
-            const bool cin = lds.cancel[jin] != 0, cout = lds.cancel[jout] != 0;
-            keepm[d] = (bit ? cin : cout) ? R(0) : R(1);
-            keepp[d] = (bit ? cout : cin) ? R(0) : R(1);
-            if (!inT && noD[d] < 0 && noD[d] > kNeiReflective) pairD[d] = gld(a.rpair, oct * 6 + 2 * d + bit);
-          }
-          const int jm = bit ? jin : jout, jp = bit ? jout : jin;
-          R Fm[4], Fp[4], ve, vx, vy, vz;
-          Closure<R> qv;
-          lds.get(jm, ve, vx, vy, vz, qv);
-          lf_flux<R>(d, 0, ue, ux, uy, uz, Q, ve, vx, vy, vz, qv, hc, Fm);
-          lds.get(jp, ve, vx, vy, vz, qv);
-          lf_flux<R>(d, 1, ue, ux, uy, uz, Q, ve, vx, vy, vz, qv, hc, Fp);
-#pragma unroll
-          for (int v = 0; v < 4; v++) {
-            Fm[v] *= keepm[d];
-            Fp[v] *= keepp[d];
-          }
-          // the minus face first, as the six faces are numbered
-          De += Fm[0] * dts;
-          Dx += Fm[1] * dts;
-          Dy += Fm[2] * dts;
-          Dz += Fm[3] * dts;
-          De -= Fp[0] * dts;
-          Dx -= Fp[1] * dts;
-          Dy -= Fp[2] * dts;
-          Dz -= Fp[3] * dts;
-          if (pairD[d] >= 0) {
-            // the cell's place in the oct face: its two coordinates across d
-            const int q = ((ic >> ((d + 1) % 3)) & 1) | (((ic >> ((d + 2) % 3)) & 1) << 1);
-            R F[4];
-#pragma unroll
-            for (int v = 0; v < 4; v++) F[v] = bit ? Fp[v] : Fm[v];
-            reflux<R, GA>(a, pairD[d], q, 2 * d + bit, g, F, dts);
-          }
-        }
-        if (ch <= -2) fold_reflux<R, GA, 1, kRefluxCell>(a, ch, g, 1, &Te[g], &Tx[g], &Ty[g], &Tz[g]);
-        Te[g] += De;
-        Tx[g] += Dx;
-        Ty[g] += Dy;
-        Tz[g] += Dz;
-      }
-      if (g + 1 < G) __syncthreads();  // the next group overwrites the tile's state
+      for (int v = 0; v < 4; v++) F[v] = bit ? Fp[v] : Fm[v];
+      reflux<R, GA>(a, cf.pairD[d], q, 2 * d + bit, g, F, dts);
     }
   }
-  unsigned int nit_acc = 0, leaf = 0;
-  if (valid) {
-    if (a.t_first != nullptr) xion_times(a, cell);
-    if (restricted) {
-      restrict_cell(a, cell, ch, G);
-    } else if (ch >= 0) {
-      transport_split_cell<R, G>(a, cell, G, Te, Tx, Ty, Tz);
-    } else {
-      if (!transport && ch <= -2) {
+  if (fold) fold_reflux<R, GA, 1, kRefluxCell>(a, cf.ch, g, 1, &T[0], &T[1], &T[2], &T[3]);
 #pragma unroll
-        for (int g = 0; g < G; g++)
-          fold_reflux<R, GA, 1, kRefluxCell>(a, ch, g, 1, &Te[g], &Tx[g], &Ty[g], &Tz[g]);
-      }
+  for (int v = 0; v < 4; v++) T[v] += D[v];
+}
+
+// One group, FP64: transport and chemistry in one kernel, four waves per SIMD
+// (64^3 cells 22.2 us with the allocation left free, 20.1 so).
+__global__ __launch_bounds__(kTileCells) __attribute__((amdgpu_waves_per_eu(4))) void level_step_kernel(
+    LevelArgs<double> a_by_value, ChemConst K_by_value) {
+  const KernArgs<double> args = kernargs<double>();
+  const LevelArgs<double>& a = args.a;
+  CellLds<double>& lds = *cell_lds<double>();
+  const int tile = xcd_block(a.nblocks), lc = (int)threadIdx.x;
+  HaloCell hl;
+  const CellFaces cf = cell_faces(a, tile, lc, lds, hl);
+  double T[4];
+  transport_group<double, 1, false>(a, cf, hl, tile, lc, lds, 0, T);
+  unsigned int nit_acc = 0, leaf = 0;
+  if (cf.valid) {
+    if (a.t_first != nullptr) xion_times(a, cf.cell);
+    if (cf.restricted) {
+      restrict_cell(a, cf.cell, cf.ch, 1);
+    } else if (cf.ch >= 0) {
+      transport_split_cell<double, 1>(a, cf.cell, 1, &T[0], &T[1], &T[2], &T[3]);
+    } else {
       leaf = 1;
-      nit_acc = (unsigned)finish_leaf<R, G, Fast, kRefluxCell>(a, K, cell, G, Te, Tx, Ty, Tz);
+      nit_acc = (unsigned)finish_leaf<double, 1, false, kRefluxCell>(a, args.K, cf.cell, 1, &T[0], &T[1], &T[2], &T[3]);
     }
   }
   if (a.counters != nullptr) block_counters<kTileWaves>(a.counters, nit_acc, leaf);
 }
 
-// Waves per SIMD the register allocation aims at: FP64 with one group fits
-// four (64^3 cells 22.2 -> 20.1 us), with two or three groups three (64^3
-// cells 69 -> 64 us); more groups would spill.
-constexpr int cell_step_waves(size_t rb, int g) { return rb != 8 ? 1 : g == 1 ? 4 : g <= 3 ? 3 : 1; }
+// More groups: the transport as a kernel of its own, one group a work-group
+// (gridDim.y of them side by side), which leaves the transported state in the
+// next state's arrays, and the chemistry after it.  In one kernel the chemistry's
+// registers (168 to 256) held the transport to one to three waves per SIMD, and
+// a small level waited for all groups' transport in one wave's chain; apart, the
+// transport takes 125 (FP32 76).  A level step of 32^3 cells, nine FP64 groups:
+// 41 -> 27 us, though the transported state is written and read once more;
+// 64^3 cells, nine FP32 groups 55.4 -> 52.2 us, three FP64 groups 64 -> 62 us,
+// of 4,600 and 20,000 cells below it 27 -> 22.8 and 42 -> 41 us.
+template <typename R, int GA, bool Fast>
+__global__ __launch_bounds__(kTileCells) void transport_kernel(LevelArgs<R> a_by_value, ChemConst K_by_value) {
+  const LevelArgs<R>& a = kernargs<R>().a;
+  CellLds<R>& lds = *cell_lds<R>();
+  const int tile = xcd_block(a.nblocks), lc = (int)threadIdx.x;
+  HaloCell hl;
+  const CellFaces cf = cell_faces(a, tile, lc, lds, hl);
+  for (int g = (int)blockIdx.y; g < a.ng; g += (int)gridDim.y) {
+    R T[4];
+    transport_group<R, GA, Fast>(a, cf, hl, tile, lc, lds, g, T);
+    if (cf.valid && !cf.restricted) {
+      const size_t o = (size_t)g * a.ncell;
+      gst(a.eo + o, cf.cell, T[0]);
+      gst(a.fxo + o, cf.cell, T[1]);
+      gst(a.fyo + o, cf.cell, T[2]);
+      gst(a.fzo + o, cf.cell, T[3]);
+      // COARSERAD: a split cell's check (a leaf's is the chemistry's)
+      if (cf.ch >= 0 && ((g == 0 && (T[0] < R(0) || isnan(T[0]))) || (g == 1 && isnan(T[0]))))
+        raise_status(a.status, -3, a.level, cf.cell);
+    }
+    if (g + (int)gridDim.y < a.ng) __syncthreads();  // the next group overwrites the tile's state
+  }
+}
+
+// (191 VGPRs for three FP64 groups, 208 for nine FP32 ones: held to 128 or 168
+// the spills cost more than the waves bring, 62 -> 71 and 52 -> 70 us a step)
 template <typename R, int G, bool Fast>
-__global__ __launch_bounds__(kTileCells) __attribute__((amdgpu_waves_per_eu(cell_step_waves(sizeof(R), G)))) void
-level_step_kernel(LevelArgs<R> a_by_value, ChemConst K_by_value) {
+__global__ __launch_bounds__(kTileCells) void chemistry_kernel(LevelArgs<R> a_by_value, ChemConst K_by_value) {
   const KernArgs<R> args = kernargs<R>();
-  cell_step_lds<R, G, Fast>(args.a, args.K, xcd_block(args.a.nblocks), (int)threadIdx.x, *cell_lds<R>());
+  const LevelArgs<R>& a = args.a;
+  const int cell = xcd_block(a.nblocks) * kTileCells + (int)threadIdx.x;
+  unsigned int nit_acc = 0, leaf = 0;
+  if (cell < a.ncell) {
+    const int ch = gld(a.child, cell);
+    if (a.t_first != nullptr) xion_times(a, cell);
+    if (ch >= 0 && !a.update_split) {
+      restrict_cell(a, cell, ch, G);
+    } else if (ch >= 0) {
+      gst(a.nhpluso, cell, gld(a.nhplus, cell));
+      gst(a.einto, cell, gld(a.eint, cell));
+      gst(a.tempo, cell, gld(a.temp, cell));
+    } else {
+      R Te[G], Tx[G], Ty[G], Tz[G];
+#pragma unroll
+      for (int g = 0; g < G; g++) {
+        const size_t o = (size_t)g * a.ncell;
+        Te[g] = gld(a.eo + o, cell);
+        Tx[g] = gld(a.fxo + o, cell);
+        Ty[g] = gld(a.fyo + o, cell);
+        Tz[g] = gld(a.fzo + o, cell);
+      }
+      leaf = 1;
+      nit_acc = (unsigned)finish_leaf<R, G, Fast, kRefluxCell>(a, args.K, cell, G, Te, Tx, Ty, Tz);
+    }
+  }
+  if (a.counters != nullptr) block_counters<kTileWaves>(a.counters, nit_acc, leaf);
 }
 
 // ------------------------------------------------------------------ tiled level step
@@ -1932,6 +2024,15 @@ __global__ __launch_bounds__(kTileCells) __attribute__((amdgpu_waves_per_eu(Tile
 }
 
 // ------------------------------------------------------------------ launchers
+// Work-groups side by side over the photon groups of a tile: all of them while
+// that is up to eight work-groups per CU (32^3 cells, nine groups: 27 us, with
+// three at a time 29), otherwise three, so that a tile's topology and halo
+// list serve several groups (64^3 cells: 52 us, with nine 57).
+static unsigned transport_groups(int nb, int ng) {
+  constexpr int kFull = 2048;
+  return (unsigned)(nb * ng <= kFull ? ng : std::min(ng, 3));
+}
+
 template <int G>
 static void launch_split(LevelArgs<float> a, const ChemConst& K, hipStream_t s) {
   a.nblocks = ((a.ncell + kSplitCells - 1) / kSplitCells + 7) & ~7;
@@ -1979,27 +2080,38 @@ hipError_t launch_level_step(const LevelArgs<R>& a0, const ChemConst& K, hipStre
   a.nblocks = nb;
   const dim3 grid(nb), block(kTileCells);
   constexpr bool fast = sizeof(R) == 4;
+  if constexpr (!fast) {
+    if (a.ng == 1) {
+      hipLaunchKernelGGL(level_step_kernel, grid, block, 0, s, a, K);
+      return hipGetLastError();
+    }
+  }
+  const dim3 tgrid(nb, transport_groups(nb, a.ng));
+  if (!fast && a.ng == 3)  // (three FP32 groups took the tiled kernel)
+    hipLaunchKernelGGL((transport_kernel<R, 3, fast>), tgrid, block, 0, s, a, K);
+  else
+    hipLaunchKernelGGL((transport_kernel<R, kMaxGrp, fast>), tgrid, block, 0, s, a, K);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
   switch (a.ng) {
-#define EMMA_STEP(g) \
-  case g: hipLaunchKernelGGL((level_step_kernel<R, g, fast>), grid, block, 0, s, a, K); break
-    EMMA_STEP(2);
-    EMMA_STEP(4);
-    EMMA_STEP(5);
-    EMMA_STEP(6);
-    EMMA_STEP(7);
-    EMMA_STEP(8);
-    EMMA_STEP(9);
+#define EMMA_CHEM(g) \
+  case g: hipLaunchKernelGGL((chemistry_kernel<R, g, fast>), grid, block, 0, s, a, K); break
+    EMMA_CHEM(2);
+    EMMA_CHEM(4);
+    EMMA_CHEM(5);
+    EMMA_CHEM(6);
+    EMMA_CHEM(7);
+    EMMA_CHEM(8);
+    EMMA_CHEM(9);
+#undef EMMA_CHEM
     default:
-      if constexpr (fast) {
-        return hipErrorInvalidValue;  // 1 and 3 groups took the tiled kernel
-      } else {
-        switch (a.ng) {
-          EMMA_STEP(1);
-          EMMA_STEP(3);
-          default: return hipErrorInvalidValue;
+      if constexpr (!fast) {
+        if (a.ng == 3) {
+          hipLaunchKernelGGL((chemistry_kernel<R, 3, fast>), grid, block, 0, s, a, K);
+          break;
         }
       }
-#undef EMMA_STEP
+      return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
