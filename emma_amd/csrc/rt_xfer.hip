@@ -28,11 +28,14 @@
 namespace emma {
 namespace {
 
-// 128^3 cells with three groups, both ways: slots of 1 MiB 6.0 / 5.6 ms, of
-// 512 KiB 6.8 / 6.5, of 256 KiB 8.8 / 8.6; of 2 MiB 5.6 / 4.8, but a 64^3
-// level back then 1.5 instead of 1.0 ms (fewer chunks than threads).  Twelve
-// threads gain nothing over eight.
-constexpr size_t kSlotBytes = 1u << 20;
+// 128^3 cells with three groups (193 MB), both ways: chunks of 1 MiB 6.0 /
+// 5.6 ms, of 512 KiB 6.8 / 6.5, of 256 KiB 8.8 / 8.6; of 2 MiB 5.6 / 4.8, but
+// 64^3 cells with nine groups (55 MB) back then 1.7 instead of 1.45 ms and
+// with one FP64 group (19 MB) 1.5 instead of 1.0 (fewer chunks than threads):
+// 2 MiB from 128 MB on.  Twelve threads gain nothing over eight.
+constexpr size_t kSlotBytes = 2u << 20;
+constexpr size_t kPackBytes = 1u << 20;  // up to here one gathering kernel
+constexpr size_t kChunkBytes = 1u << 20, kLargeTotal = 128u << 20;
 constexpr int kMaxThreads = 8;
 constexpr size_t kBytesPerThread = 4u << 20;  // host bytes that pay for starting a thread (0.02 to 2 ms)
 constexpr size_t kKeepSlots = 2 * kMaxThreads;
@@ -252,8 +255,10 @@ int host_threads() {
 template <bool ToHost>
 hipError_t chunked(int device, hipStream_t s, const XferPart* parts, int np, size_t total) {
   std::vector<Chunk> chunks;
+  size_t moved = 0;
+  for (int k = 0; k < np; k++) moved += parts[k].n * (parts[k].f32 ? sizeof(float) : sizeof(double));
   for (int k = 0; k < np; k++) {
-    const size_t per = kSlotBytes / (parts[k].f32 ? sizeof(float) : sizeof(double));
+    const size_t per = (moved >= kLargeTotal ? kSlotBytes : kChunkBytes) / (parts[k].f32 ? sizeof(float) : sizeof(double));
     for (size_t i = 0; i < parts[k].n; i += per) chunks.push_back({&parts[k], i, std::min(per, parts[k].n - i)});
   }
   Job job;
@@ -285,7 +290,7 @@ hipError_t transfer(int device, hipStream_t s, const XferPart* in, int nin) {
     total += in[k].n;
   }
   if (np == 0) return hipStreamSynchronize(s);
-  if (total * sizeof(double) <= kSlotBytes) return packed<ToHost>(s, parts, np, total);
+  if (total * sizeof(double) <= kPackBytes) return packed<ToHost>(s, parts, np, total);
   try {
     return chunked<ToHost>(device, s, parts, np, total);
   } catch (...) {
