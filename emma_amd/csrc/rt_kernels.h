@@ -26,6 +26,10 @@ struct LevelArgs {
   // Morton order, and the tiled kernel walks each XCD's octant of tiles in
   // raster order (z fastest) instead of Morton order (see raster_tile)
   int raster_m;
+  // the launch steps these tiles only (null: every tile of the level)
+  const int* tiles;
+  int ntiles;
+  int leave_room;  // the launch runs beside small levels' launches
   int cnslot;  // accumulators in cracc
   // chemistry stragglers (tiled mixed kernel): a leaf whose sub-step loop is
   // still running after chem_budget tries (> 0; <= 0: no limit) stores its

@@ -29,6 +29,15 @@ __device__ __forceinline__ int xcd_block(int nb) {
   return (b & 7) * per + (b >> 3);
 }
 
+// The tile of a block: of all tiles of the level, or of the launch's list (-1:
+// no tile; the whole block)
+template <typename R>
+__device__ __forceinline__ int block_tile(const LevelArgs<R>& a) {
+  const int i = xcd_block(a.nblocks);
+  if (a.tiles == nullptr) return i;
+  return i < a.ntiles ? a.tiles[i] : -1;
+}
+
 // The tile a block takes on a complete Morton-ordered cube of n = 2^m octs a
 // side.  A tile is 32 Morton-consecutive octs, a 4 x 4 x 2 brick, so the
 // tile index interleaves the tile coordinates (z, x, y from the lowest bit:
@@ -835,7 +844,8 @@ __global__ __launch_bounds__(kTileCells) __attribute__((amdgpu_waves_per_eu(4)))
   const KernArgs<double> args = kernargs<double>();
   const LevelArgs<double>& a = args.a;
   CellLds<double>& lds = *cell_lds<double>();
-  const int tile = xcd_block(a.nblocks), lc = (int)threadIdx.x;
+  const int tile = block_tile(a), lc = (int)threadIdx.x;
+  if (tile < 0) return;
   HaloCell hl;
   const CellFaces cf = cell_faces(a, tile, lc, lds, hl);
   double T[4];
@@ -868,7 +878,8 @@ template <typename R, int GA, bool Fast>
 __global__ __launch_bounds__(kTileCells) void transport_kernel(LevelArgs<R> a_by_value, ChemConst K_by_value) {
   const LevelArgs<R>& a = kernargs<R>().a;
   CellLds<R>& lds = *cell_lds<R>();
-  const int tile = xcd_block(a.nblocks), lc = (int)threadIdx.x;
+  const int tile = block_tile(a), lc = (int)threadIdx.x;
+  if (tile < 0) return;
   HaloCell hl;
   const CellFaces cf = cell_faces(a, tile, lc, lds, hl);
   for (int g = (int)blockIdx.y; g < a.ng; g += (int)gridDim.y) {
@@ -894,7 +905,9 @@ template <typename R, int G, bool Fast>
 __global__ __launch_bounds__(kTileCells) void chemistry_kernel(LevelArgs<R> a_by_value, ChemConst K_by_value) {
   const KernArgs<R> args = kernargs<R>();
   const LevelArgs<R>& a = args.a;
-  const int cell = xcd_block(a.nblocks) * kTileCells + (int)threadIdx.x;
+  const int tile = block_tile(a);
+  if (tile < 0) return;
+  const int cell = tile * kTileCells + (int)threadIdx.x;
   unsigned int nit_acc = 0, leaf = 0;
   if (cell < a.ncell) {
     const int ch = gld(a.child, cell);
@@ -1360,7 +1373,8 @@ __global__ __launch_bounds__(kTileCells) __attribute__((amdgpu_waves_per_eu(4)))
   const KernArgs<float> args = kernargs<float>();
   __shared__ TileLds<G> lds;
   const int m = args.a.raster_m;
-  const int tile = m > 0 ? raster_tile(m) : xcd_block(args.a.nblocks);
+  const int tile = m > 0 ? raster_tile(m) : block_tile(args.a);
+  if (tile < 0) return;
   if constexpr (PerDir)
     tiled_step<G, kPerDir>(args.a, args.K, tile, lds, (int)threadIdx.x);
   else if (args.a.ncoarse == 0)  // wave-uniform: the level's arguments
@@ -1419,6 +1433,8 @@ __global__ __launch_bounds__(64 * G) void level_step_split(LevelArgs<float> a_by
   const LevelArgs<float>& a = args.a;
   const ChemConst& K = args.K;
   __shared__ SplitLds<G> lds;
+  // ahead of a large level's waves that step beside it (emma_rt_coarse_step)
+  __builtin_amdgcn_s_setprio(3);
   const int g = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
   const int tile = xcd_block(a.nblocks);
   const int n = a.ncell;
@@ -2033,6 +2049,8 @@ static unsigned transport_groups(int nb, int ng) {
   return (unsigned)(nb * ng <= kFull ? ng : std::min(ng, 3));
 }
 
+constexpr unsigned kCuLds = 160 * 1024;
+static_assert(sizeof(TileLds<3>) < kCuLds / 4, "four work-groups a CU");
 template <int G>
 static void launch_split(LevelArgs<float> a, const ChemConst& K, hipStream_t s) {
   a.nblocks = ((a.ncell + kSplitCells - 1) / kSplitCells + 7) & ~7;
@@ -2044,7 +2062,7 @@ hipError_t launch_level_step(const LevelArgs<R>& a0, const ChemConst& K, hipStre
   LevelArgs<R> a = a0;
   if constexpr (sizeof(R) == 4) {
     if (a.ng == 1 || a.ng == 3) {
-      int nb = (a.ncell + kTileCells - 1) / kTileCells;
+      int nb = a.tiles ? a.ntiles : (a.ncell + kTileCells - 1) / kTileCells;
       nb = (nb + 7) & ~7;
       a.nblocks = nb;
       // sparse levels: per-direction halo faces
@@ -2053,6 +2071,9 @@ hipError_t launch_level_step(const LevelArgs<R>& a0, const ChemConst& K, hipStre
       if (defer && (a.defer_list == nullptr || a.defer_ctl == nullptr || a.defer_cap < a.ncell))
         return hipErrorInvalidValue;
       // the list holds at most the level's cells
+      // beside smaller levels' launches: LDS beyond a quarter of a CU's, so that
+      // three work-groups instead of four share it and the small ones start at once
+      const unsigned share = a.leave_room ? kCuLds / 4 + 256 - (unsigned)sizeof(TileLds<3>) : 0u;
       const dim3 sg(std::min(kStragglerBlocks, (a.ncell + kStragglerThreads - 1) / kStragglerThreads)),
           sb(kStragglerThreads);
       if (a.ng == 1) {
@@ -2067,15 +2088,15 @@ hipError_t launch_level_step(const LevelArgs<R>& a0, const ChemConst& K, hipStre
         if (v == kLatency)
           launch_split<3>(a, K, s);
         else if (v == kPerDir)
-          hipLaunchKernelGGL((level_step_tiled<3, true>), dim3(nb), dim3(kTileCells), 0, s, a, K);
+          hipLaunchKernelGGL((level_step_tiled<3, true>), dim3(nb), dim3(kTileCells), share, s, a, K);
         else
-          hipLaunchKernelGGL((level_step_tiled<3, false>), dim3(nb), dim3(kTileCells), 0, s, a, K);
+          hipLaunchKernelGGL((level_step_tiled<3, false>), dim3(nb), dim3(kTileCells), share, s, a, K);
         if (defer) hipLaunchKernelGGL((chem_straggler_kernel<3>), sg, sb, 0, s, a, K);
       }
       return hipGetLastError();
     }
   }
-  int nb = (a.ncell + 255) / 256;
+  int nb = a.tiles ? a.ntiles : (a.ncell + kTileCells - 1) / kTileCells;
   nb = (nb + 7) & ~7;
   a.nblocks = nb;
   const dim3 grid(nb), block(kTileCells);
