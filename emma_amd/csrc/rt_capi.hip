@@ -78,6 +78,8 @@ struct DevLevel {
   int* tiles = nullptr;
   int nfree = 0, ntile = 0;
   int fork = 0;  // 1: the free tiles may step beside the finer levels, 2: leaving room for their work-groups
+  int* defer = nullptr;  // fork: the level's own straggler list (its free tiles append beside other levels' lists)
+  int fork_slot = 0;     // and the list-length word its two launches share
   hipStream_t side = nullptr;  // where the free tiles' step runs beside the finer levels'
   hipEvent_t forked = nullptr, joined = nullptr;
   std::vector<int> hchild;  // host copy with the reflux pairs encoded
@@ -232,6 +234,7 @@ static void free_tree(emma_rt_ctx* c) {
     (void)hipFree(L.racc);
     (void)hipFree(L.rpair);
     (void)hipFree(L.tiles);
+    (void)hipFree(L.defer);
     if (L.forked) (void)hipEventDestroy(L.forked);
     if (L.joined) (void)hipEventDestroy(L.joined);
     if (L.side) (void)hipStreamDestroy(L.side);
@@ -694,6 +697,8 @@ extern "C" int emma_rt_tree_create(emma_rt_ctx* c, int lmin, int lmax, const int
     for (auto& L : c->lev) cap = std::max(cap, L.ncell);
     HIPCHK(dalloc(&c->d_defer, (size_t)cap));
     c->defer_cap = cap;
+    for (auto& L : c->lev)
+      if (L.fork) HIPCHK(dalloc(&L.defer, (size_t)L.ncell));
   }
   c->has_tree = true;
   if (c->xion) {
@@ -826,12 +831,15 @@ static LevelArgs<R> level_args(emma_rt_ctx* c, int k, double dtnew, double aexp,
     A.ntiles = part == kFreeTiles ? L.nfree : L.ntile - L.nfree;
     A.leave_room = part == kFreeTiles && L.fork == 2;
   }
-  if (c->d_defer != nullptr && L.chem_budget > 0 && c->defer_seq < c->defer_slots) {
+  const bool shares = part == kTouchedTiles;  // the list of the free tiles' launch
+  if (c->d_defer != nullptr && L.chem_budget > 0 && (shares || c->defer_seq < c->defer_slots)) {
     A.chem_budget = L.chem_budget;
     A.chem_keep = L.chem_keep;
-    A.defer_cap = c->defer_cap;
-    A.defer_list = c->d_defer;
-    A.defer_ctl = c->d_defer_ctl + c->defer_seq++;
+    A.defer_cap = L.defer ? L.ncell : c->defer_cap;
+    A.defer_list = L.defer ? L.defer : c->d_defer;
+    const int slot = shares ? L.fork_slot : c->defer_seq++;
+    if (part == kFreeTiles) L.fork_slot = slot;
+    A.defer_ctl = c->d_defer_ctl + slot;
   }
   A.e = (const R*)L.e[a];
   A.fx = (const R*)L.fx[a];
@@ -894,20 +902,15 @@ static LevelArgs<R> level_args(emma_rt_ctx* c, int k, double dtnew, double aexp,
   return A;
 }
 
-static hipError_t launch_level(emma_rt_ctx* c, int k, double dtnew, double aexp, int chemonly, bool counters,
-                               int part, hipStream_t s) {
-  DevLevel& L = c->lev[k];
-  const ChemConst K = make_chem(c->p, dtnew, aexp);
-  hipError_t e = hipSuccess;
-  if (part == kTouchedTiles && L.ntile == L.nfree) {
-    // every tile was free
-  } else if (c->rbytes == 8) {
-    e = launch_level_step<double>(level_args<double>(c, k, dtnew, aexp, chemonly, counters, part), K, s);
-  } else {
-    e = launch_level_step<float>(level_args<float>(c, k, dtnew, aexp, chemonly, counters, part), K, s);
-  }
-  if (part != kFreeTiles) L.cur = 1 - L.cur;
-  return e;
+template <typename R>
+static hipError_t launch_part(emma_rt_ctx* c, int k, double dtnew, double aexp, int chemonly, int part, hipStream_t s) {
+  return launch_level_step<R>(level_args<R>(c, k, dtnew, aexp, chemonly, c->counters != 0, part),
+                              make_chem(c->p, dtnew, aexp), part == kAllTiles, s);
+}
+
+static hipError_t launch_level(emma_rt_ctx* c, int k, double dtnew, double aexp, int chemonly, int part, hipStream_t s) {
+  return c->rbytes == 8 ? launch_part<double>(c, k, dtnew, aexp, chemonly, part, s)
+                        : launch_part<float>(c, k, dtnew, aexp, chemonly, part, s);
 }
 
 // A level's step beside the finer levels' steps before it.  In the RADSTEP
@@ -918,30 +921,34 @@ static hipError_t launch_level(emma_rt_ctx* c, int k, double dtnew, double aexp,
 // captured, the free tiles' launch goes on a side stream before the finer
 // levels' launches (fork_free) and is joined after the touched tiles' launch
 // (join_free): the small levels' launches, each a few work-groups' latency,
-// run beside it.  Not with FillRad's block or the hydro injection (they touch
-// all cells), a chemistry budget (one straggler list per launch), or the
-// raster order.  Results are the same bit for bit.  The five-level tree's coarse
+// run beside it.  With a chemistry budget both launches append to one straggler
+// list, whose pass follows the join.  Not with FillRad's block or the hydro
+// injection (they touch all cells), or the raster order.  Results are the same bit for bit.  The five-level tree's coarse
 // step (24 of 31 launches of at most 190 tiles): 0.575 -> 0.541 ms, its first
 // one, with long chemistry chains in the large levels, 1.07 -> 0.91 ms.
 static bool can_fork(emma_rt_ctx* c, int k) {
   const DevLevel& L = c->lev[k];
   return c->capturing && !c->rec && L.tiles != nullptr && c->mode == EMMA_RT_RADSTEP && !c->hydro && !c->star &&
-         !c->stars && !(c->d_defer != nullptr && L.chem_budget > 0) && !(L.raster && L.morton_m > 0) &&
-         L.variant != kLatency && L.side != nullptr;
+         !c->stars && !(L.raster && L.morton_m > 0) && L.variant != kLatency && L.side != nullptr;
 }
 
 static int fork_free(emma_rt_ctx* c, int k, double dt, double aexp) {
   DevLevel& L = c->lev[k];
   HIPCHK(hipEventRecord(L.forked, c->stream));
   HIPCHK(hipStreamWaitEvent(L.side, L.forked, 0));
-  HIPCHK(launch_level(c, k, dt, aexp, 0, c->counters != 0, kFreeTiles, L.side));
+  HIPCHK(launch_level(c, k, dt, aexp, 0, kFreeTiles, L.side));
   HIPCHK(hipEventRecord(L.joined, L.side));
   return EMMA_RT_OK;
 }
 
 static int join_free(emma_rt_ctx* c, int k, double dt, double aexp) {
-  HIPCHK(launch_level(c, k, dt, aexp, 0, c->counters != 0, kTouchedTiles, c->stream));
-  HIPCHK(hipStreamWaitEvent(c->stream, c->lev[k].joined, 0));
+  DevLevel& L = c->lev[k];
+  if (L.ntile > L.nfree) HIPCHK(launch_level(c, k, dt, aexp, 0, kTouchedTiles, c->stream));
+  HIPCHK(hipStreamWaitEvent(c->stream, L.joined, 0));
+  if (c->d_defer != nullptr && L.chem_budget > 0)
+    HIPCHK(launch_stragglers(level_args<float>(c, k, dt, aexp, 0, c->counters != 0, kTouchedTiles),
+                             make_chem(c->p, dt, aexp), c->stream));
+  L.cur = 1 - L.cur;
   c->stats.level_steps++;
   return EMMA_RT_OK;
 }
@@ -1012,7 +1019,8 @@ static int timed_launch(emma_rt_ctx* c, int k, double dtnew, double aexp, int ch
     c->ev_level.push_back(k);
     HIPCHK(hipEventRecord(e0, c->stream));
   }
-  HIPCHK(launch_level(c, k, dtnew, aexp, chemonly, c->counters != 0, kAllTiles, c->stream));
+  HIPCHK(launch_level(c, k, dtnew, aexp, chemonly, kAllTiles, c->stream));
+  c->lev[k].cur = 1 - c->lev[k].cur;
   if (c->timing) HIPCHK(hipEventRecord(e1, c->stream));
   c->stats.level_steps++;
   return EMMA_RT_OK;

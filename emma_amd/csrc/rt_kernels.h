@@ -159,8 +159,11 @@ inline long long max_level_cells(int ng) {
   return by_index < (1LL << 29) ? by_index : (1LL << 29);
 }
 
+// stragglers: the straggler pass follows (a chemistry budget set)
 template <typename R>
-hipError_t launch_level_step(const LevelArgs<R>& a, const ChemConst& K, hipStream_t s);
+hipError_t launch_level_step(const LevelArgs<R>& a, const ChemConst& K, bool stragglers, hipStream_t s);
+// the straggler pass by itself
+hipError_t launch_stragglers(const LevelArgs<float>& a, const ChemConst& K, hipStream_t s);
 
 // Levels of a tree for the COARSERAD transfers between the coarse level and
 // the leaves (putE2coarse / distribE): per level (index level - lcoarse) the

@@ -2057,8 +2057,18 @@ static void launch_split(LevelArgs<float> a, const ChemConst& K, hipStream_t s) 
   hipLaunchKernelGGL((level_step_split<G>), dim3(a.nblocks), dim3(64 * G), 0, s, a, K);
 }
 
+hipError_t launch_stragglers(const LevelArgs<float>& a, const ChemConst& K, hipStream_t s) {
+  // the list holds at most the level's cells
+  const dim3 grid(std::min(kStragglerBlocks, (a.ncell + kStragglerThreads - 1) / kStragglerThreads));
+  if (a.ng == 1)
+    hipLaunchKernelGGL((chem_straggler_kernel<1>), grid, dim3(kStragglerThreads), 0, s, a, K);
+  else
+    hipLaunchKernelGGL((chem_straggler_kernel<3>), grid, dim3(kStragglerThreads), 0, s, a, K);
+  return hipGetLastError();
+}
+
 template <typename R>
-hipError_t launch_level_step(const LevelArgs<R>& a0, const ChemConst& K, hipStream_t s) {
+hipError_t launch_level_step(const LevelArgs<R>& a0, const ChemConst& K, bool stragglers, hipStream_t s) {
   LevelArgs<R> a = a0;
   if constexpr (sizeof(R) == 4) {
     if (a.ng == 1 || a.ng == 3) {
@@ -2070,12 +2080,9 @@ hipError_t launch_level_step(const LevelArgs<R>& a0, const ChemConst& K, hipStre
       const bool defer = a.chem_budget > 0;
       if (defer && (a.defer_list == nullptr || a.defer_ctl == nullptr || a.defer_cap < a.ncell))
         return hipErrorInvalidValue;
-      // the list holds at most the level's cells
       // beside smaller levels' launches: LDS beyond a quarter of a CU's, so that
       // three work-groups instead of four share it and the small ones start at once
       const unsigned share = a.leave_room ? kCuLds / 4 + 256 - (unsigned)sizeof(TileLds<3>) : 0u;
-      const dim3 sg(std::min(kStragglerBlocks, (a.ncell + kStragglerThreads - 1) / kStragglerThreads)),
-          sb(kStragglerThreads);
       if (a.ng == 1) {
         if (v == kLatency)
           launch_split<1>(a, K, s);
@@ -2083,7 +2090,6 @@ hipError_t launch_level_step(const LevelArgs<R>& a0, const ChemConst& K, hipStre
           hipLaunchKernelGGL((level_step_tiled<1, true>), dim3(nb), dim3(kTileCells), 0, s, a, K);
         else
           hipLaunchKernelGGL((level_step_tiled<1, false>), dim3(nb), dim3(kTileCells), 0, s, a, K);
-        if (defer) hipLaunchKernelGGL((chem_straggler_kernel<1>), sg, sb, 0, s, a, K);
       } else {
         if (v == kLatency)
           launch_split<3>(a, K, s);
@@ -2091,9 +2097,9 @@ hipError_t launch_level_step(const LevelArgs<R>& a0, const ChemConst& K, hipStre
           hipLaunchKernelGGL((level_step_tiled<3, true>), dim3(nb), dim3(kTileCells), share, s, a, K);
         else
           hipLaunchKernelGGL((level_step_tiled<3, false>), dim3(nb), dim3(kTileCells), share, s, a, K);
-        if (defer) hipLaunchKernelGGL((chem_straggler_kernel<3>), sg, sb, 0, s, a, K);
       }
-      return hipGetLastError();
+      const hipError_t e = hipGetLastError();
+      return e == hipSuccess && defer && stragglers ? launch_stragglers(a, K, s) : e;
     }
   }
   int nb = a.tiles ? a.ntiles : (a.ncell + kTileCells - 1) / kTileCells;
@@ -2201,8 +2207,8 @@ hipError_t launch_call_end(int* status, unsigned long long* counters, int* defer
   return hipGetLastError();
 }
 
-template hipError_t launch_level_step<double>(const LevelArgs<double>&, const ChemConst&, hipStream_t);
-template hipError_t launch_level_step<float>(const LevelArgs<float>&, const ChemConst&, hipStream_t);
+template hipError_t launch_level_step<double>(const LevelArgs<double>&, const ChemConst&, bool, hipStream_t);
+template hipError_t launch_level_step<float>(const LevelArgs<float>&, const ChemConst&, bool, hipStream_t);
 template int persistent_blocks_per_cu<double>(int, bool);
 template int persistent_blocks_per_cu<float>(int, bool);
 template hipError_t launch_persistent<double>(const SchedArgs&, int, bool, int, hipStream_t);

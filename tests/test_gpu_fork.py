@@ -32,13 +32,14 @@ def workload(table, lmin, counts, seed):
                                                ("Starburst99_1grpT_3grpS", 7, [60000, 2000, 300]),
                                                ("SB99_equiv_mono_TH", 7, [500, 100]),
                                                ("Starburst99_1grpT_3grpS", 6, [3000, 900])])
-@pytest.mark.parametrize("precision", [rt.FP64, rt.MIXED])
-def test_same_as_one_after_the_other(gpu_lib, table, lmin, counts, precision):
+@pytest.mark.parametrize("precision,budget", [(rt.FP64, 0), (rt.MIXED, 0), (rt.MIXED, 2)])
+def test_same_as_one_after_the_other(gpu_lib, table, lmin, counts, precision, budget):
     params, tree, fields = workload(table, lmin, counts, 5 + lmin + len(counts))
     out = []
     for timing in (rt.TIMING_LAUNCH, rt.TIMING_OFF):
         g = rt.RadGPU(params, precision)
         g.setup(params, tree, fields)
+        g.set_chem_budget(budget)  # > 0: both launches' straggler list
         g.save_state()
         for rep in range(3):
             g.restore_state()
