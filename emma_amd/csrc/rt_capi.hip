@@ -167,6 +167,9 @@ struct emma_rt_ctx {
   CallRecord* h_call = nullptr;  // page-locked: what the call's last kernel reports
   bool words_dirty = false;      // a call began and did not reach its end
   bool capturing = false;        // a coarse step's launches go into a graph
+  // coarse steps: the injection of the level step before waits for the next FillRad
+  bool hydro_waits = false;
+  HydroArgs hydro_args;
   void* scratch = nullptr;  // this device's no-alloc staging area (emma_rt_advance_stencil_noalloc)
   double* d_photons = nullptr;
   // straggler list of the tiled mixed kernel (capacity: the largest level's
@@ -1282,6 +1285,10 @@ static hipError_t launch_fill_cells(emma_rt_ctx* c, int k, double aexp) {
     memcpy(c->pending_fill[k].data(), &f, sizeof(f));
     return hipSuccess;
   }
+  if (c->hydro_waits) {  // with the injection of the step before
+    c->hydro_waits = false;
+    return launch_couple<R>(c->hydro_args, f, c->stream);
+  }
   return launch_fill_level<R>(f, c->stream);
 }
 
@@ -1291,7 +1298,9 @@ static hipError_t fill_cells(emma_rt_ctx* c, int k, double aexp) {
 }
 
 // RadSolver's injection into the hydro state after the level's final update
-static hipError_t to_hydro(emma_rt_ctx* c, int k) {
+// RadSolver's injection of level k; wait: with the next level step's FillRad
+// (end_hydro launches the last one)
+static hipError_t to_hydro(emma_rt_ctx* c, int k, bool wait = false) {
   DevLevel& L = c->lev[k];
   if (!c->hydro || L.noct == 0) return hipSuccess;
   HydroArgs h;
@@ -1322,7 +1331,18 @@ static hipError_t to_hydro(emma_rt_ctx* c, int k) {
     }
     return hipErrorInvalidValue;
   }
+  if (wait) {
+    c->hydro_args = h;
+    c->hydro_waits = true;
+    return hipSuccess;
+  }
   return launch_rad_to_hydro(h, c->stream);
+}
+
+static hipError_t end_hydro(emma_rt_ctx* c) {
+  if (!c->hydro_waits) return hipSuccess;
+  c->hydro_waits = false;
+  return launch_rad_to_hydro(c->hydro_args, c->stream);
 }
 
 extern "C" int emma_rt_set_hydro(emma_rt_ctx* c, int level, const double* d, const double* u, const double* v,
@@ -1493,7 +1513,7 @@ static int recurse_coarserad(emma_rt_ctx* c, int k, double aexp) {
   int st = timed_launch(c, k, dtrad_of(c->p, c->lmin, aexp), aexp, 0);
   if (st) return st;
   if (k == 0 && nl > 1) HIPCHK(launch_distrib(c));
-  HIPCHK(to_hydro(c, k));
+  HIPCHK(to_hydro(c, k, true));
   return EMMA_RT_OK;
 }
 
@@ -1516,7 +1536,7 @@ static int recurse(emma_rt_ctx* c, int k, double aexp) {
     HIPCHK(fill_cells(c, k, aexp));  // FillRad before RadSolver (advanceamr.c:1035)
     st = fork ? join_free(c, k, dt, aexp) : timed_launch(c, k, dt, aexp, 0);
     if (st) return st;
-    HIPCHK(to_hydro(c, k));
+    HIPCHK(to_hydro(c, k, true));
   }
   return EMMA_RT_OK;
 }
@@ -1720,10 +1740,12 @@ extern "C" int emma_rt_coarse_step(emma_rt_ctx* c, double aexp, int ncoarse) {
   st = begin_call(c);
   if (st) return st;
   if (eager && c->sched == EMMA_RT_SCHED_GRAPH) {  // eager launches with per-kernel events
+    c->hydro_waits = false;
     for (int i = 0; i < ncoarse; i++) {
       st = recurse(c, 0, aexp);
       if (st) return st;
     }
+    HIPCHK(end_hydro(c));
     return end_call(c);
   }
   GraphKey key;
@@ -1766,7 +1788,9 @@ extern "C" int emma_rt_coarse_step(emma_rt_ctx* c, double aexp, int ncoarse) {
       const int timing = c->timing;
       c->timing = 0;  // no event records inside the graph
       c->capturing = true;
+      c->hydro_waits = false;
       for (int i = 0; i < ncoarse && rs == EMMA_RT_OK; i++) rs = recurse(c, 0, aexp);
+      if (rs == EMMA_RT_OK && end_hydro(c) != hipSuccess) rs = EMMA_RT_ERR_HIP;
       c->capturing = false;
       if (rs == EMMA_RT_OK && queue_call_end(c) != hipSuccess) rs = EMMA_RT_ERR_HIP;
       c->timing = timing;

@@ -247,6 +247,9 @@ struct HydroArgs {
   double* E;
 };
 hipError_t launch_rad_to_hydro(const HydroArgs& h, hipStream_t s);
+// the injection of one level, then FillRad's block of another (or the same)
+template <typename R>
+hipError_t launch_couple(const HydroArgs& h, const FillArgs<R>& f, hipStream_t s);
 
 // ---------------------------------------------------------------- persistent coarse step
 // A coarse step (all its level steps, with FillRad's block before and the
