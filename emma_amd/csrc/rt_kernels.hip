@@ -665,13 +665,13 @@ __device__ __forceinline__ bool halo_cancel(const LevelArgs<R>& a, const HaloCel
   return h.on && !h.coarse && !a.keep_split_flux && gld(a.child, h.j) >= 0;
 }
 
-// group g of its state into LDS slot i, with its closure
-template <typename R, bool Fast>
-__device__ __forceinline__ void halo_put(const LevelArgs<R>& a, CellLds<R>& lds, const HaloCell& h, int g, int i) {
+// group g of its state
+template <typename R>
+__device__ __forceinline__ void halo_load(const LevelArgs<R>& a, const HaloCell& h, int g, R v[4]) {
   if (!h.on) return;
   // the lane's array is this level's plus a per-lane distance (0, or the
-  // coarse array's address minus this level's), both bases scalar: a 64-bit
-  // address per lane and array would live across the group loop
+  // coarse array's address minus this level's), both bases scalar: no 64-bit
+  // address per lane and array
   const size_t o = byte_offset<R>(h.j);
   auto load = [&](const R* own, const R* coarser) {
     const R* const ob = own + (size_t)g * a.ncell;
@@ -679,8 +679,18 @@ __device__ __forceinline__ void halo_put(const LevelArgs<R>& a, CellLds<R>& lds,
     const unsigned long long dist = (unsigned long long)cb - (unsigned long long)ob;
     return *(const EMMA_GLOBAL R*)(uniform_base(ob) + (h.coarse ? dist : 0ull) + o);
   };
-  const R ve = load(a.e, a.ce);
-  R vx = load(a.fx, a.cfx), vy = load(a.fy, a.cfy), vz = load(a.fz, a.cfz);
+  v[0] = load(a.e, a.ce);
+  v[1] = load(a.fx, a.cfx);
+  v[2] = load(a.fy, a.cfy);
+  v[3] = load(a.fz, a.cfz);
+}
+
+// into LDS slot i, with its closure
+template <typename R, bool Fast>
+__device__ __forceinline__ void halo_put(const LevelArgs<R>& a, CellLds<R>& lds, const HaloCell& h, const R v[4], int i) {
+  if (!h.on) return;
+  const R ve = v[0];
+  R vx = v[1], vy = v[2], vz = v[3];
   if (h.refl) {
     if (h.d == 0) vx = -vx;
     if (h.d == 1) vy = -vy;
@@ -693,10 +703,28 @@ __device__ __forceinline__ bool in_tile32(int no, int tile) {
   return no >= tile * kTileOcts && no < (tile + 1) * kTileOcts;
 }
 
-// the tile's cancel flags and, on complete levels, each wave's halo list (this
-// lane's entry in hl); before the first group's transport
+// sparse levels: the cell's own halo face of direction d
+__device__ __forceinline__ HaloCell own_face(const CellFaces& c, int tile, int d) {
+  return halo_cell(c.moves && !in_tile32(c.noD[d], tile), c.cell, d, c.noD[d]);
+}
+
+// group g of the cell's state
 template <typename R>
-__device__ __forceinline__ CellFaces cell_faces(const LevelArgs<R>& a, int tile, int lc, CellLds<R>& lds, HaloCell& hl) {
+__device__ __forceinline__ void own_load(const LevelArgs<R>& a, int cell, int g, R T[4]) {
+  if (cell >= a.ncell) return;
+  T[0] = gld(a.e + (size_t)g * a.ncell, cell);
+  T[1] = gld(a.fx + (size_t)g * a.ncell, cell);
+  T[2] = gld(a.fy + (size_t)g * a.ncell, cell);
+  T[3] = gld(a.fz + (size_t)g * a.ncell, cell);
+}
+
+// the tile's cancel flags and, on complete levels, each wave's halo list (this
+// lane's entry in hl); before the first group's transport.  The loads that group
+// g needs first go out here, with the ones they'd otherwise wait behind: the
+// cell's state T with the topology, the halo state H with the cancel flags
+template <typename R>
+__device__ __forceinline__ CellFaces cell_faces(const LevelArgs<R>& a, int tile, int lc, CellLds<R>& lds, HaloCell& hl,
+                                                int g, R T[4], R H[4]) {
   CellFaces c;
   const int wv = lc >> 6, lane = lc & 63;
   c.cell = tile * kTileCells + lc;
@@ -719,6 +747,7 @@ __device__ __forceinline__ CellFaces cell_faces(const LevelArgs<R>& a, int tile,
       for (int d = 0; d < 3; d++) c.noD[d] = gld(a.nei, oct * 6 + 2 * d + ((ic >> d) & 1));
     }
   }
+  own_load(a, c.cell, g, T);
   c.restricted = c.ch >= 0 && !a.update_split;  // takes its children's mean, no transport
   c.moves = c.valid && transport && !c.restricted;
   hl.on = false;
@@ -750,34 +779,38 @@ __device__ __forceinline__ CellFaces cell_faces(const LevelArgs<R>& a, int tile,
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const int it = lds.item[wv][lane];
     hl = halo_cell(lane < nhalo, (c.cell & ~63) + (it >> 2), it & 3, lds.item_nei[wv][lane]);
+    halo_load(a, hl, g, H);
     lds.cancel[kTileCells + lc] = (unsigned char)halo_cancel(a, hl);
   } else {
     // each lane's own slot serves one direction after the other: their flags
-    // as bits of one byte
+    // as bits of one byte (the three loads at once, lanes without a face read
+    // cell 0)
     unsigned flags = 0;
+    int hch[3];
+    bool on[3];
+    halo_load(a, own_face(c, tile, 0), g, H);
 #pragma unroll
-    for (int d = 0; d < 3; d++)
-      if (c.moves && !in_tile32(c.noD[d], tile))
-        flags |= halo_cancel(a, halo_cell(true, c.cell, d, c.noD[d])) ? 1u << d : 0u;
+    for (int d = 0; d < 3; d++) {
+      const HaloCell h = own_face(c, tile, d);
+      on[d] = h.on && !h.coarse && !a.keep_split_flux;
+      hch[d] = gld(a.child, on[d] ? h.j : 0);
+    }
+#pragma unroll
+    for (int d = 0; d < 3; d++) flags |= on[d] && hch[d] >= 0 ? 1u << d : 0u;
     lds.cancel[kTileCells + lc] = (unsigned char)flags;
   }
   return c;
 }
 
 // Transport of group g of the thread's cell: its updated state in T, the
-// refluxes of the finer octs folded in.  GA: groups of a reflux accumulator.
-// All threads of the work-group; the LDS is free again after a barrier.
+// refluxes of the finer octs folded in.  T and H come with the cell's and the
+// halo's state (from cell_faces; H is used up).  GA: groups of a reflux
+// accumulator.  All threads of the work-group.
 template <typename R, int GA, bool Fast>
 __device__ __forceinline__ void transport_group(const LevelArgs<R>& a, const CellFaces& cf, const HaloCell& hl, int tile,
-                                                int lc, CellLds<R>& lds, int g, R T[4]) {
+                                                int lc, CellLds<R>& lds, int g, R T[4], R H[4]) {
   const int ic = cf.cell & 7, hslot0 = kTileCells + (lc & ~63), lane = lc & 63;
   const R c = a.c, hc = a.hc, dts = a.dtsurdx;
-  if (cf.valid) {
-    T[0] = gld(a.e + (size_t)g * a.ncell, cf.cell);
-    T[1] = gld(a.fx + (size_t)g * a.ncell, cf.cell);
-    T[2] = gld(a.fy + (size_t)g * a.ncell, cf.cell);
-    T[3] = gld(a.fz + (size_t)g * a.ncell, cf.cell);
-  }
   const bool fold = cf.valid && !cf.restricted && cf.ch <= -2;
   if (!a.transport) {
     if (fold) fold_reflux<R, GA, 1, kRefluxCell>(a, cf.ch, g, 1, &T[0], &T[1], &T[2], &T[3]);
@@ -789,7 +822,7 @@ __device__ __forceinline__ void transport_group(const LevelArgs<R>& a, const Cel
     Q = closure_of<R, Fast>(ux, uy, uz, ue, c);
     lds.put(lc, ue, ux, uy, uz, Q);
   }
-  if (cf.listed) halo_put<R, Fast>(a, lds, hl, g, hslot0 + lane);
+  if (cf.listed) halo_put<R, Fast>(a, lds, hl, H, hslot0 + lane);
   __syncthreads();
   if (!cf.moves) return;
   R D[4] = {R(0), R(0), R(0), R(0)};
@@ -803,7 +836,10 @@ __device__ __forceinline__ void transport_group(const LevelArgs<R>& a, const Cel
     const int slot = cf.listed ? cf.hbase[d] + lanes_below_mask(cf.hball[d]) : lane;
     const int jout = inT ? jl : hslot0 + slot;
     // (own slot: written and read by this lane alone)
-    if (!cf.listed && !inT) halo_put<R, Fast>(a, lds, halo_cell(true, cf.cell, d, cf.noD[d]), g, jout);
+    if (!cf.listed) {
+      halo_put<R, Fast>(a, lds, own_face(cf, tile, d), H, hslot0 + lane);
+      if (d < 2) halo_load(a, own_face(cf, tile, d + 1), g, H);
+    }
     const bool cin = lds.cancel[jin] != 0;
     const bool cout = (cf.listed || inT) ? lds.cancel[jout] != 0 : ((lds.cancel[jout] >> d) & 1) != 0;
     // the flux from a neighbour is multiplied by 0 or 1 (rad_utils.c:518-526)
@@ -847,9 +883,9 @@ __global__ __launch_bounds__(kTileCells) __attribute__((amdgpu_waves_per_eu(4)))
   const int tile = block_tile(a), lc = (int)threadIdx.x;
   if (tile < 0) return;
   HaloCell hl;
-  const CellFaces cf = cell_faces(a, tile, lc, lds, hl);
-  double T[4];
-  transport_group<double, 1, false>(a, cf, hl, tile, lc, lds, 0, T);
+  double T[4], H[4];
+  const CellFaces cf = cell_faces(a, tile, lc, lds, hl, 0, T, H);
+  transport_group<double, 1, false>(a, cf, hl, tile, lc, lds, 0, T, H);
   unsigned int nit_acc = 0, leaf = 0;
   if (cf.valid) {
     if (a.t_first != nullptr) xion_times(a, cf.cell);
@@ -866,37 +902,34 @@ __global__ __launch_bounds__(kTileCells) __attribute__((amdgpu_waves_per_eu(4)))
 }
 
 // More groups: the transport as a kernel of its own, one group a work-group
-// (gridDim.y of them side by side), which leaves the transported state in the
-// next state's arrays, and the chemistry after it.  In one kernel the chemistry's
-// registers (168 to 256) held the transport to one to three waves per SIMD, and
-// a small level waited for all groups' transport in one wave's chain; apart, the
-// transport takes 125 (FP32 76).  A level step of 32^3 cells, nine FP64 groups:
-// 41 -> 27 us, though the transported state is written and read once more;
-// 64^3 cells, nine FP32 groups 55.4 -> 52.2 us, three FP64 groups 64 -> 62 us,
-// of 4,600 and 20,000 cells below it 27 -> 22.8 and 42 -> 41 us.
+// (gridDim.y = ng), which leaves the transported state in the next state's
+// arrays, and the chemistry after it.  In one kernel the chemistry's registers
+// (168 to 256) held the transport to one to three waves per SIMD, and a small
+// level waited for all groups' transport in one wave's chain; apart, the
+// transport takes 94 (FP32 51).  A level step of 32^3 cells, nine FP64 groups:
+// 41 -> 26.2 us, though the transported state is written and read once more;
+// 64^3 cells, nine FP32 groups 55.4 -> 49.6 us.  A work-group that took several
+// groups in turn to reuse the topology kept more alive across them (125 and 76
+// registers) and was slower at both sizes, 27.0 and 51.3 us.
 template <typename R, int GA, bool Fast>
 __global__ __launch_bounds__(kTileCells) void transport_kernel(LevelArgs<R> a_by_value, ChemConst K_by_value) {
   const LevelArgs<R>& a = kernargs<R>().a;
   CellLds<R>& lds = *cell_lds<R>();
-  const int tile = block_tile(a), lc = (int)threadIdx.x;
+  const int tile = block_tile(a), lc = (int)threadIdx.x, g = (int)blockIdx.y;
   if (tile < 0) return;
   HaloCell hl;
-  const CellFaces cf = cell_faces(a, tile, lc, lds, hl);
-  for (int g = (int)blockIdx.y; g < a.ng; g += (int)gridDim.y) {
-    R T[4];
-    transport_group<R, GA, Fast>(a, cf, hl, tile, lc, lds, g, T);
-    if (cf.valid && !cf.restricted) {
-      const size_t o = (size_t)g * a.ncell;
-      gst(a.eo + o, cf.cell, T[0]);
-      gst(a.fxo + o, cf.cell, T[1]);
-      gst(a.fyo + o, cf.cell, T[2]);
-      gst(a.fzo + o, cf.cell, T[3]);
-      // COARSERAD: a split cell's check (a leaf's is the chemistry's)
-      if (cf.ch >= 0 && ((g == 0 && (T[0] < R(0) || isnan(T[0]))) || (g == 1 && isnan(T[0]))))
-        raise_status(a.status, -3, a.level, cf.cell);
-    }
-    if (g + (int)gridDim.y < a.ng) __syncthreads();  // the next group overwrites the tile's state
-  }
+  R T[4], H[4];
+  const CellFaces cf = cell_faces(a, tile, lc, lds, hl, g, T, H);
+  transport_group<R, GA, Fast>(a, cf, hl, tile, lc, lds, g, T, H);
+  if (!cf.valid || cf.restricted) return;
+  const size_t o = (size_t)g * a.ncell;
+  gst(a.eo + o, cf.cell, T[0]);
+  gst(a.fxo + o, cf.cell, T[1]);
+  gst(a.fyo + o, cf.cell, T[2]);
+  gst(a.fzo + o, cf.cell, T[3]);
+  // COARSERAD: a split cell's check (a leaf's is the chemistry's)
+  if (cf.ch >= 0 && ((g == 0 && (T[0] < R(0) || isnan(T[0]))) || (g == 1 && isnan(T[0]))))
+    raise_status(a.status, -3, a.level, cf.cell);
 }
 
 // (191 VGPRs for three FP64 groups, 208 for nine FP32 ones: held to 128 or 168
@@ -2040,15 +2073,6 @@ __global__ __launch_bounds__(kTileCells) __attribute__((amdgpu_waves_per_eu(Tile
 }
 
 // ------------------------------------------------------------------ launchers
-// Work-groups side by side over the photon groups of a tile: all of them while
-// that is up to eight work-groups per CU (32^3 cells, nine groups: 27 us, with
-// three at a time 29), otherwise three, so that a tile's topology and halo
-// list serve several groups (64^3 cells: 52 us, with nine 57).
-static unsigned transport_groups(int nb, int ng) {
-  constexpr int kFull = 2048;
-  return (unsigned)(nb * ng <= kFull ? ng : std::min(ng, 3));
-}
-
 constexpr unsigned kCuLds = 160 * 1024;
 static_assert(sizeof(TileLds<3>) < kCuLds / 4, "four work-groups a CU");
 template <int G>
@@ -2113,11 +2137,13 @@ hipError_t launch_level_step(const LevelArgs<R>& a0, const ChemConst& K, bool st
       return hipGetLastError();
     }
   }
-  const dim3 tgrid(nb, transport_groups(nb, a.ng));
-  if (!fast && a.ng == 3)  // (three FP32 groups took the tiled kernel)
-    hipLaunchKernelGGL((transport_kernel<R, 3, fast>), tgrid, block, 0, s, a, K);
-  else
-    hipLaunchKernelGGL((transport_kernel<R, kMaxGrp, fast>), tgrid, block, 0, s, a, K);
+  const dim3 tgrid(nb, a.ng);
+  bool three = false;
+  if constexpr (!fast) {  // (three FP32 groups took the tiled kernel)
+    three = a.ng == 3;
+    if (three) hipLaunchKernelGGL((transport_kernel<R, 3, fast>), tgrid, block, 0, s, a, K);
+  }
+  if (!three) hipLaunchKernelGGL((transport_kernel<R, kMaxGrp, fast>), tgrid, block, 0, s, a, K);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   switch (a.ng) {
