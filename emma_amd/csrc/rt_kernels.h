@@ -70,7 +70,7 @@ struct LevelArgs {
   const int* child;
   const int* nei;
   const int* rpair;  // [noct][6]: the coarser level's reflux pair of each oct face, -1 if none
-  R* racc;           // this level's reflux accumulators: [nslot][4][GA], an accumulator's values contiguous
+  R* racc;           // this level's reflux accumulators: [pair][GA][4][sub-slot] (acc_at)
   // coarser level: current state (injection), child table, reflux accumulators
   const R* ce;
   const R* cfx;

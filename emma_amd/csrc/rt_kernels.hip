@@ -244,20 +244,31 @@ __device__ __forceinline__ void restrict_cell(const LevelArgs<R>& a, int cell, i
   restrict_scalars(a, cell, ch);
 }
 
+// Reflux accumulators: [pair][group][component][sub-slot].  The sub-slots (one
+// per cell of the oct face, Sub = 4, or the face's sum, Sub = 1) are innermost:
+// the four lanes of an oct face add a component to adjacent words, one request
+// of the L2's atomic units in place of four, and a (pair, group) is one 128 B
+// line in FP64, read back with wide loads.  With the sub-slot outside
+// ([pair][sub-slot][component][group]) the three-group FP64 tree of 64^3 cells
+// and 9,000 and 2,500 octs took 213.5 us a coarse step, 41 of them the adds and
+// 9 the reads; now 171.5.
+template <int GA, int Sub>
+__device__ __forceinline__ size_t acc_at(int pair, int g) {
+  return ((size_t)pair * GA + g) * (4 * Sub);
+}
+
 // reflux of one face flux into the coarse leaf behind it (scatterstencilrad,
 // rad_utils.c:1738-1762): the coarse cell gains -/+ F dt/dx / 8.  The cell's
 // own accumulator of the reflux pair p (sub-slot q: its place in the oct
-// face), its 4 x GA values contiguous.  No other lane adds to it in this
-// launch, so the sum is the same every run; the add is an atomic only so
-// that the lane need not wait for the old value.
+// face).  No other lane adds to it in this launch, so the sum is the same every
+// run; the add is an atomic only so that the lane need not wait for the old
+// value.
 template <typename R, int GA>
 __device__ __forceinline__ void reflux(const LevelArgs<R>& a, int p, int q, int f, int g, const R F[4], R dts) {
-  R* acc = a.cracc + ((size_t)p * kRefluxCell + q) * 4 * GA;
+  R* acc = a.cracc + acc_at<GA, kRefluxCell>(p, g) + q;
   const R w = (f & 1) ? R(1) : R(-1);  // pow(-1, face+1)
-  atomicAdd(acc + 0 * GA + g, F[0] * dts * w * R(0.125));
-  atomicAdd(acc + 1 * GA + g, F[1] * dts * w * R(0.125));
-  atomicAdd(acc + 2 * GA + g, F[2] * dts * w * R(0.125));
-  atomicAdd(acc + 3 * GA + g, F[3] * dts * w * R(0.125));
+#pragma unroll
+  for (int v = 0; v < 4; v++) atomicAdd(acc + v * kRefluxCell, F[v] * dts * w * R(0.125));
 }
 
 // the refluxes of the finer octs behind a leaf's faces, added to its base
@@ -266,38 +277,42 @@ __device__ __forceinline__ void reflux(const LevelArgs<R>& a, int p, int q, int 
 template <typename R, int GA, int NG, int Sub>
 __device__ __forceinline__ void fold_reflux(const LevelArgs<R>& a, int ch, int g0, int ng, R* Ue, R* Ux, R* Uy, R* Uz) {
   const int code = -2 - ch;
-  R* acc = a.racc + (size_t)(code >> 3) * Sub * 4 * GA + g0;
-  const int m = (code & 7) * Sub;
+  const int p0 = code >> 3, m = code & 7;
   // all loads before the clearing stores.  A leaf has at most six pairs:
   // the tiled kernel's loop unrolls, and its loads (an accumulator's 4G
   // values are contiguous), clamped to the leaf's last accumulator, go out
-  // together instead of one pair after another
-  constexpr int kMaxSub = 6 * Sub;
+  // together instead of one pair after another; the per-cell kernels take a
+  // pair's 16 values of a group at a time
+  constexpr int kPairs = 6;
   R s[NG][4];
 #pragma unroll
   for (int g = 0; g < NG; g++) s[g][0] = s[g][1] = s[g][2] = s[g][3] = R(0);
-#pragma unroll(Sub == 1 ? kMaxSub : 1)
-  for (int i = 0; i < (Sub == 1 ? kMaxSub : m); i++) {
-    const R* p = acc + (size_t)min(i, m - 1) * 4 * GA;
+#pragma unroll(Sub == 1 ? kPairs : 1)
+  for (int i = 0; i < (Sub == 1 ? kPairs : m); i++) {
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
+    for (int g = 0; g < NG; g++) {
+      if (g < ng) {
+        const R* p = a.racc + acc_at<GA, Sub>(p0 + min(i, m - 1), g0 + g);
+        R x[4 * Sub];
 #pragma unroll
-      for (int g = 0; g < NG; g++) {
-        if (g < ng) {
-          const R x = p[v * GA + g];
-          s[g][v] += i < m ? x : R(0);
-        }
+        for (int k = 0; k < 4 * Sub; k++) x[k] = p[k];
+#pragma unroll
+        for (int q = 0; q < Sub; q++)
+#pragma unroll
+          for (int v = 0; v < 4; v++) s[g][v] += i < m ? x[v * Sub + q] : R(0);
       }
     }
   }
-#pragma unroll(Sub == 1 ? kMaxSub : 1)
-  for (int i = 0; i < kMaxSub; i++) {
+#pragma unroll(Sub == 1 ? kPairs : 1)
+  for (int i = 0; i < (Sub == 1 ? kPairs : m); i++) {
     if (i < m) {
 #pragma unroll
-      for (int v = 0; v < 4; v++) {
+      for (int g = 0; g < NG; g++) {
+        if (g < ng) {
+          R* p = a.racc + acc_at<GA, Sub>(p0 + i, g0 + g);
 #pragma unroll
-        for (int g = 0; g < NG; g++)
-          if (g < ng) acc[(size_t)i * 4 * GA + v * GA + g] = R(0);
+          for (int k = 0; k < 4 * Sub; k++) p[k] = R(0);
+        }
       }
     }
   }
@@ -906,7 +921,7 @@ __global__ __launch_bounds__(kTileCells) __attribute__((amdgpu_waves_per_eu(4)))
 // arrays, and the chemistry after it.  In one kernel the chemistry's registers
 // (168 to 256) held the transport to one to three waves per SIMD, and a small
 // level waited for all groups' transport in one wave's chain; apart, the
-// transport takes 94 (FP32 51).  A level step of 32^3 cells, nine FP64 groups:
+// transport takes 106 (FP32 58).  A level step of 32^3 cells, nine FP64 groups:
 // 41 -> 26.2 us, though the transported state is written and read once more;
 // 64^3 cells, nine FP32 groups 55.4 -> 49.6 us.  A work-group that took several
 // groups in turn to reuse the topology kept more alive across them (125 and 76
@@ -1343,20 +1358,20 @@ __device__ __forceinline__ void tiled_step(const LevelArgs<float>& a, const Chem
         const unsigned long long mine = rmask & grp;
         const int pr = pairD[d];
         if (rj >= 0 && pr >= 0) {
-          float* acc = a.cracc + (size_t)pr * kRefluxTiled * 4 * G;
+          float* acc = a.cracc + acc_at<G, kRefluxTiled>(pr, 0);
           const float w = (bit ? 1.f : -1.f) * (0.5f * dts) * 0.125f;  // pow(-1, face+1) dt/dx / 8, shares doubled
           if (mine == grp) {  // the face's four cells all carry flux (always, with 2:1 balance)
             const int k = __popcll(mine & ((1ull << lane) - 1ull));  // component of this lane
 #pragma unroll
             for (int g = 0; g < G; g++) {
               const float x = k == 0 ? Rf[g][0] : (k == 1 ? Rf[g][1] : (k == 2 ? Rf[g][2] : Rf[g][3]));
-              atomicAdd(acc + k * G + g, x * w);
+              atomicAdd(acc + g * 4 + k, x * w);
             }
           } else if (lane == __builtin_ctzll(mine)) {
 #pragma unroll
             for (int g = 0; g < G; g++)
 #pragma unroll
-              for (int v = 0; v < 4; v++) atomicAdd(acc + v * G + g, Rf[g][v] * w);
+              for (int v = 0; v < 4; v++) atomicAdd(acc + g * 4 + v, Rf[g][v] * w);
           }
         }
       }
@@ -1615,15 +1630,15 @@ __global__ __launch_bounds__(64 * G) void level_step_split(LevelArgs<float> a_by
         const unsigned long long mine = rmask & grp;
         const int pr = pairD[d];
         if (rj >= 0 && pr >= 0) {
-          float* acc = a.cracc + (size_t)pr * kRefluxTiled * 4 * G + g;
+          float* acc = a.cracc + acc_at<G, kRefluxTiled>(pr, g);
           const float w = (bit ? 1.f : -1.f) * (0.5f * dts) * 0.125f;  // pow(-1, face+1) dt/dx / 8, shares doubled
           if (mine == grp) {
             const int k = __popcll(mine & ((1ull << lane) - 1ull));  // component of this lane
             const float x = k == 0 ? Rf[0] : (k == 1 ? Rf[1] : (k == 2 ? Rf[2] : Rf[3]));
-            atomicAdd(acc + k * G, x * w);
+            atomicAdd(acc + k, x * w);
           } else if (lane == __builtin_ctzll(mine)) {
 #pragma unroll
-            for (int v = 0; v < 4; v++) atomicAdd(acc + v * G, Rf[v] * w);
+            for (int v = 0; v < 4; v++) atomicAdd(acc + v, Rf[v] * w);
           }
         }
       }
