@@ -71,6 +71,8 @@ struct DevLevel {
   int* nei = nullptr;
   int* rpair = nullptr;  // [noct][6] reflux pair of each face in the coarser level, -1 if none
   void* racc = nullptr;
+  int* split = nullptr;  // the coarsest level's split cells (COARSERAD transfers)
+  int nsplit = 0;
   double* t_first = nullptr;
   double* t_last = nullptr;
   // the level's tiles that no finer level touches (no split cell, no leaf with
@@ -237,6 +239,7 @@ static void free_tree(emma_rt_ctx* c) {
     (void)hipFree(L.racc);
     (void)hipFree(L.rpair);
     (void)hipFree(L.tiles);
+    (void)hipFree(L.split);
     (void)hipFree(L.defer);
     if (L.forked) (void)hipEventDestroy(L.forked);
     if (L.joined) (void)hipEventDestroy(L.joined);
@@ -659,6 +662,16 @@ extern "C" int emma_rt_tree_create(emma_rt_ctx* c, int lmin, int lmax, const int
         tiles.insert(tiles.end(), touched.begin(), touched.end());
         HIPCHK(dalloc(&L.tiles, tiles.size()));
         HIPCHK(hipMemcpy(L.tiles, tiles.data(), tiles.size() * sizeof(int), hipMemcpyHostToDevice));
+      }
+    }
+    if (k == 0 && nl > 1) {
+      std::vector<int> split;
+      for (int i = 0; i < L.ncell; i++)
+        if (L.hchild[i] >= 0) split.push_back(i);
+      if (!split.empty()) {
+        HIPCHK(dalloc(&L.split, split.size()));
+        HIPCHK(hipMemcpy(L.split, split.data(), split.size() * sizeof(int), hipMemcpyHostToDevice));
+        L.nsplit = (int)split.size();
       }
     }
     const size_t gn = (size_t)G * L.ncell;
@@ -1148,6 +1161,8 @@ static TreeView<R> tree_view(emma_rt_ctx* c) {
   t.nlev = (int)c->lev.size();
   t.ng = c->p.ngrp;
   t.lcoarse = c->lmin;
+  t.nsplit = c->lev[0].nsplit;
+  t.split = c->lev[0].split;
   for (int k = 0; k < t.nlev; k++) {
     DevLevel& L = c->lev[k];
     t.ncell[k] = L.ncell;

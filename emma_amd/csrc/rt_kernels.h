@@ -167,11 +167,13 @@ hipError_t launch_stragglers(const LevelArgs<float>& a, const ChemConst& K, hipS
 
 // Levels of a tree for the COARSERAD transfers between the coarse level and
 // the leaves (putE2coarse / distribE): per level (index level - lcoarse) the
-// child table and the current photon density / flux.
+// child table and the current photon density / flux; split: the coarse level's
+// split cells.
 constexpr int kMaxLevels = 16;
 template <typename R>
 struct TreeView {
-  int nlev, ng, lcoarse, pad;
+  int nlev, ng, lcoarse, nsplit;
+  const int* split;
   int ncell[kMaxLevels];
   const int* child[kMaxLevels];
   R* e[kMaxLevels];
