@@ -184,12 +184,15 @@ def _dominant(W, precision, level_us, launches_per_step):
 
 
 KERNEL_NAMES = {"listed": "emma::level_step_tiled<{G}, false>", "perdir": "emma::level_step_tiled<{G}, true>",
-                "latency": "emma::level_step_tiled_latency<{G}>"}
+                "latency": "emma::level_step_split<{G}>"}
 
 
 def _kernel_name(W, level, precision, tuning):
     if precision != "mixed" or W.params.ngrp not in (1, 3):
-        return f"emma::level_step_kernel<{'double' if precision == 'fp64' else 'float'}, {W.params.ngrp}, ...>"
+        real, G = "double" if precision == "fp64" else "float", W.params.ngrp
+        if precision == "fp64" and G == 1:
+            return "emma::level_step_kernel"
+        return f"emma::transport_kernel<{real}, ...> + emma::chemistry_kernel<{real}, {G}, ...>"
     t = tuning[level]
     name = KERNEL_NAMES[t["variant"]].format(G=W.params.ngrp)
     return name + (" + emma::chem_straggler_kernel<%d>" % W.params.ngrp if t["chem_budget"] > 0 else "")

@@ -939,9 +939,10 @@ static hipError_t launch_level(emma_rt_ctx* c, int k, double dtnew, double aexp,
 // (join_free): the small levels' launches, each a few work-groups' latency,
 // run beside it.  With a chemistry budget both launches append to one straggler
 // list, whose pass follows the join.  Not with FillRad's block or the hydro
-// injection (they touch all cells), or the raster order.  Results are the same bit for bit.  The five-level tree's coarse
-// step (24 of 31 launches of at most 190 tiles): 0.575 -> 0.541 ms, its first
-// one, with long chemistry chains in the large levels, 1.07 -> 0.91 ms.
+// injection (they touch all cells), or the raster order.  Results are the same
+// bit for bit.  The five-level tree's coarse step (24 of 31 launches of at most
+// 190 tiles): 0.575 -> 0.541 ms, its first one, with long chemistry chains in
+// the large levels, 1.07 -> 0.91 ms.
 static bool can_fork(emma_rt_ctx* c, int k) {
   const DevLevel& L = c->lev[k];
   return c->capturing && !c->rec && L.tiles != nullptr && c->mode == EMMA_RT_RADSTEP && !c->hydro && !c->star &&
@@ -1072,9 +1073,10 @@ static long long steps_per_call(emma_rt_ctx* c, int ncoarse) {
 // A call finds them zero: its last kernel (call_end_kernel) reports the status
 // and the summed counters into a page-locked record and clears the words for
 // the next call, in place of three fill launches before the call's work and two
-// copies behind it (a level step of 16^3 cells from the host: 41 us a call
-// with them, 23 us now, 6 us of it the level step).  A call that ended early left them dirty: the
-// next one clears them.
+// copies behind it (a level step of 16^3 cells from the host: 41 us a call with
+// them, 23 us now, 6 us of it the level step; reported by the level step's own
+// last work-group, the counting of work-groups takes what the launch saves).  A
+// call that ended early left them dirty: the next one clears them.
 static int clear_call_words(emma_rt_ctx* c) {
   HIPCHK(launch_fill((unsigned int*)c->d_status, 4, 0u, c->stream));
   if (c->defer_slots > 0) HIPCHK(launch_fill((unsigned int*)c->d_defer_ctl, c->defer_slots, 0u, c->stream));
@@ -2198,8 +2200,7 @@ static int advance_stencil_on(emma_rt_ctx* c, void* dbuf, int real_bytes, void* 
   }
   // Ordinary memory: whole records in one copy each way (strided copies of
   // the parts alone run row by row there: 1501 records with three FP32 groups
-  // took 205 ms).  What the kernel does not write comes back as
-  // it went.
+  // took 205 ms).  What the kernel does not write comes back as it went.
   HIPCHK(hipMemcpyAsync(dbuf, h, total, hipMemcpyHostToDevice, c->stream));
   HIPCHK(launch(dbuf, false));
   HIPCHK(hipMemcpyAsync(h, dbuf, total, hipMemcpyDeviceToHost, c->stream));

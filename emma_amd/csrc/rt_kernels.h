@@ -19,8 +19,8 @@ struct LevelArgs {
   // level and not for chemonly calls, fluxes of split neighbours kept, split
   // cells transport-updated (their chemistry still skipped).
   int transport, keep_split_flux, update_split;
-  // mixed path, 1 or 3 groups: the halo variant of the tiled kernel
-  // (kListed, kPerDir or kLatency)
+  // kListed, kPerDir or kLatency: how the mixed path's kernels for 1 and 3
+  // groups reach the halo; the per-cell kernels know kListed from the others
   int variant;
   // > 0: the level is a complete periodic cube of 2^raster_m octs a side in
   // Morton order, and the tiled kernel walks each XCD's octant of tiles in
@@ -134,11 +134,10 @@ constexpr int kTileWaves = kTileCells / 64;
 //           start of pass d (up to 192 per wave: sparse AMR levels); the
 //           leaves' chemistry inputs are loaded at the start of the last
 //           pass (fewer live registers: four work-groups per CU).
-//  kLatency as kPerDir, but the halo faces of all three directions and the
-//           chemistry inputs are loaded up front: one memory round trip
-//           instead of four, with the registers that takes (two waves per
-//           SIMD).  For levels too small to fill the GPU, whose step is one
-//           work-group's latency chain.
+//  kLatency a kernel of its own (level_step_split): 64 cells a work-group,
+//           one wave per photon group, every halo load up front.  For levels
+//           too small to fill the GPU, whose step is one work-group's latency
+//           chain.
 constexpr int kListed = 0;
 constexpr int kPerDir = 1;
 constexpr int kLatency = 2;

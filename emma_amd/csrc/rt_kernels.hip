@@ -502,7 +502,7 @@ __device__ __forceinline__ void block_counters(unsigned long long* counters, uns
 // One thread per cell; neighbours straight from global memory.  Fast selects
 // the mixed-precision physics (rt_physics_fast.h); FP64 (Fast = false) keeps
 // the reference's operation order.  The persistent kernel's per-cell items;
-// the per-level launches run cell_step_lds below.
+// the per-level launches run the kernels below through LDS.
 // The cells of block `block` (256 consecutive cells, 32 octs).
 template <typename R, int G, bool Fast>
 __device__ __forceinline__ void cell_step(const LevelArgs<R>& a, const ChemConst& K, int block, int lc) {
@@ -1021,8 +1021,7 @@ __device__ __forceinline__ float lane_xor(float x, int m) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(t, 0x1B, 0xF, 0xF, true));              // quad_perm 3,2,1,0
 }
 
-// The halo variants kListed, kPerDir, kLatency (rt_kernels.h) share this
-// body; the kernels below instantiate it.
+// The halo variants kListed and kPerDir (rt_kernels.h) share the body below.
 // one halo face: the neighbour's state, its split flag, the face direction
 // and the side the neighbour lies on
 template <int G>

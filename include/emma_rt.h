@@ -334,8 +334,9 @@ int emma_rt_set_chem_keep(emma_rt_ctx *ctx, int level, double keep);
            complete levels; EMMA_RT_ERR_ARG on a level with more);
    PERDIR  each lane's own halo face per direction pass, chemistry inputs
            loaded late (fewest live registers; large sparse levels);
-   LATENCY all halo faces and inputs loaded up front (one memory round trip;
-           small levels whose step is one work-group's latency);
+   LATENCY 64 cells a work-group, one wave per photon group, all halo faces
+           and inputs loaded up front (small levels whose step is one
+           work-group's latency);
    AUTO    the library's choice at tree creation (LISTED where possible,
            LATENCY on sparse levels of at most 256 tiles of 32 octs, PERDIR
            otherwise).  The reference's analogue is the CUDA launch shape it
