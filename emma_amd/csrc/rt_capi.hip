@@ -166,7 +166,7 @@ struct emma_rt_ctx {
   std::vector<DevLevel> lev;  // index level - lmin
   int* d_status = nullptr;
   unsigned long long* d_counters = nullptr;
-  CallRecord* h_call = nullptr;  // page-locked: what the call's last kernel reports
+  CallRecord* h_call = nullptr;  // page-locked, coherent: what the call's last kernel reports
   bool words_dirty = false;      // a call began and did not reach its end
   bool capturing = false;        // a coarse step's launches go into a graph
   // coarse steps: the injection of the level step before waits for the next FillRad
@@ -439,7 +439,7 @@ extern "C" int emma_rt_create(const emma_rt_params* p, emma_rt_ctx** out) {
       hipMalloc((void**)&c->d_status, 4 * sizeof(int)) != hipSuccess ||
       hipMalloc((void**)&c->d_counters, kCounterSlots * kCounterStride * sizeof(unsigned long long)) != hipSuccess ||
       hipMalloc((void**)&c->d_photons, sizeof(double)) != hipSuccess ||
-      hipHostMalloc((void**)&c->h_call, sizeof(CallRecord)) != hipSuccess) {
+      hipHostMalloc((void**)&c->h_call, sizeof(CallRecord), hipHostMallocCoherent) != hipSuccess) {
     emma_rt_destroy(c);
     return EMMA_RT_ERR_HIP;
   }
@@ -2139,7 +2139,7 @@ extern "C" int emma_rt_create_pinned_stencil(emma_rt_ctx* c, int stride, int rea
   RgridLayout L;
   if (!rgrid_layout(c->p.ngrp, real_bytes, &L)) return EMMA_RT_ERR_ARG;
   *out = nullptr;
-  HIPCHK(hipHostMalloc(out, (size_t)stride * L.v[19], hipHostMallocDefault));
+  HIPCHK(hipHostMalloc(out, (size_t)stride * L.v[19], hipHostMallocCoherent));
   memset(*out, 0, (size_t)stride * L.v[19]);
   return EMMA_RT_OK;
 }
@@ -2147,7 +2147,7 @@ extern "C" int emma_rt_create_pinned_stencil(emma_rt_ctx* c, int stride, int rea
 extern "C" int emma_rt_alloc_pinned(size_t bytes, void** out) {
   if (out == nullptr || bytes == 0) return EMMA_RT_ERR_ARG;
   *out = nullptr;
-  HIPCHK(hipHostMalloc(out, bytes, hipHostMallocDefault));
+  HIPCHK(hipHostMalloc(out, bytes, hipHostMallocCoherent));
   memset(*out, 0, bytes);
   return EMMA_RT_OK;
 }
@@ -2158,8 +2158,9 @@ extern "C" int emma_rt_destroy_pinned_stencil(void* stencil) {
 }
 
 // the device address of page-locked host memory [h, h + bytes), null where it
-// is not (all) page-locked
-static void* mapped_host(char* h, size_t bytes) {
+// is not (all) page-locked; coherent: allocated with hipHostMallocCoherent, so
+// that the host reads a finished kernel's stores without a synchronisation
+static void* mapped_host(char* h, size_t bytes, bool* coherent) {
   hipPointerAttribute_t a, b;
   if (hipPointerGetAttributes(&a, h) != hipSuccess || hipPointerGetAttributes(&b, h + bytes - 1) != hipSuccess) {
     (void)hipGetLastError();  // ordinary memory
@@ -2168,6 +2169,12 @@ static void* mapped_host(char* h, size_t bytes) {
   if (a.type != hipMemoryTypeHost || b.type != hipMemoryTypeHost || a.devicePointer == nullptr ||
       (char*)b.devicePointer - (char*)a.devicePointer != (ptrdiff_t)(bytes - 1))
     return nullptr;
+  unsigned flags = 0;
+  if (hipHostGetFlags(&flags, h) != hipSuccess) {
+    (void)hipGetLastError();
+    flags = 0;
+  }
+  *coherent = (flags & hipHostMallocCoherent) != 0;
   return a.devicePointer;
 }
 
@@ -2193,10 +2200,16 @@ static int advance_stencil_on(emma_rt_ctx* c, void* dbuf, int real_bytes, void* 
   };
   const size_t rsize = (size_t)L.v[19], total = rsize * (size_t)nread;
   char* h = (char*)stencil;
-  void* mapped = mapped_host(h, total);
+  bool coherent = false;
+  void* mapped = mapped_host(h, total, &coherent);
   if (mapped != nullptr && ((size_t)mapped & 15) == 0) {
     HIPCHK(launch(mapped, true));
-    return end_call(c);
+    if (coherent) return end_call(c);
+    // the record's flag says that the stores are done, not that the host sees
+    // them in memory of another kind
+    HIPCHK(queue_call_end(c));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    return end_call(c, true);
   }
   // Ordinary memory: whole records in one copy each way (strided copies of
   // the parts alone run row by row there: 1501 records with three FP32 groups

@@ -1,0 +1,74 @@
+"""The library's host code against a host model of the HIP runtime."""
+import ctypes
+import dataclasses
+
+import numpy as np
+
+import hip_model as hm
+from emma_amd import rgrid, synth
+from emma_amd import tree as T
+from emma_amd.params import make_params
+from hip_model import modelled
+
+
+def _params(G, level):
+    p = make_params({1: "SB99_equiv_mono_TH", 3: "Starburst99_1grpT_3grpS"}[G])
+    return dataclasses.replace(p, lcoarse=level)
+
+
+def _fields(G, tree, seed=1):
+    rng = np.random.default_rng(seed)
+    p = _params(G, tree.lmin)
+    return {l: synth.random_fields(p, np.ones(tree.level(l).ncell), rng) for l in range(tree.lmin, tree.lmax + 1)}
+
+
+def _batch(n, G=1, align=16):
+    """n records in ordinary memory, their first byte at a multiple of `align` but not of twice that"""
+    size = rgrid.rgrid_dtype(G, 8).itemsize * n
+    raw = np.zeros(size + 4096, np.uint8)
+    at = (-raw.ctypes.data) % 4096 + align % 4096
+    st = raw[at : at + size].view(rgrid.rgrid_dtype(G, 8))
+    return raw, st
+
+
+def _stencil_context(rt, n, G=1):
+    p = _params(G, 4)
+    g = rt.RadGPU(p, rt.FP64)
+    g.create_radstencil(n, 8)
+    return g, lambda st: g.advance_stencil(st, n, 0.5**4, p.dt_rad(4))
+
+
+# ---------------------------------------------------------------- batches in place
+@modelled
+def test_records_not_known_coherent_are_waited_for(m, rt):
+    """Results written into page-locked memory by a kernel are the host's to
+    read after a runtime synchronisation, or at once if the memory is coherent."""
+    g, advance = _stencil_context(rt, 5)
+    keep = []  # the model holds on to their ranges
+    for flags in (0, hm.PORTABLE, hm.NONCOHERENT):
+        raw, st = _batch(5)
+        keep.append(raw)
+        m.model_lock(raw.ctypes.data, raw.nbytes, flags)
+        m.model_forget()
+        before = m.model_stream_waits()
+        advance(st)
+        assert any("stencil_direct_kernel" in k for k in m.launched()), flags
+        assert m.model_stream_waits() > before, flags
+    pinned = g.pinned_stencil(5, 8)
+    pinned.array[:] = st
+    m.model_forget()
+    before = m.model_stream_waits()
+    advance(pinned.array)
+    assert any("stencil_direct_kernel" in k for k in m.launched())
+    assert m.model_stream_waits() == before
+
+
+@modelled
+def test_own_page_locked_memory_is_coherent(m, rt):
+    """the call record is polled while kernels run; transfer slots change hands between host and kernels"""
+    tree = T.uniform_tree(5)
+    g = rt.RadGPU(_params(1, 5), rt.FP64)
+    g.setup(_params(1, 5), tree, _fields(1, tree))
+    g.pinned_stencil(3, 8)
+    assert m.model_host_blocks() >= 4  # the record, two slots, the batch
+    assert m.model_common_flags() & hm.COHERENT
