@@ -2157,18 +2157,20 @@ extern "C" int emma_rt_destroy_pinned_stencil(void* stencil) {
   return EMMA_RT_OK;
 }
 
-// the device address of page-locked host memory [h, h + bytes), null where it
-// is not (all) page-locked; coherent: allocated with hipHostMallocCoherent, so
-// that the host reads a finished kernel's stores without a synchronisation
+// the device address of page-locked host memory [h, h + bytes), null where the
+// range is not within one allocation of it (locked ends say nothing about what
+// lies between); coherent: allocated with hipHostMallocCoherent, so that the
+// host reads a finished kernel's stores without a synchronisation
 static void* mapped_host(char* h, size_t bytes, bool* coherent) {
-  hipPointerAttribute_t a, b;
-  if (hipPointerGetAttributes(&a, h) != hipSuccess || hipPointerGetAttributes(&b, h + bytes - 1) != hipSuccess) {
+  hipPointerAttribute_t a;
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  if (hipPointerGetAttributes(&a, h) != hipSuccess || a.type != hipMemoryTypeHost || a.devicePointer == nullptr ||
+      hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)a.devicePointer) != hipSuccess) {
     (void)hipGetLastError();  // ordinary memory
     return nullptr;
   }
-  if (a.type != hipMemoryTypeHost || b.type != hipMemoryTypeHost || a.devicePointer == nullptr ||
-      (char*)b.devicePointer - (char*)a.devicePointer != (ptrdiff_t)(bytes - 1))
-    return nullptr;
+  if ((char*)a.devicePointer + bytes > (char*)base + size) return nullptr;
   unsigned flags = 0;
   if (hipHostGetFlags(&flags, h) != hipSuccess) {
     (void)hipGetLastError();

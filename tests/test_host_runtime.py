@@ -72,3 +72,25 @@ def test_own_page_locked_memory_is_coherent(m, rt):
     g.pinned_stencil(3, 8)
     assert m.model_host_blocks() >= 4  # the record, two slots, the batch
     assert m.model_common_flags() & hm.COHERENT
+
+
+@modelled
+def test_batch_between_locked_ranges_is_copied(m, rt):
+    """both ends page-locked, the middle not"""
+    g, advance = _stencil_context(rt, 5)
+    raw, st = _batch(5)
+    at = st.ctypes.data
+    for a in (at, at + st.nbytes - 4096):
+        m.model_lock(a, 4096, hm.COHERENT)
+    advance(st)
+    assert not any("stencil_direct_kernel" in k for k in m.launched())
+    assert any("stencil_kernel" in k for k in m.launched())
+
+
+@modelled
+def test_misaligned_batch_is_copied(m, rt):
+    g, advance = _stencil_context(rt, 5)
+    raw, st = _batch(5, align=8)
+    m.model_lock(raw.ctypes.data, raw.nbytes, hm.COHERENT)
+    advance(st)
+    assert any("stencil_kernel" in k for k in m.launched())
