@@ -6,8 +6,12 @@
 // both operands and patches the special cases (11 instructions); the operands
 // here are far from the range's ends, so the same two Newton steps and one
 // residual correction without the scaling give the same correctly rounded
-// quotient, and quotients by one divisor share its reciprocal.  A zero or
-// infinite divisor gives NaN (the callers' states hold neither).  Powers: the
+// quotient (operands and quotient within 2^-900 .. 2^900), and quotients by one
+// divisor share its reciprocal.  div64 keeps the hardware's patch of the special
+// cases: zeros, infinities and NaN divide as in IEEE arithmetic.  quot64 leaves
+// that out, for operands known to be ordinary or with a check of the result: a
+// zero, infinite or denormal divisor, or an infinite numerator, gives NaN.
+// Powers: the
 // rate fits raise two numbers to six powers; pow() takes an extended-precision
 // logarithm and a full range check each time.  Here a base's logarithm is taken once, as
 // an unevaluated sum of two doubles good to about 2^-59, and products of
@@ -26,9 +30,13 @@ __device__ __forceinline__ double rcp64(double b) {
   return r;
 }
 // a/b correctly rounded, r = 1/b to about one ulp
-__device__ __forceinline__ double div64(double a, double b, double r) {
+__device__ __forceinline__ double quot64(double a, double b, double r) {
   const double q = a * r;
   return fma(fma(-q, b, a), r, q);
+}
+__device__ __forceinline__ double quot64(double a, double b) { return quot64(a, b, rcp64(b)); }
+__device__ __forceinline__ double div64(double a, double b, double r) {
+  return __builtin_amdgcn_div_fixup(quot64(a, b, r), b, a);
 }
 __device__ __forceinline__ double div64(double a, double b) { return div64(a, b, rcp64(b)); }
 

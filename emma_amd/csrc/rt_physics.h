@@ -83,20 +83,8 @@ __device__ __forceinline__ Closure<R> closure(R fx, R fy, R fz, R ee, R c) {
   q.n[1] = R(0);
   q.n[2] = R(0);
   R arg, chi;
-  if constexpr (sizeof(R) == 8) {  // the three n_i share |F|'s reciprocal
-    if (ee > R(0)) {
-      ff = sqrt(fx * fx + fy * fy + fz * fz);
-      if (ff > R(0)) {
-        const R r = rcp64(ff);
-        q.n[0] = div64(fx, ff, r);
-        q.n[1] = div64(fy, ff, r);
-        q.n[2] = div64(fz, ff, r);
-      }
-      ff = div64(ff, c * ee);
-    }
-    arg = fmax(R(4) - R(3) * ff * ff, R(0));
-    chi = div64(R(3) + R(4) * ff * ff, R(5) + R(2) * sqrt(arg));
-  } else {
+  auto plain = [&] {
+    q.n[0] = q.n[1] = q.n[2] = ff = R(0);
     if (ee > R(0)) {
       ff = sqrt(fx * fx + fy * fy + fz * fz);
       if (ff > R(0)) {
@@ -108,6 +96,23 @@ __device__ __forceinline__ Closure<R> closure(R fx, R fy, R fz, R ee, R c) {
     }
     arg = fmax(R(4) - R(3) * ff * ff, R(0));
     chi = (R(3) + R(4) * ff * ff) / (R(5) + R(2) * sqrt(arg));
+  };
+  if constexpr (sizeof(R) == 8) {  // the three n_i share |F|'s reciprocal
+    if (ee > R(0)) {
+      ff = sqrt(fx * fx + fy * fy + fz * fz);
+      if (ff > R(0)) {
+        const R r = rcp64(ff);
+        q.n[0] = quot64(fx, ff, r);
+        q.n[1] = quot64(fy, ff, r);
+        q.n[2] = quot64(fz, ff, r);
+      }
+      ff = quot64(ff, c * ee);
+    }
+    arg = fmax(R(4) - R(3) * ff * ff, R(0));
+    chi = quot64(R(3) + R(4) * ff * ff, R(5) + R(2) * sqrt(arg));
+    if (isnan(chi)) plain();  // a density next to the smallest double, an infinite flux: not for quot64
+  } else {
+    plain();
   }
   q.diag = (R(1) - chi) / R(2) * c2e;
   q.arg = (R(3) * chi - R(1)) / R(2) * c2e;
@@ -159,19 +164,21 @@ struct Rates {
 };
 
 __device__ __forceinline__ Rates rates_of(double temp) {
+  // (a temperature of 0, infinity or NaN gives rates that no sub-step accepts,
+  // with or without the special cases of the divisions)
   Rates r;
   const double sT = sqrt(temp);
-  const double sT5 = sqrt(div64(temp, 1e5, 1e-5));
+  const double sT5 = sqrt(quot64(temp, 1e5, 1e-5));
   const double rT = rcp64(temp);
   const double g = 1. + sT5, rg = rcp64(g);
-  r.A1 = div64(exp64(div64(-157809.1e0, temp, rT)) * 2.54e-21 * sT, g, rg);
-  r.A3 = div64(exp64(div64(-118348e0, temp, rT)) * 7.5e-19, g, rg);
+  r.A1 = quot64(exp64(quot64(-157809.1e0, temp, rT)) * 2.54e-21 * sT, g, rg);
+  r.A3 = quot64(exp64(quot64(-118348e0, temp, rT)) * 7.5e-19, g, rg);
   r.A4 = 1.42e-27 * 1.5e0 * sT;
-  const double b = div64(1.17e-10 * sT, g, rg) * exp64(-div64(157809e0, temp, rT));
+  const double b = quot64(1.17e-10 * sT, g, rg) * exp64(-quot64(157809e0, temp, rT));
   r.beta = b * 1e-6 * 1.;
   // lam^1.970 / (1 + (lam/2.250)^0.376)^3.720 and
   // lam^1.5 / (1 + (lam/2.740)^0.407)^2.242, lam = 2 x 157807 / T
-  const Dd L = log_dd(div64(2e0 * 157807e0, temp, rT));
+  const Dd L = log_dd(quot64(2e0 * 157807e0, temp, rT));
   const Dd ln225 = {0x1.9f323ecbf984cp-1, -0x1.a92e513217f5cp-58}, ln274 = {0x1.020987bfdcb15p+0, 0x1.953b86e09d8b0p-55};
   const Dd W6 = log_dd(1. + exp_of(dd_scale(0.376e0, dd_sub(L, ln225))));
   r.A6 = 3.435e-30 * temp * exp_of(dd_sub(dd_scale(1.970e0, L), dd_scale(3.720e0, W6)));

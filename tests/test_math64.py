@@ -1,0 +1,165 @@
+"""The FP64 path's divisions, logarithm and exponential (rt_math64.h), its rate
+fits and its closure (rt_physics.h), compiled for the host, against IEEE
+division and 50-digit arithmetic.  The hardware's reciprocal estimate is
+modelled with its largest error either way."""
+import ctypes
+import math
+import os
+import subprocess
+from decimal import Decimal, getcontext
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(os.path.dirname(HERE), "emma_amd", "csrc")
+EPS = 2.0**-53  # half a unit in the last place of 1
+INF, NAN, TINY = np.inf, np.nan, 5e-324
+
+getcontext().prec = 50
+
+
+@pytest.fixture(scope="module", params=[0.0, 2.0**-23, -(2.0**-23)], ids=["exact", "high", "low"])
+def lib(request, tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("math64") / "libmath64.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-ffp-contract=off", "-fPIC", "-shared", "-w",
+                    "-I", os.path.join(HERE, "host_device"), "-I", CSRC, os.path.join(HERE, "math64_host.cpp"), "-o", out],
+                   check=True)
+    L = ctypes.CDLL(out)
+    L.set_rcp_error.argtypes = [ctypes.c_double]
+    L.set_rcp_error(request.param)
+    return L
+
+
+def _p(a):
+    return a.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
+
+
+def _div(lib, a, b):
+    a, b = (np.ascontiguousarray(x, dtype=np.float64) for x in np.broadcast_arrays(a, b))
+    q = np.empty(a.size)
+    lib.div_all(a.size, _p(a), _p(b), _p(q))
+    return q
+
+
+def _same(x, y):
+    return np.array_equal(x, y, equal_nan=True) and np.array_equal(np.signbit(x[~np.isnan(x)]), np.signbit(y[~np.isnan(y)]))
+
+
+def test_division_is_correctly_rounded(lib):
+    """operands of any sign within 2^-450 .. 2^450"""
+    rng = np.random.default_rng(1)
+    n = 400000
+    a, b = (np.ldexp(rng.uniform(1, 2, n) * rng.choice([-1.0, 1.0], n), rng.integers(-450, 450, n)) for _ in range(2))
+    near = np.nextafter(b, rng.choice([0.0, INF], n))  # quotients next to 1, and exact ones
+    for x, y in ((a, b), (b, near), (b * 3, b), (b, b)):
+        assert _same(_div(lib, x, y), x / y)
+
+
+def test_division_of_special_values(lib):
+    """zeros, infinities and NaN as IEEE division gives them"""
+    v = np.array([0.0, -0.0, 1.0, -2.5, 1e-290, 1e290, INF, -INF, NAN])
+    a, b = (x.ravel() for x in np.meshgrid(v, v))
+    keep = ~((np.abs(a) == 1e290) & (np.abs(b) == 1e-290))  # an overflowing quotient is not promised
+    a, b = a[keep], b[keep]
+    with np.errstate(all="ignore"):
+        want = a / b
+    got = _div(lib, a, b)
+    assert np.array_equal(got, want, equal_nan=True), [(x, y) for x, y, p, q in zip(a, b, got, want) if not p == q][:5]
+
+
+def _closure_plain(u, c):
+    """the reference's operations (rad_utils.c:448-475), IEEE division throughout"""
+    e, f = u[:, 0], u[:, 1:]
+    with np.errstate(all="ignore"):
+        norm = np.sqrt(f[:, 0] * f[:, 0] + f[:, 1] * f[:, 1] + f[:, 2] * f[:, 2])
+        lit = e > 0
+        n = np.where((lit & (norm > 0))[:, None], f / norm[:, None], 0.0)
+        ff = np.where(lit, norm / (c * e), 0.0)
+        arg = np.fmax(4.0 - 3.0 * ff * ff, 0.0)
+        chi = (3.0 + 4.0 * ff * ff) / (5.0 + 2.0 * np.sqrt(arg))
+        c2e = e * c * c
+        return np.column_stack([(1.0 - chi) / 2.0 * c2e, (3.0 * chi - 1.0) / 2.0 * c2e, n])
+
+
+def test_closure_of_any_state(lib):
+    """ordinary states, and densities down to the smallest, zero, infinite ones"""
+    rng = np.random.default_rng(2)
+    n = 20000
+    e = 10.0 ** rng.uniform(-60, 10, n)
+    F = rng.normal(size=(n, 3))
+    F *= (rng.uniform(0, 1.2, n) * 3e-3 * e / np.linalg.norm(F, axis=1))[:, None]
+    u = np.column_stack([e, F])
+    odd = np.array([0.0, TINY, 1e-320, 3e-310, 1e-308, 1e-300, 1.0, 1e300, INF, NAN, -1.0])
+    flux = np.array([0.0, TINY, 1e-310, -1e-162, 1e-3, -1e160, INF, NAN])
+    E, X, Y = (x.ravel() for x in np.meshgrid(odd, flux, flux))
+    u = np.concatenate([u, np.column_stack([E, X, Y, np.zeros_like(E)])])
+    for c in (1e-3, 1.0, 3.7e4):
+        out = np.empty((len(u), 5))
+        lib.closure_all(len(u), _p(np.ascontiguousarray(u)), ctypes.c_double(c), _p(out))
+        want = _closure_plain(u, c)
+        bad = ~((out == want) | (np.isnan(out) & np.isnan(want))).all(axis=1)
+        assert not bad.any(), (c, u[bad][:3], out[bad][:3], want[bad][:3])
+
+
+def _ln(x):
+    return Decimal(float(x)).ln()
+
+
+def test_log(lib):
+    """a sum of two doubles within 2^-57 of ln x: the polynomial's last roundings are 4 x 2^-53 of
+    a term of 1 % of the sum"""
+    rng = np.random.default_rng(3)
+    x = np.concatenate([10.0 ** rng.uniform(-300, 300, 1500), 1 + rng.uniform(-0.3, 0.5, 1500),
+                        1 + 2.0 ** rng.uniform(-52, -1, 300), np.ldexp([0.5, math.sqrt(0.5), 0.75, 1.0, math.sqrt(2)], 7)])
+    h, l = np.empty(x.size), np.empty(x.size)
+    lib.log_all(x.size, _p(x), _p(h), _p(l))
+    for v, a, b in zip(x, h, l):
+        want = _ln(v)
+        assert abs(Decimal(float(a)) + Decimal(float(b)) - want) <= abs(want) * Decimal(2.0**-57), v
+
+
+def test_exp(lib):
+    """within one unit in the last place where the result is normal; 0 below"""
+    rng = np.random.default_rng(4)
+    x = np.concatenate([rng.uniform(-708, 700, 3000), rng.uniform(-1, 1, 500), [0.0, -708.0, 700.0]])
+    y = np.empty(x.size)
+    lib.exp_all(x.size, _p(x), _p(y))
+    for v, a in zip(x, y):
+        want = Decimal(float(v)).exp()
+        assert abs(Decimal(float(a)) - want) <= want * Decimal(2 * EPS), v
+    x = np.array([-750.0, -1e4, -1e300, -INF])
+    y = np.empty(x.size)
+    lib.exp_all(x.size, _p(x), _p(y))
+    assert (y == 0).all()
+
+
+def test_rates(lib):
+    """the fits of chem_utils.c:37-187 over 1 K .. 1e8 K.  Sums and products of at most ten rounded
+    factors; an exponential carries its argument's rounding too."""
+    rng = np.random.default_rng(5)
+    T = 10.0 ** np.concatenate([rng.uniform(0, 8, 500), [0, 4, 8]])
+    out = np.empty((T.size, 6))
+    lib.rates_all(T.size, _p(T), _p(out))
+    D = Decimal
+
+    def power(x, y):
+        return (x.ln() * D(y)).exp()
+
+    for t, got in zip(T, out):
+        t = D(float(t))
+        st, s5 = t.sqrt(), (t / 100000).sqrt()
+        lam = 2 * D(157807) / t
+        want = [
+            ((D(-157809.1) / t).exp() * D(2.54e-21) * st / (1 + s5), 157809.1),
+            ((D(-118348) / t).exp() * D(7.5e-19) / (1 + s5), 118348.0),
+            (D(1.42e-27) * D(1.5) * st, 0.0),
+            (D(3.435e-30) * t * power(lam, 1.970) / power(1 + power(lam / D(2.250), 0.376), 3.720), 0.0),
+            (D(2.753e-14) * power(lam, 1.5) / power(1 + power(lam / D(2.740), 0.407), 2.242) * D(1e-6), 0.0),
+            (D(1.17e-10) * st / (1 + s5) * (D(-157809) / t).exp() * D(1e-6), 157809.0)]
+        for (w, a), g in zip(want, got):
+            arg = a / float(t)
+            # ten factors; the fits' powers carry up to 2.3 (1.970 x, 3.720 x ...) of a rounding of their bases;
+            # below the smallest normal number, a rounding is half of 2^-1074
+            bound = w * D((14 + 2 * arg) * EPS) + D(4 * 2.0**-1074)
+            assert abs(D(float(g)) - w) <= bound, (float(t), float(g), float(w))
