@@ -20,7 +20,7 @@ COHERENT, NONCOHERENT = 0x40000000, 0x80000000  # hipHostMalloc's flags
 @pytest.mark.parametrize("groups,real", [(1, 8), (3, 4)])
 def test_same_in_any_memory(gpu_lib, flags, offset, groups, real):
     n = 67
-    params, st = batch(groups, real, n, 7)
+    params, st = batch(groups, real, n, 100 * groups + n)
     p = ctypes.c_void_p()
     size = st.nbytes + 64
     # the runtime the library is linked to
@@ -33,8 +33,10 @@ def test_same_in_any_memory(gpu_lib, flags, offset, groups, real):
     rng = np.random.default_rng(8)
     for call in range(4):
         here = st.copy()
-        here["oct"]["rfield"]["e"] *= rng.uniform(0.5, 1.0)
-        here["New"]["rfieldnew"]["src"] *= rng.uniform(0.5, 1.0)
+        scale = rng.uniform(0.5, 1.0)
+        for state in (here["oct"]["rfield"], here["New"]["rfieldnew"]):
+            for k in ("e", "fx", "fy", "fz", "src"):
+                state[k] *= scale
         raw[:] = 5
         raw[offset : offset + st.nbytes] = here.view(np.uint8)  # padding bytes too
         g.advance_stencil(here, n, 0.5**4, dt)
