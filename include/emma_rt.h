@@ -150,7 +150,7 @@ int emma_rt_alloc_pinned(size_t bytes, void **out);
    reference's RGRID layout.  Page-locked records aligned to 16 bytes (from
    emma_rt_create_pinned_stencil) are read and written in place by the kernel,
    and only the parts it needs cross the bus; records in ordinary memory go to
-   the device buffer and back whole, at less than a third of the rate.
+   the device buffer whole and their results come back, at a sixth of the rate.
    Page-locked records of another allocation need not be coherent: the call
    then waits for the stream before it returns.  In EMMA_RT_COARSERAD mode
    (emma_rt_set_mode) the batch follows the COARSERAD build: the sweeps and

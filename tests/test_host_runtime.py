@@ -94,3 +94,28 @@ def test_misaligned_batch_is_copied(m, rt):
     m.model_lock(raw.ctypes.data, raw.nbytes, hm.COHERENT)
     advance(st)
     assert any("stencil_kernel" in k for k in m.launched())
+
+
+@modelled
+def test_ordinary_batch_keeps_what_others_write(m, rt):
+    """only rfieldnew and rflux of the records are the call's to write"""
+    for n in (1, 700):  # one copy back, several
+        g, advance = _stencil_context(rt, n)
+        raw, st = _batch(n)
+        ours = np.zeros(st.nbytes, bool)
+        lay = rgrid.layout(1, 8)
+        new, cell, at, end = lay[21], lay[12], lay[15], lay[12]  # New, a cell of it, its rfieldnew up to its end
+        for c in range(8):
+            ours.reshape(n, -1)[:, new + c * cell + at : new + c * cell + end] = True
+        raw8 = st.view(np.uint8)
+        old = raw8.copy()
+
+        def meanwhile():
+            raw8[~ours] = 77
+
+        f = ctypes.CFUNCTYPE(None)(meanwhile)
+        m.model_during(b"stencil_kernel", f)
+        advance(st)
+        m.model_during(b"none", None)
+        assert (raw8[~ours] == 77).all(), n
+        assert np.array_equal(raw8[ours], old[ours]), n  # the model runs no kernel
