@@ -974,10 +974,11 @@ static int join_free(emma_rt_ctx* c, int k, double dt, double aexp) {
 
 // the side streams of the levels that may fork, made before a capture
 static int ensure_side_streams(emma_rt_ctx* c) {
+  const DeviceScope on(c->device);
   for (auto& L : c->lev) {
     if (L.tiles == nullptr || L.side != nullptr) continue;
-    HIPCHK(hipEventCreateWithFlags(&L.forked, hipEventDisableTiming));
-    HIPCHK(hipEventCreateWithFlags(&L.joined, hipEventDisableTiming));
+    if (L.forked == nullptr) HIPCHK(hipEventCreateWithFlags(&L.forked, hipEventDisableTiming));
+    if (L.joined == nullptr) HIPCHK(hipEventCreateWithFlags(&L.joined, hipEventDisableTiming));
     HIPCHK(hipStreamCreate(&L.side));
   }
   return EMMA_RT_OK;

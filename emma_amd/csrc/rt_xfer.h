@@ -8,6 +8,25 @@
 
 namespace emma {
 
+// A device made current for a scope.  Streams, events and allocations belong to
+// the device that is current when they are made, and a context's calls may come
+// from a thread that has another one.
+class DeviceScope {
+ public:
+  explicit DeviceScope(int device) {
+    int now = device;
+    if (hipGetDevice(&now) == hipSuccess && now != device && hipSetDevice(device) == hipSuccess) before_ = now;
+  }
+  ~DeviceScope() {
+    if (before_ >= 0) (void)hipSetDevice(before_);
+  }
+  DeviceScope(const DeviceScope&) = delete;
+  DeviceScope& operator=(const DeviceScope&) = delete;
+
+ private:
+  int before_ = -1;
+};
+
 // one array: n values, device storage float (f32) or double.  floor > 0 (to
 // the device, f32): a value at or above it that rounds below it becomes
 // floor_up, the smallest float at or above it.
@@ -22,7 +41,7 @@ struct XferPart {
 constexpr int kMaxXferParts = 24;
 
 // Both wait for the work queued on the stream before and return with the copy
-// done.  Callable from several threads; the staging memory is shared by all
+// done.  Callable from several threads, whatever their current device; the staging memory is shared by all
 // callers, bounded, and released with the last xfer_release().
 hipError_t xfer_to_host(int device, hipStream_t s, const XferPart* parts, int np);
 hipError_t xfer_to_device(int device, hipStream_t s, const XferPart* parts, int np);

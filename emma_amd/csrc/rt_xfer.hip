@@ -282,6 +282,7 @@ hipError_t chunked(int device, hipStream_t s, const XferPart* parts, int np, siz
 
 template <bool ToHost>
 hipError_t transfer(int device, hipStream_t s, const XferPart* in, int nin) {
+  const DeviceScope on(device);
   XferPart parts[kMaxXferParts];
   int np = 0;
   size_t total = 0;

@@ -22,6 +22,11 @@ def _fields(G, tree, seed=1):
     return {l: synth.random_fields(p, np.ones(tree.level(l).ncell), rng) for l in range(tree.lmin, tree.lmax + 1)}
 
 
+def _tree(lmin, counts, seed=3):
+    rng = np.random.default_rng(seed)
+    return T.amr_tree(lmin, counts, synth.lognormal_sampler(synth.gaussian_field(8, rng), 1.0), rng)
+
+
 def _batch(n, G=1, align=16):
     """n records in ordinary memory, their first byte at a multiple of `align` but not of twice that"""
     size = rgrid.rgrid_dtype(G, 8).itemsize * n
@@ -119,3 +124,34 @@ def test_ordinary_batch_keeps_what_others_write(m, rt):
         m.model_during(b"none", None)
         assert (raw8[~ours] == 77).all(), n
         assert np.array_equal(raw8[ours], old[ours]), n  # the model runs no kernel
+
+
+# ---------------------------------------------------------------- devices
+@modelled
+def test_transfers_from_a_thread_on_another_device(m, rt):
+    m.model_device(1)
+    tree = T.uniform_tree(5)
+    F = _fields(1, tree)
+    g = rt.RadGPU(_params(1, 5), rt.FP64)
+    g.setup(_params(1, 5), tree, F)
+    H = synth.hydro_like(F[5], np.random.default_rng(2))
+    m.model_device(0)
+    g.set(5, 0, F[5])
+    B = g.get(5)
+    assert np.array_equal(B.e, F[5].e) and np.array_equal(B.nh, F[5].nh)
+    g.set_hydro(5, H)
+    assert np.array_equal(g.get_hydro(5)[0], H.p)
+    assert m.model_current() == 0
+
+
+@modelled
+def test_coarse_step_from_a_thread_on_another_device(m, rt):
+    m.model_device(1)
+    tree = _tree(7, [4000, 1500])
+    g = rt.RadGPU(_params(3, 7), rt.FP64)
+    g.setup(_params(3, 7), tree, {})
+    m.model_device(0)
+    m.model_forget()
+    g.coarse_step(1.0, 1)
+    assert sum("transport_kernel" in k for k in m.launched()) == 8  # 1 + 2 + 4 level steps, the first in two parts
+    assert m.model_current() == 0
