@@ -1317,9 +1317,8 @@ static hipError_t fill_cells(emma_rt_ctx* c, int k, double aexp) {
   return launch_fill_cells<float>(c, k, aexp);
 }
 
-// RadSolver's injection into the hydro state after the level's final update
-// RadSolver's injection of level k; wait: with the next level step's FillRad
-// (end_hydro launches the last one)
+// RadSolver's injection into the hydro state after level k's final update;
+// wait: with the next level step's FillRad (end_hydro launches the last one)
 static hipError_t to_hydro(emma_rt_ctx* c, int k, bool wait = false) {
   DevLevel& L = c->lev[k];
   if (!c->hydro || L.noct == 0) return hipSuccess;
@@ -1759,8 +1758,13 @@ extern "C" int emma_rt_coarse_step(emma_rt_ctx* c, double aexp, int ncoarse) {
   const bool eager = c->timing == 1;  // launches with their own events
   st = begin_call(c);
   if (st) return st;
+  // however the call ends, no injection waits for another call's FillRad: its
+  // arguments are those of this call's tree and buffers
+  struct NoWait {
+    emma_rt_ctx* c;
+    ~NoWait() { c->hydro_waits = false; }
+  } no_wait{c};
   if (eager && c->sched == EMMA_RT_SCHED_GRAPH) {  // eager launches with per-kernel events
-    c->hydro_waits = false;
     for (int i = 0; i < ncoarse; i++) {
       st = recurse(c, 0, aexp);
       if (st) return st;
@@ -1808,7 +1812,6 @@ extern "C" int emma_rt_coarse_step(emma_rt_ctx* c, double aexp, int ncoarse) {
       const int timing = c->timing;
       c->timing = 0;  // no event records inside the graph
       c->capturing = true;
-      c->hydro_waits = false;
       for (int i = 0; i < ncoarse && rs == EMMA_RT_OK; i++) rs = recurse(c, 0, aexp);
       if (rs == EMMA_RT_OK && end_hydro(c) != hipSuccess) rs = EMMA_RT_ERR_HIP;
       c->capturing = false;

@@ -155,3 +155,30 @@ def test_coarse_step_from_a_thread_on_another_device(m, rt):
     g.coarse_step(1.0, 1)
     assert sum("transport_kernel" in k for k in m.launched()) == 8  # 1 + 2 + 4 level steps, the first in two parts
     assert m.model_current() == 0
+
+
+# ---------------------------------------------------------------- failed calls
+@modelled
+def test_pending_injection_ends_with_a_failed_call(m, rt):
+    tree = _tree(3, [20, 30])
+    F = _fields(1, tree)
+    rng = np.random.default_rng(4)
+    for timing in (rt.TIMING_LAUNCH, rt.TIMING_OFF):
+        for n in range(8):
+            g = rt.RadGPU(_params(1, 3), rt.FP64)
+            g.setup(_params(1, 3), tree, F, mode=rt.COARSERAD)
+            for l in F:
+                g.set_hydro(l, synth.hydro_like(F[l], rng))
+            g.set_coupling(True)
+            g.enable_timing(timing)
+            m.model_set(hm.FAIL_LAUNCH, n)
+            try:
+                g.coarse_step(1.0, 1)
+                assert False, "no launch failed"
+            except rt.EmmaRTError:
+                pass
+            m.model_forget()
+            g.fillrad(3)
+            assert not any("couple_kernel" in k for k in m.launched()), (timing, n)
+            g.coarse_step(1.0, 1)
+            g.close()
