@@ -984,6 +984,18 @@ static int ensure_side_streams(emma_rt_ctx* c) {
   return EMMA_RT_OK;
 }
 
+// After a capture that failed: a side stream it did not join is of no more use
+static void drop_side_streams(emma_rt_ctx* c) {
+  for (auto& L : c->lev) {
+    if (L.side == nullptr) continue;
+    (void)hipStreamDestroy(L.side);
+    (void)hipEventDestroy(L.forked);
+    (void)hipEventDestroy(L.joined);
+    L.side = nullptr;
+    L.forked = L.joined = nullptr;
+  }
+}
+
 static hipEvent_t next_event(emma_rt_ctx* c) {
   if (c->ev_used == c->ev.size()) {
     hipEvent_t e;
@@ -1823,6 +1835,7 @@ extern "C" int emma_rt_coarse_step(emma_rt_ctx* c, double aexp, int ncoarse) {
       // starts from (the launch below advances it), also on the error paths
       for (size_t k = 0; k < c->lev.size(); k++) c->lev[k].cur = key.parity[k];
       if (rs || ce != hipSuccess) {
+        drop_side_streams(c);
         if (ce == hipSuccess) (void)hipGraphDestroy(g);
         if (rs) return rs;
         HIPCHK(ce);

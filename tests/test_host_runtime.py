@@ -182,3 +182,20 @@ def test_pending_injection_ends_with_a_failed_call(m, rt):
             assert not any("couple_kernel" in k for k in m.launched()), (timing, n)
             g.coarse_step(1.0, 1)
             g.close()
+
+
+@modelled
+def test_forked_level_after_a_failed_capture(m, rt):
+    """a side stream left in a failed capture does not fail later calls"""
+    tree = _tree(7, [4000, 1500])
+    g = rt.RadGPU(_params(3, 7), rt.FP64)
+    g.setup(_params(3, 7), tree, {})
+    for n in range(14):
+        m.model_set(hm.FAIL_LAUNCH, n)
+        try:
+            g.coarse_step(1.0, 1)
+            assert False, "no launch failed"
+        except rt.EmmaRTError:
+            pass
+        m.model_set(hm.FAIL_LAUNCH, -1)
+    g.coarse_step(1.0, 1)
