@@ -81,7 +81,7 @@ struct DevLevel {
   // a finer oct behind a face), then the others
   int* tiles = nullptr;
   int nfree = 0, ntile = 0;
-  int fork = 0;  // 1: the free tiles may step beside the finer levels, 2: leaving room for their work-groups
+  int fork = 0;  // 1: the free tiles may step beside the finer levels, 2: leaving room for their work-groups (fork_kind)
   int* defer = nullptr;  // fork: the level's own straggler list (its free tiles append beside other levels' lists)
   int fork_slot = 0;     // and the list-length word its two launches share
   hipStream_t side = nullptr;  // where the free tiles' step runs beside the finer levels'
@@ -534,16 +534,28 @@ static int morton_cube(int noct, const int* nei) {
 }
 
 // Whether level k's free tiles step beside the finer levels' launches of one
-// of its steps (see fork_free): at least four work-groups per CU of them, and
-// finer launches that take at least a quarter as long.  A launch of few tiles
-// takes as long as about 800 (12 us).  Where the finer launches take longer
-// than the free tiles (2), those leave room for them.  On the five-level tree
-// both large levels fork: coarse step 0.575 ms -> 0.555 (1), 0.541 (2); with
-// the largest alone 0.550.
-constexpr int kForkTiles = 1024, kLaunchTiles = 800;
-static int fork_kind(const std::vector<DevLevel>& lev, int k) {
+// of its steps (see fork_free).  A fork costs a launch (two in the families that
+// step in two kernels) and slows the small launches it runs beside, so its free
+// tiles have to be worth about 70 us of the whole chip.  In units of the mixed
+// one-group tile (a tile's time, roughly) at least kForkWork of them: measured
+// steady coarse steps, one after the other -> forked, by units,
+//   below: 6.2e3 mixed G=4 575 -> 588 us, 7.8e3 mixed G=1 114 -> 121 and G=2
+//     215 -> 229, 8.7e3 FP64 G=1 442 -> 457, 1.0e4 mixed G=9 310 -> 323, 1.24e4
+//     FP64 G=2 642 -> 665, 1.39e4 FP64 G=3 270 -> 277;
+//   above: 1.43e4 mixed G=3 380 -> 382 (the first one, with long chemistry
+//     chains, 874 -> 793), 1.56e4 173 -> 169, 1.6e4 155 -> 147; 1.86e4 FP64 G=3
+//     896 -> 888; 2.1e4 FP64 G=2 1197 -> 1125; 3.1e4 FP64 G=1 227 -> 202, mixed
+//     G=4 312 -> 306; 6.3e4 mixed G=1 643 -> 635; 6.4e4 mixed G=9 1269 -> 1225.
+// And the finer launches have to take at least a quarter as long as the free
+// tiles.  A launch of few tiles takes as long as about 800 (12 us).  Where they
+// take longer than the free tiles (2), the three-group mixed tiles, whose LDS
+// allows it, leave room for them (five-level tree: 543 us, 534 with 1, 527 with
+// 2; with level 8's 2,170 free tiles forked too 557).
+constexpr int kForkWork = 14000, kLaunchTiles = 800;
+static int tile_work(int ng, bool fp64) { return fp64 ? 4 * ng : ng == 3 ? 2 : ng < 3 ? 1 : ng; }
+static int fork_kind(const std::vector<DevLevel>& lev, int k, int ng, bool fp64) {
   const DevLevel& L = lev[k];
-  if (L.nfree < kForkTiles) return 0;
+  if ((long long)L.nfree * tile_work(ng, fp64) < kForkWork) return 0;
   long long finer = 0;
   for (size_t j = k + 1; j < lev.size() && lev[j].noct > 0; j++)
     finer += (long long)std::max(kLaunchTiles, (lev[j].ncell + kTileCells - 1) / kTileCells) << std::min<size_t>(j - k, 20);
@@ -659,7 +671,7 @@ extern "C" int emma_rt_tree_create(emma_rt_ctx* c, int lmin, int lmax, const int
       }
       L.nfree = (int)tiles.size();
       L.ntile = L.nfree + (int)touched.size();
-      L.fork = fork_kind(c->lev, k);
+      L.fork = fork_kind(c->lev, k, G, c->rbytes == 8);
       if (L.fork) {
         tiles.insert(tiles.end(), touched.begin(), touched.end());
         HIPCHK(dalloc(&L.tiles, tiles.size()));
