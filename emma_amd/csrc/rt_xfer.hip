@@ -33,47 +33,90 @@ namespace {
 // 64^3 cells with nine groups (55 MB) back then 1.7 instead of 1.45 ms and
 // with one FP64 group (19 MB) 1.5 instead of 1.0 (fewer chunks than threads):
 // 2 MiB from 128 MB on.  Twelve threads gain nothing over eight.
-constexpr size_t kSlotBytes = 2u << 20;
 constexpr size_t kPackBytes = 1u << 20;  // up to here one gathering kernel
-constexpr size_t kChunkBytes = 1u << 20, kLargeTotal = 128u << 20;
+constexpr size_t kChunkBytes = 1u << 20, kLargeChunkBytes = 2u << 20, kLargeTotal = 128u << 20;
 constexpr int kMaxThreads = 8;
 constexpr size_t kBytesPerThread = 4u << 20;  // host bytes that pay for starting a thread (0.02 to 2 ms)
-constexpr size_t kKeepSlots = 2 * kMaxThreads;
+constexpr size_t kKeepBytes = 2 * kMaxThreads * kLargeChunkBytes;
+constexpr size_t kKeepBlocks = 16;
 
+// The page-locked memory of a transfer: one block, two slots of a chunk for each
+// thread.  Freeing page-locked memory takes 0.28 ms a block whatever its size,
+// and allocating 32 MiB 2.2 ms in one block, 6 in sixteen: closing the last
+// context of a program after 64^3 cells and two finer levels, three FP64 groups,
+// takes 5.8 ms, 9.7 with sixteen slots of their own, 4.8 with none.
+struct FreeBlock {
+  char* p;
+  size_t bytes;
+};
 std::mutex g_mu;
-std::vector<void*> g_free;  // slots nobody uses, at most kKeepSlots
+std::vector<FreeBlock> g_free;  // blocks nobody uses, kKeepBytes at most
+size_t g_kept = 0;
 int g_users = 0;
 
-void* take_slot() {
-  {
-    std::lock_guard<std::mutex> lock(g_mu);
-    if (!g_free.empty()) {
-      void* p = g_free.back();
-      g_free.pop_back();
-      return p;
+class Block {
+ public:
+  // n units of `unit` bytes, or the half, the quarter ... if there is no more
+  Block(size_t n, size_t unit) {
+    for (; n > 0 && p == nullptr; n /= 2) {
+      take(n * unit);
+      count = p != nullptr ? n : 0;
     }
   }
-  // coherent: a slot goes from kernel to host and back with no more than an
-  // event in between (same rates either way, 50 GB/s in and 54 out)
-  void* p = nullptr;
-  return hipHostMalloc(&p, kSlotBytes, hipHostMallocPortable | hipHostMallocCoherent) == hipSuccess ? p : nullptr;
-}
+  ~Block() {
+    if (p == nullptr) return;
+    std::vector<FreeBlock> gone;
+    {
+      std::lock_guard<std::mutex> lock(g_mu);
+      if (g_users > 0 && bytes_ <= kKeepBytes) {
+        while (!g_free.empty() && (g_kept + bytes_ > kKeepBytes || g_free.size() == kKeepBlocks)) drop(gone, 0);
+        if (g_free.size() < g_free.capacity()) {
+          g_free.push_back({p, bytes_});
+          g_kept += bytes_;
+          p = nullptr;
+        }
+      }
+    }
+    for (const FreeBlock& f : gone) (void)hipHostFree(f.p);
+    if (p != nullptr) (void)hipHostFree(p);
+  }
+  Block(const Block&) = delete;
+  Block& operator=(const Block&) = delete;
 
-void give_slot(void* p) {
-  if (p == nullptr) return;
-  {
-    std::lock_guard<std::mutex> lock(g_mu);
-    if (g_users > 0 && g_free.size() < kKeepSlots && g_free.size() < g_free.capacity()) {
-      g_free.push_back(p);
-      return;
+  char* p = nullptr;  // null: no page-locked memory to be had
+  size_t count = 0;   // units
+
+ private:
+  static void drop(std::vector<FreeBlock>& gone, size_t i) {
+    gone.push_back(g_free[i]);
+    g_kept -= g_free[i].bytes;
+    g_free.erase(g_free.begin() + i);
+  }
+  void take(size_t want) {
+    {
+      std::lock_guard<std::mutex> lock(g_mu);
+      size_t best = g_free.size();
+      for (size_t i = 0; i < g_free.size(); i++)
+        if (g_free[i].bytes >= want && (best == g_free.size() || g_free[i].bytes < g_free[best].bytes)) best = i;
+      if (best < g_free.size()) {
+        p = g_free[best].p;
+        bytes_ = g_free[best].bytes;
+        g_kept -= bytes_;
+        g_free.erase(g_free.begin() + best);
+        return;
+      }
+    }
+    // coherent: a slot goes from kernel to host and back with no more than an
+    // event in between (same rates either way, 50 GB/s in and 54 out)
+    void* fresh = nullptr;
+    if (hipHostMalloc(&fresh, want, hipHostMallocPortable | hipHostMallocCoherent) == hipSuccess) {
+      p = (char*)fresh;
+      bytes_ = want;
+    } else {
+      (void)hipGetLastError();
     }
   }
-  (void)hipHostFree(p);
-}
-
-struct Slot {
-  void* p = take_slot();
-  ~Slot() { give_slot(p); }
+  size_t bytes_ = 0;
 };
 
 // ---- one kernel for all arrays of a small level
@@ -107,7 +150,7 @@ __global__ __launch_bounds__(256) void pack_kernel(PackArgs a, double* slot) {
 
 template <bool ToHost>
 hipError_t packed(hipStream_t s, const XferPart* parts, int np, size_t total) {
-  Slot slot;
+  const Block slot(1, kPackBytes);
   if (slot.p == nullptr) return hipErrorOutOfMemory;
   PackArgs a;
   a.np = np;
@@ -180,6 +223,7 @@ void into_slot(const Chunk& c, void* slot) {
 struct Job {
   int device;
   hipStream_t s;
+  size_t chunk;  // bytes, at most
   const std::vector<Chunk>* chunks;
   std::atomic<size_t> next{0};
   std::atomic<int> err{(int)hipSuccess};
@@ -187,17 +231,13 @@ struct Job {
 
 // one thread's share: two slots, one in flight while the other is converted
 template <bool ToHost>
-void work(Job& job, bool own_thread) {
+void work(Job& job, char* slots, bool own_thread) {
   auto failed = [&](hipError_t e) {
     if (e != hipSuccess) job.err = (int)e;
     return job.err != (int)hipSuccess;
   };
-  if (own_thread && failed(hipSetDevice(job.device))) return;
-  Slot slot[2];
-  if (slot[0].p == nullptr || slot[1].p == nullptr) {
-    failed(hipErrorOutOfMemory);
-    return;
-  }
+  if (own_thread && hipSetDevice(job.device) != hipSuccess) return;  // its chunks go to the others
+  char* const slot[2] = {slots, slots + job.chunk};
   hipEvent_t ev[2] = {nullptr, nullptr};
   bool flying[2] = {false, false};
   for (auto& e : ev)
@@ -210,8 +250,8 @@ void work(Job& job, bool own_thread) {
   };
   auto send = [&](size_t k, int b) {
     const Chunk& c = ch[k];
-    hipError_t e = ToHost ? copy_chunk(slot[b].p, c.dev(), c.bytes(), hipMemcpyDeviceToHost, job.s)
-                          : copy_chunk(c.dev(), slot[b].p, c.bytes(), hipMemcpyHostToDevice, job.s);
+    hipError_t e = ToHost ? copy_chunk(slot[b], c.dev(), c.bytes(), hipMemcpyDeviceToHost, job.s)
+                          : copy_chunk(c.dev(), slot[b], c.bytes(), hipMemcpyHostToDevice, job.s);
     if (e == hipSuccess) {
       e = hipEventRecord(ev[b], job.s);
       flying[b] = e == hipSuccess;
@@ -227,7 +267,7 @@ void work(Job& job, bool own_thread) {
           const size_t n = job.next++;
           if (n < ch.size() && !send(n, 1 - b)) break;
           if (!wait(b)) break;
-          from_slot(ch[k], slot[b].p);
+          from_slot(ch[k], slot[b]);
           k = n;
           b = 1 - b;
         }
@@ -235,7 +275,7 @@ void work(Job& job, bool own_thread) {
     } else {
       for (size_t k = job.next++; k < ch.size(); k = job.next++, b = 1 - b) {
         if (!wait(b)) break;
-        into_slot(ch[k], slot[b].p);
+        into_slot(ch[k], slot[b]);
         if (!send(k, b)) break;
       }
     }
@@ -259,23 +299,27 @@ hipError_t chunked(int device, hipStream_t s, const XferPart* parts, int np, siz
   std::vector<Chunk> chunks;
   size_t moved = 0;
   for (int k = 0; k < np; k++) moved += parts[k].n * (parts[k].f32 ? sizeof(float) : sizeof(double));
-  for (int k = 0; k < np; k++) {
-    const size_t per = (moved >= kLargeTotal ? kSlotBytes : kChunkBytes) / (parts[k].f32 ? sizeof(float) : sizeof(double));
-    for (size_t i = 0; i < parts[k].n; i += per) chunks.push_back({&parts[k], i, std::min(per, parts[k].n - i)});
-  }
   Job job;
   job.device = device;
   job.s = s;
+  job.chunk = moved >= kLargeTotal ? kLargeChunkBytes : kChunkBytes;
   job.chunks = &chunks;
+  for (int k = 0; k < np; k++) {
+    const size_t per = job.chunk / (parts[k].f32 ? sizeof(float) : sizeof(double));
+    for (size_t i = 0; i < parts[k].n; i += per) chunks.push_back({&parts[k], i, std::min(per, parts[k].n - i)});
+  }
   const size_t bytes = total * sizeof(double);
-  const int nt = (int)std::min<size_t>({(size_t)host_threads(), chunks.size(), 1 + bytes / kBytesPerThread});
+  const size_t want = std::min<size_t>({(size_t)host_threads(), chunks.size(), 1 + bytes / kBytesPerThread});
+  const Block slots(want, 2 * job.chunk);  // fewer slots, fewer threads
+  if (slots.p == nullptr) return hipErrorOutOfMemory;
   std::vector<std::thread> th;
   try {
-    th.reserve(nt);
-    for (int i = 1; i < nt; i++) th.emplace_back(work<ToHost>, std::ref(job), true);
+    th.reserve(slots.count);
+    for (size_t i = 1; i < slots.count; i++)
+      th.emplace_back(work<ToHost>, std::ref(job), slots.p + 2 * i * job.chunk, true);
   } catch (...) {  // fewer threads: the ones that run take all chunks
   }
-  work<ToHost>(job, false);
+  work<ToHost>(job, slots.p, false);
   for (auto& t : th) t.join();
   return (hipError_t)job.err.load();
 }
@@ -314,18 +358,21 @@ void xfer_retain() {
   std::lock_guard<std::mutex> lock(g_mu);
   g_users++;
   try {
-    g_free.reserve(kKeepSlots);
+    g_free.reserve(kKeepBlocks);
   } catch (...) {  // nothing is kept then
   }
 }
 
 void xfer_release() {
-  std::vector<void*> gone;
+  std::vector<FreeBlock> gone;
   {
     std::lock_guard<std::mutex> lock(g_mu);
-    if (--g_users == 0) gone.swap(g_free);
+    if (--g_users == 0) {
+      gone.swap(g_free);
+      g_kept = 0;
+    }
   }
-  for (void* p : gone) (void)hipHostFree(p);
+  for (const FreeBlock& f : gone) (void)hipHostFree(f.p);
 }
 
 }  // namespace emma

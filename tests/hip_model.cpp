@@ -53,9 +53,9 @@ std::vector<Stream*> streams;
 std::string meanwhile_name;
 void (*meanwhile)() = nullptr;
 
-enum Key { kFailLaunch, kHostBlocks, kDelayFlag, kCount };
+enum Key { kFailLaunch, kHostBytes, kDelayFlag, kCount };
 long keys[kCount] = {-1, -1, 0};
-long host_blocks = 0, yields = 0, stream_waits = 0;
+long host_blocks = 0, host_bytes = 0, yields = 0, stream_waits = 0;
 
 Block* block_of(const void* p, char** base) {
   auto it = blocks.upper_bound((char*)p);
@@ -68,11 +68,14 @@ Block* block_of(const void* p, char** base) {
 
 hipError_t alloc(void** p, size_t n, unsigned flags, bool host) {
   std::lock_guard<std::recursive_mutex> lock(mu);
-  if (host && keys[kHostBlocks] >= 0 && host_blocks >= keys[kHostBlocks]) return hipErrorOutOfMemory;
+  if (host && keys[kHostBytes] >= 0 && host_bytes + (long)n > keys[kHostBytes]) return hipErrorOutOfMemory;
   *p = aligned_alloc(4096, (n + 4095) / 4096 * 4096);
   memset(*p, 0, n);
   blocks[(char*)*p] = {n, flags, host};
-  host_blocks += host;
+  if (host) {
+    host_blocks++;
+    host_bytes += n;
+  }
   return hipSuccess;
 }
 
@@ -81,8 +84,11 @@ hipError_t release(void* p, bool host) {
   if (p == nullptr) return hipSuccess;
   auto it = blocks.find((char*)p);
   if (it == blocks.end() || it->second.host != host) return hipErrorInvalidValue;
+  if (host) {
+    host_blocks--;
+    host_bytes -= it->second.bytes;
+  }
   blocks.erase(it);
-  host_blocks -= host;
   free(p);
   return hipSuccess;
 }
@@ -114,6 +120,7 @@ extern "C" {
 // ---- the tests' side
 void model_set(int key, long value) { keys[key] = value; }
 long model_host_blocks() { return host_blocks; }
+long model_host_bytes() { return host_bytes; }
 long model_yields() { return yields; }
 long model_stream_waits() { return stream_waits; }
 void model_device(int d) { device = d; }

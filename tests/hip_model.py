@@ -11,7 +11,7 @@ import tempfile
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 
-FAIL_LAUNCH, HOST_BLOCKS, DELAY_FLAG = range(3)  # model_set's keys
+FAIL_LAUNCH, HOST_BYTES, DELAY_FLAG = range(3)  # model_set's keys
 PORTABLE, COHERENT, NONCOHERENT = 0x1, 0x40000000, 0x80000000  # hipHostMalloc's flags
 
 
@@ -43,6 +43,7 @@ sys.path[:0] = [{HERE!r}, {ROOT!r}]
 m = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
 m.model_launched.restype = ctypes.c_char_p
 m.model_common_flags.restype = ctypes.c_uint
+m.model_host_bytes.restype = m.model_host_blocks.restype = ctypes.c_long
 m.model_set.argtypes = [ctypes.c_int, ctypes.c_long]
 m.model_lock.argtypes = [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_uint]
 m.launched = lambda: m.model_launched().decode().split()

@@ -75,7 +75,7 @@ def test_own_page_locked_memory_is_coherent(m, rt):
     g = rt.RadGPU(_params(1, 5), rt.FP64)
     g.setup(_params(1, 5), tree, _fields(1, tree))
     g.pinned_stencil(3, 8)
-    assert m.model_host_blocks() >= 4  # the record, two slots, the batch
+    assert m.model_host_blocks() >= 3  # the record, the slots, the batch
     assert m.model_common_flags() & hm.COHERENT
 
 
@@ -220,3 +220,51 @@ def test_forked_level_after_a_failed_capture(m, rt):
             pass
         m.model_set(hm.FAIL_LAUNCH, -1)
     g.coarse_step(1.0, 1)
+
+
+# ---------------------------------------------------------------- the transfers' page-locked memory
+def _exact(F):
+    """fields that FP32 storage holds exactly"""
+    F.e[:] = 0.5
+    for k in ("fx", "fy", "fz", "src"):
+        getattr(F, k)[:] = np.float32(getattr(F, k))
+    return F
+
+
+@modelled
+def test_transfers_keep_few_bounded_blocks(m, rt):
+    """one block a transfer, 32 MiB kept at most, all of it given back with the last context"""
+    shapes = [(rt.RadGPU(_params(G, l), precision), T.uniform_tree(l), G)
+              for l, G, precision in ((6, 3, rt.FP64), (7, 3, rt.MIXED), (5, 1, rt.FP64))]
+    for g, tree, G in shapes:
+        g.load_tree(tree)
+    record = m.model_host_blocks()
+    for g, tree, G in shapes[:1] * 2 + shapes + shapes[:1]:
+        l = tree.lmin
+        F = _exact(_fields(G, tree)[l])
+        g.set(l, 0, F)
+        B = g.get(l)
+        for k in synth.Fields.NAMES:
+            assert g.precision == rt.MIXED or np.array_equal(getattr(B, k), getattr(F, k)), k
+        assert m.model_host_blocks() - record <= 2
+        assert m.model_host_bytes() <= (32 << 20) + 4096
+    for g, tree, G in shapes:
+        g.close()
+    assert m.model_host_blocks() == 0
+
+
+@modelled
+def test_transfers_with_little_page_locked_memory(m, rt):
+    """as many slots as there are, fewer threads with them"""
+    tree = T.uniform_tree(6)
+    F = _fields(1, tree)[6]
+    for free in (2 << 20, 3 << 20, 4 << 20, 9 << 20):
+        g = rt.RadGPU(_params(1, 6), rt.FP64)
+        g.load_tree(tree)
+        m.model_set(hm.HOST_BYTES, m.model_host_bytes() + free)
+        g.set(6, 0, F)
+        B = g.get(6)
+        for k in synth.Fields.NAMES:
+            assert np.array_equal(getattr(B, k), getattr(F, k)), (free, k)
+        m.model_set(hm.HOST_BYTES, -1)
+        g.close()
