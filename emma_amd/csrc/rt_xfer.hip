@@ -19,7 +19,9 @@
 
 #include <algorithm>
 #include <atomic>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -119,71 +121,7 @@ class Block {
   size_t bytes_ = 0;
 };
 
-// ---- one kernel for all arrays of a small level
-struct PackArgs {
-  int np;
-  unsigned off[kMaxXferParts + 1];  // first element of each part
-  XferPart part[kMaxXferParts];
-};
-
-template <bool ToHost>
-__global__ __launch_bounds__(256) void pack_kernel(PackArgs a, double* slot) {
-  const unsigned i = blockIdx.x * 256u + threadIdx.x;
-  if (i >= a.off[a.np]) return;
-  int k = 0;
-  while (i >= a.off[k + 1]) k++;
-  const XferPart& p = a.part[k];
-  const unsigned j = i - a.off[k];
-  if (ToHost) {
-    slot[i] = p.f32 ? (double)((const float*)p.dev)[j] : ((const double*)p.dev)[j];
-  } else {
-    const double v = slot[i];
-    if (p.f32) {
-      float f = (float)v;
-      if (v >= p.floor && (double)f < p.floor) f = p.floor_up;
-      ((float*)p.dev)[j] = f;
-    } else {
-      ((double*)p.dev)[j] = v;
-    }
-  }
-}
-
-template <bool ToHost>
-hipError_t packed(hipStream_t s, const XferPart* parts, int np, size_t total) {
-  const Block slot(1, kPackBytes);
-  if (slot.p == nullptr) return hipErrorOutOfMemory;
-  PackArgs a;
-  a.np = np;
-  a.off[0] = 0;
-  for (int k = 0; k < np; k++) {
-    a.part[k] = parts[k];
-    a.off[k + 1] = a.off[k] + (unsigned)parts[k].n;
-    if (!ToHost) memcpy((double*)slot.p + a.off[k], parts[k].host, parts[k].n * sizeof(double));
-  }
-  hipLaunchKernelGGL((pack_kernel<ToHost>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, a, (double*)slot.p);
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
-  if (e == hipSuccess && ToHost)
-    for (int k = 0; k < np; k++) memcpy(parts[k].host, (double*)slot.p + a.off[k], parts[k].n * sizeof(double));
-  return e;
-}
-
-// ---- chunks through slots
-// A chunk's copy as a kernel, 16 bytes a thread: the runtime's copies cost
-// about 35 us each on one stream whatever their size, kernels follow each
-// other within a few (128^3 cells with three groups back: 6.9 against 5.6 ms).
-__global__ __launch_bounds__(256) void copy_kernel(uint4* dst, const uint4* src, unsigned n) {
-  const unsigned i = blockIdx.x * 256u + threadIdx.x;
-  if (i < n) dst[i] = src[i];
-}
-
-hipError_t copy_chunk(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t s) {
-  if (((size_t)dst | (size_t)src | bytes) & 15) return hipMemcpyAsync(dst, src, bytes, kind, s);
-  const unsigned n = (unsigned)(bytes / 16);
-  hipLaunchKernelGGL(copy_kernel, dim3((n + 255) / 256), dim3(256), 0, s, (uint4*)dst, (const uint4*)src, n);
-  return hipGetLastError();
-}
-
+// ---- a chunk of an array, and its conversion
 struct Chunk {
   const XferPart* part;
   size_t first, n;
@@ -218,6 +156,91 @@ void into_slot(const Chunk& c, void* slot) {
   } else {
     for (size_t i = 0; i < c.n; i++) f[i] = (float)h[i];
   }
+}
+
+// ---- without page-locked memory: the runtime's copies, converted a piece at a time
+template <bool ToHost>
+hipError_t plain(hipStream_t s, const XferPart* parts, int np) {
+  std::unique_ptr<char[]> piece(new (std::nothrow) char[kChunkBytes]);
+  if (!piece) return hipErrorOutOfMemory;
+  for (int k = 0; k < np; k++) {
+    const size_t per = kChunkBytes / (parts[k].f32 ? sizeof(float) : sizeof(double));
+    for (size_t i = 0; i < parts[k].n; i += per) {
+      const Chunk c = {&parts[k], i, std::min(per, parts[k].n - i)};
+      if (!ToHost) into_slot(c, piece.get());
+      hipError_t e = ToHost ? hipMemcpyAsync(piece.get(), c.dev(), c.bytes(), hipMemcpyDeviceToHost, s)
+                            : hipMemcpyAsync(c.dev(), piece.get(), c.bytes(), hipMemcpyHostToDevice, s);
+      if (e == hipSuccess) e = hipStreamSynchronize(s);
+      if (e != hipSuccess) return e;
+      if (ToHost) from_slot(c, piece.get());
+    }
+  }
+  return hipSuccess;
+}
+
+// ---- one kernel for all arrays of a small level
+struct PackArgs {
+  int np;
+  unsigned off[kMaxXferParts + 1];  // first element of each part
+  XferPart part[kMaxXferParts];
+};
+
+template <bool ToHost>
+__global__ __launch_bounds__(256) void pack_kernel(PackArgs a, double* slot) {
+  const unsigned i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= a.off[a.np]) return;
+  int k = 0;
+  while (i >= a.off[k + 1]) k++;
+  const XferPart& p = a.part[k];
+  const unsigned j = i - a.off[k];
+  if (ToHost) {
+    slot[i] = p.f32 ? (double)((const float*)p.dev)[j] : ((const double*)p.dev)[j];
+  } else {
+    const double v = slot[i];
+    if (p.f32) {
+      float f = (float)v;
+      if (v >= p.floor && (double)f < p.floor) f = p.floor_up;
+      ((float*)p.dev)[j] = f;
+    } else {
+      ((double*)p.dev)[j] = v;
+    }
+  }
+}
+
+template <bool ToHost>
+hipError_t packed(hipStream_t s, const XferPart* parts, int np, size_t total) {
+  const Block slot(1, kPackBytes);
+  if (slot.p == nullptr) return plain<ToHost>(s, parts, np);
+  PackArgs a;
+  a.np = np;
+  a.off[0] = 0;
+  for (int k = 0; k < np; k++) {
+    a.part[k] = parts[k];
+    a.off[k + 1] = a.off[k] + (unsigned)parts[k].n;
+    if (!ToHost) memcpy((double*)slot.p + a.off[k], parts[k].host, parts[k].n * sizeof(double));
+  }
+  hipLaunchKernelGGL((pack_kernel<ToHost>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, a, (double*)slot.p);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  if (e == hipSuccess && ToHost)
+    for (int k = 0; k < np; k++) memcpy(parts[k].host, (double*)slot.p + a.off[k], parts[k].n * sizeof(double));
+  return e;
+}
+
+// ---- chunks through slots
+// A chunk's copy as a kernel, 16 bytes a thread: the runtime's copies cost
+// about 35 us each on one stream whatever their size, kernels follow each
+// other within a few (128^3 cells with three groups back: 6.9 against 5.6 ms).
+__global__ __launch_bounds__(256) void copy_kernel(uint4* dst, const uint4* src, unsigned n) {
+  const unsigned i = blockIdx.x * 256u + threadIdx.x;
+  if (i < n) dst[i] = src[i];
+}
+
+hipError_t copy_chunk(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t s) {
+  if (((size_t)dst | (size_t)src | bytes) & 15) return hipMemcpyAsync(dst, src, bytes, kind, s);
+  const unsigned n = (unsigned)(bytes / 16);
+  hipLaunchKernelGGL(copy_kernel, dim3((n + 255) / 256), dim3(256), 0, s, (uint4*)dst, (const uint4*)src, n);
+  return hipGetLastError();
 }
 
 struct Job {
@@ -311,7 +334,7 @@ hipError_t chunked(int device, hipStream_t s, const XferPart* parts, int np, siz
   const size_t bytes = total * sizeof(double);
   const size_t want = std::min<size_t>({(size_t)host_threads(), chunks.size(), 1 + bytes / kBytesPerThread});
   const Block slots(want, 2 * job.chunk);  // fewer slots, fewer threads
-  if (slots.p == nullptr) return hipErrorOutOfMemory;
+  if (slots.p == nullptr) return plain<ToHost>(s, parts, np);
   std::vector<std::thread> th;
   try {
     th.reserve(slots.count);

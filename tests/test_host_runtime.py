@@ -268,3 +268,21 @@ def test_transfers_with_little_page_locked_memory(m, rt):
             assert np.array_equal(getattr(B, k), getattr(F, k)), (free, k)
         m.model_set(hm.HOST_BYTES, -1)
         g.close()
+
+
+@modelled
+def test_transfers_without_page_locked_memory(m, rt):
+    """the runtime's copies serve, converted on the host"""
+    for l in (3, 6):
+        tree = T.uniform_tree(l)
+        F = _exact(_fields(1, tree)[l])
+        for precision in (rt.FP64, rt.MIXED):
+            g = rt.RadGPU(_params(1, l), precision)
+            g.load_tree(tree)
+            m.model_set(hm.HOST_BYTES, 0)
+            g.set(l, 0, F)
+            B = g.get(l)
+            for k in synth.Fields.NAMES:
+                assert np.array_equal(getattr(B, k), getattr(F, k)), (l, precision, k)
+            m.model_set(hm.HOST_BYTES, -1)
+            g.close()
