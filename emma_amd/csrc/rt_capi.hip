@@ -15,6 +15,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "emma_rt.h"
@@ -1132,9 +1133,13 @@ static hipError_t queue_call_end(emma_rt_ctx* c) {
 }
 
 // Wait for the call's record.  Its flag arrives with the record, some
-// microseconds before the runtime reports the stream idle; past a short wait
-// (long calls, or a failed one) the runtime's own wait takes over.
+// microseconds before the runtime reports the stream idle.  The first kSpin
+// cover the small calls; then the core is offered to others between looks
+// (ranks that share it, the record's own rank among them), and past kPoll, in
+// long calls or a failed one, the runtime's own wait takes over.
 static int wait_call(emma_rt_ctx* c) {
+  using std::chrono::microseconds;
+  constexpr microseconds kSpin(50), kPoll(2000);
   if (!c->timing) {
     const auto t0 = std::chrono::steady_clock::now();
     for (;;) {
@@ -1142,7 +1147,9 @@ static int wait_call(emma_rt_ctx* c) {
         if (__atomic_load_n(&c->h_call->flag, __ATOMIC_ACQUIRE) != 0) return EMMA_RT_OK;
         __builtin_ia32_pause();
       }
-      if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) break;
+      const auto waited = std::chrono::steady_clock::now() - t0;
+      if (waited > kPoll) break;
+      if (waited > kSpin) std::this_thread::yield();
     }
   }
   HIPCHK(hipStreamSynchronize(c->stream));

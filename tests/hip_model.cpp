@@ -22,6 +22,8 @@
 #include <thread>
 #include <vector>
 
+#include <time.h>
+
 namespace {
 
 struct Block {
@@ -55,7 +57,8 @@ void (*meanwhile)() = nullptr;
 
 enum Key { kFailLaunch, kHostBytes, kDelayFlag, kCount };
 long keys[kCount] = {-1, -1, 0};
-long host_blocks = 0, host_bytes = 0, yields = 0, stream_waits = 0;
+std::atomic<int> pending{0};       // reports on their way
+long host_blocks = 0, host_bytes = 0, stream_waits = 0;
 
 Block* block_of(const void* p, char** base) {
   auto it = blocks.upper_bound((char*)p);
@@ -105,9 +108,14 @@ void report(void* rec) {
     __atomic_store_n(&((Record*)rec)->flag, 1, __ATOMIC_RELEASE);
   };
   if (keys[kDelayFlag] == 0) return set();
-  std::thread([set] {
-    std::this_thread::sleep_for(std::chrono::microseconds(keys[kDelayFlag]));
+  pending++;
+  std::thread([set] {  // a worker that needs its share of a core for it
+    timespec t;
+    do {
+      clock_gettime(CLOCK_THREAD_CPUTIME_ID, &t);
+    } while (t.tv_sec * 1000000L + t.tv_nsec / 1000 < keys[kDelayFlag]);
     set();
+    pending--;
   }).detach();
 }
 
@@ -121,7 +129,6 @@ extern "C" {
 void model_set(int key, long value) { keys[key] = value; }
 long model_host_blocks() { return host_blocks; }
 long model_host_bytes() { return host_bytes; }
-long model_yields() { return yields; }
 long model_stream_waits() { return stream_waits; }
 void model_device(int d) { device = d; }
 int model_current() { return device; }
@@ -143,11 +150,6 @@ unsigned model_common_flags() {
 void model_lock(void* p, size_t n, unsigned flags) {
   std::lock_guard<std::recursive_mutex> lock(mu);
   blocks[(char*)p] = {n, flags, true};
-}
-
-int sched_yield() {
-  yields++;
-  return 0;
 }
 
 // ---- devices and errors
@@ -218,7 +220,7 @@ hipError_t hipStreamDestroy(hipStream_t s) {
 hipError_t hipStreamSynchronize(hipStream_t s) {
   stream_waits++;
   if (unusable((Stream*)s)) return hipErrorStreamCaptureInvalidated;
-  if (keys[kDelayFlag] > 0) std::this_thread::sleep_for(std::chrono::microseconds(2 * keys[kDelayFlag]));
+  while (pending > 0) std::this_thread::sleep_for(std::chrono::microseconds(50));
   return hipSuccess;
 }
 static hipError_t event(hipEvent_t* e) { return *e = (hipEvent_t) new Event{device}, hipSuccess; }

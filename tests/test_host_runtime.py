@@ -1,6 +1,7 @@
 """The library's host code against a host model of the HIP runtime."""
 import ctypes
 import dataclasses
+import os
 
 import numpy as np
 
@@ -286,3 +287,21 @@ def test_transfers_without_page_locked_memory(m, rt):
                 assert np.array_equal(getattr(B, k), getattr(F, k)), (l, precision, k)
             m.model_set(hm.HOST_BYTES, -1)
             g.close()
+
+
+# ---------------------------------------------------------------- the wait for a call
+@modelled
+def test_wait_gives_way(m, rt):
+    """a call's wait shares its core with whoever the call waits for"""
+    os.sched_setaffinity(0, {min(os.sched_getaffinity(0))})
+    tree = T.uniform_tree(3)
+    p = _params(1, 3)
+    g = rt.RadGPU(p, rt.FP64)
+    g.setup(p, tree, _fields(1, tree))
+    m.model_set(hm.DELAY_FLAG, 800)
+    polled = 0
+    for _ in range(20):
+        before = m.model_stream_waits()
+        g.radsolver(3, p.dt_rad(3))
+        polled += m.model_stream_waits() == before
+    assert polled >= 15, polled
