@@ -15,6 +15,20 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an MI355X (runs the HIP library)")
 
 
+def pytest_collection_modifyitems(items):
+    """The grid dump is compared with the reference's own writer, built from the
+    reference's sources.  Without that build there is nothing to compare with:
+    skipped like the other comparisons of that kind, so that the tests after it
+    run."""
+    from oracle import ref_io_available
+
+    if ref_io_available(3):
+        return
+    for item in items:
+        if item.name.startswith("test_dump_matches_reference_writer"):
+            item.add_marker(pytest.mark.skip(reason="reference io build (oracle/_ref) not present"))
+
+
 @pytest.fixture(scope="session")
 def oracle():
     from oracle import Oracle
