@@ -2197,7 +2197,7 @@ extern "C" int emma_rt_destroy_pinned_stencil(void* stencil) {
 
 // the device address of page-locked host memory [h, h + bytes), null where the
 // range is not within one allocation of it (locked ends say nothing about what
-// lies between); coherent: allocated with hipHostMallocCoherent, so that the
+// lies between) or is locked for reading only; coherent: allocated with hipHostMallocCoherent, so that the
 // host reads a finished kernel's stores without a synchronisation
 static void* mapped_host(char* h, size_t bytes, bool* coherent) {
   hipPointerAttribute_t a;
@@ -2214,6 +2214,7 @@ static void* mapped_host(char* h, size_t bytes, bool* coherent) {
     (void)hipGetLastError();
     flags = 0;
   }
+  if (flags & hipHostRegisterReadOnly) return nullptr;
   *coherent = (flags & hipHostMallocCoherent) != 0;
   return a.devicePointer;
 }

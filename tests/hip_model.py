@@ -13,6 +13,7 @@ ROOT = os.path.dirname(HERE)
 
 FAIL_LAUNCH, HOST_BYTES, DELAY_FLAG = range(3)  # model_set's keys
 PORTABLE, COHERENT, NONCOHERENT = 0x1, 0x40000000, 0x80000000  # hipHostMalloc's flags
+REGISTER_READ_ONLY = 0x8  # of hipHostRegister's
 
 
 @functools.lru_cache(maxsize=1)

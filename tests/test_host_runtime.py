@@ -94,6 +94,17 @@ def test_batch_between_locked_ranges_is_copied(m, rt):
 
 
 @modelled
+def test_batch_locked_for_reading_is_copied(m, rt):
+    """a kernel may not write there"""
+    g, advance = _stencil_context(rt, 5)
+    raw, st = _batch(5)
+    m.model_lock(raw.ctypes.data, raw.nbytes, hm.REGISTER_READ_ONLY)
+    advance(st)
+    assert not any("stencil_direct_kernel" in k for k in m.launched())
+    assert any("stencil_kernel" in k for k in m.launched())
+
+
+@modelled
 def test_misaligned_batch_is_copied(m, rt):
     g, advance = _stencil_context(rt, 5)
     raw, st = _batch(5, align=8)
