@@ -8,7 +8,9 @@
 // residual correction without the scaling give the same correctly rounded
 // quotient (operands and quotient within 2^-900 .. 2^900), and quotients by one
 // divisor share its reciprocal.  div64 keeps the hardware's patch of the special
-// cases: zeros, infinities and NaN divide as in IEEE arithmetic.  quot64 leaves
+// cases: zeros, infinities and NaN divide as in IEEE arithmetic (64^3 cells with
+// one group: 22.5 us a level step, 22.0 without the patch, 23.2 to 23.9 with
+// plain divisions behind a test for NaN in its place).  quot64 leaves
 // that out, for operands known to be ordinary or with a check of the result: a
 // zero, infinite or denormal divisor, or an infinite numerator, gives NaN.
 // Powers: the

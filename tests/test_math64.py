@@ -1,5 +1,5 @@
 """The FP64 path's divisions, logarithm and exponential (rt_math64.h), its rate
-fits and its closure (rt_physics.h), compiled for the host, against IEEE
+fits, closure and chemistry (rt_physics.h), compiled for the host, against IEEE
 division and 50-digit arithmetic.  The hardware's reciprocal estimate is
 modelled with its largest error either way."""
 import ctypes
@@ -11,6 +11,8 @@ from decimal import Decimal, getcontext
 import numpy as np
 import pytest
 
+from emma_amd.params import ATOMIC_TABLES, RunParams, static_units
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(HERE), "emma_amd", "csrc")
 EPS = 2.0**-53  # half a unit in the last place of 1
@@ -19,16 +21,26 @@ INF, NAN, TINY = np.inf, np.nan, 5e-324
 getcontext().prec = 50
 
 
-@pytest.fixture(scope="module", params=[0.0, 2.0**-23, -(2.0**-23)], ids=["exact", "high", "low"])
-def lib(request, tmp_path_factory):
-    out = str(tmp_path_factory.mktemp("math64") / "libmath64.so")
-    subprocess.run(["g++", "-O1", "-std=c++17", "-ffp-contract=off", "-fPIC", "-shared", "-w",
+def _build(folder, *flags):
+    out = str(folder / "libmath64.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-ffp-contract=off", "-fPIC", "-shared", "-w", *flags,
                     "-I", os.path.join(HERE, "host_device"), "-I", CSRC, os.path.join(HERE, "math64_host.cpp"), "-o", out],
                    check=True)
     L = ctypes.CDLL(out)
     L.set_rcp_error.argtypes = [ctypes.c_double]
+    return L
+
+
+@pytest.fixture(scope="module", params=[0.0, 2.0**-23, -(2.0**-23)], ids=["exact", "high", "low"])
+def lib(request, tmp_path_factory):
+    L = _build(tmp_path_factory.mktemp("math64"))
     L.set_rcp_error(request.param)
     return L
+
+
+@pytest.fixture(scope="module")
+def plain(tmp_path_factory):
+    return _build(tmp_path_factory.mktemp("plain"), "-DPLAIN_DIVISION")
 
 
 def _p(a):
@@ -163,3 +175,44 @@ def test_rates(lib):
             # below the smallest normal number, a rounding is half of 2^-1074
             bound = w * D((14 + 2 * arg) * EPS) + D(4 * 2.0**-1074)
             assert abs(D(float(g)) - w) <= bound, (float(t), float(g), float(w))
+
+
+def _chem(L, u, dt, chemonly, params):
+    out = np.empty_like(u)
+    unit = np.array([params.unit_l, params.unit_t, params.unit_N, params.unit_n, params.unit_d, params.unit_v])
+    heat = [params.alphae[g] * params.hnu[g] - params.alphai[g] * 13.6 * 1.6022e-19 for g in range(2)]
+    group = np.array([[params.alphai[g], heat[g], params.factgrp[g]] for g in range(2)])
+    L.chem_all(len(u), _p(u), ctypes.c_double(dt), int(chemonly), _p(unit), _p(group), _p(out))
+    return out
+
+
+@pytest.mark.parametrize("chemonly", [False, True])
+def test_chemistry_is_that_of_plain_division(lib, plain, chemonly):
+    """every output, the status and the sub-steps, bit for bit: ordinary cells, and cells with one value
+    that is zero, infinite, NaN or next to the smallest double (a hydrogen density below the normal numbers
+    aside, whose quotients div64 does not promise)"""
+    params = RunParams.from_table(ATOMIC_TABLES["Starburst99_3grpT_3grpS"][:2], 0.1, (0.0,), **static_units())
+    rng = np.random.default_rng(6)
+    n = 300
+    nh = np.exp(rng.normal(0, 1, n))
+    x = np.where(rng.random(n) < 0.3, 10.0 ** rng.uniform(-4, -2, n), 1 - 10.0 ** rng.uniform(-5, -2, n))
+    T = 10.0 ** rng.uniform(2.5, 4.5, n)
+    e = 10.0 ** rng.uniform(-3, 0, (2, n))
+    f = rng.normal(0, 0.3, (6, n)) * params.cloc() * np.repeat(e[None], 3, 0).reshape(6, n)
+    src = np.where(rng.random((2, n)) < 0.2, 10.0 ** rng.uniform(-3, 0, (2, n)), 0.0)
+    u = np.ascontiguousarray(np.concatenate([e, f, src, [x * nh, params.eint_code(nh, x, T), nh]]).T)
+    odd = []
+    for k in range(13):
+        for v in (0.0, TINY, 1e-310, 1e-300, INF, NAN, -1e-3):
+            if k == 12 and 0 < v < 1e-308:
+                continue
+            w = u[k].copy()
+            w[k] = v
+            odd.append(w)
+    for dt, rows in ((params.dt_rad(5), np.concatenate([u, odd])), (0.0, np.concatenate([u[:20], odd]))):
+        a, b = _chem(lib, rows, dt, chemonly, params), _chem(plain, rows, dt, chemonly, params)
+        bad = ~((a == b) | (np.isnan(a) & np.isnan(b))).all(axis=1)
+        # of a failed call the status counts
+        bad &= ~((a[:, 11] != 0) & (a[:, 11] == b[:, 11]))
+        assert not bad.any(), (dt, int(bad.sum()), rows[bad][:2], a[bad][:2], b[bad][:2])
+        assert (a[: min(len(u), len(rows) - len(odd)), 11] == 0).all() or chemonly
