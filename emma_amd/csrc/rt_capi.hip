@@ -547,20 +547,30 @@ static int morton_cube(int noct, const int* nei) {
 //     chains, 874 -> 793), 1.56e4 173 -> 169, 1.6e4 155 -> 147; 1.86e4 FP64 G=3
 //     896 -> 888; 2.1e4 FP64 G=2 1197 -> 1125; 3.1e4 FP64 G=1 227 -> 202, mixed
 //     G=4 312 -> 306; 6.3e4 mixed G=1 643 -> 635; 6.4e4 mixed G=9 1269 -> 1225.
+// Fewer do, about twice the tiles the chip holds at once, where the finer launches
+// are so small that they leave it idle for kForkIdle tiles' time: mixed G=3, tiles
+// and idle tiles, 2,965 and 4,112 519 -> 495 us, 3,373 and 20,880 893 -> 871,
+// 2,224 and 9,470 503 -> 498, 1,950 and 8,540 575 -> 553, but 2,684 and 2,700
+// 584 -> 616, 2,170 and 2,484 377 -> 383, 1,799 and 4,512 436 -> 447,
+// 1,387 and 22,430 823 -> 851; FP64 G=1 2,965 and 4,112 650 -> 634, 1,799 and 4,512
+// 559 -> 596.  (Not the lightest tiles: mixed G=1, 7,136 and 17,160 379 -> 395.)
 // And the finer launches have to take at least a quarter as long as the free
 // tiles.  A launch of few tiles takes as long as about 800 (12 us).  Where they
 // take longer than the free tiles (2), the three-group mixed tiles, whose LDS
-// allows it, leave room for them (five-level tree: 543 us, 534 with 1, 527 with
-// 2; with level 8's 2,170 free tiles forked too 557).
-constexpr int kForkWork = 14000, kLaunchTiles = 800;
+// allows it, leave room for them (five-level tree: 541 us, 530 with 1, 523 with 2).
+constexpr int kForkWork = 14000, kForkTiles = 1900, kForkIdle = 4000, kLaunchTiles = 800;
 static int tile_work(int ng, bool fp64) { return fp64 ? 4 * ng : ng == 3 ? 2 : ng < 3 ? 1 : ng; }
 static int fork_kind(const std::vector<DevLevel>& lev, int k, int ng, bool fp64) {
   const DevLevel& L = lev[k];
-  if ((long long)L.nfree * tile_work(ng, fp64) < kForkWork) return 0;
-  long long finer = 0;
-  for (size_t j = k + 1; j < lev.size() && lev[j].noct > 0; j++)
-    finer += (long long)std::max(kLaunchTiles, (lev[j].ncell + kTileCells - 1) / kTileCells) << std::min<size_t>(j - k, 20);
-  return 4 * finer < L.nfree ? 0 : finer < L.nfree ? 1 : 2;
+  long long finer = 0, idle = 0;
+  for (size_t j = k + 1; j < lev.size() && lev[j].noct > 0; j++) {
+    const int tiles = (lev[j].ncell + kTileCells - 1) / kTileCells, steps = 1 << std::min<size_t>(j - k, 20);
+    finer += (long long)std::max(kLaunchTiles, tiles) * steps;
+    idle += (long long)std::max(0, kLaunchTiles - tiles) * steps;
+  }
+  const int work = tile_work(ng, fp64);
+  const bool worth = (long long)L.nfree * work >= kForkWork || (work > 1 && L.nfree >= kForkTiles && idle >= kForkIdle);
+  return !worth || 4 * finer < L.nfree ? 0 : finer < L.nfree ? 1 : 2;
 }
 
 extern "C" int emma_rt_tree_create(emma_rt_ctx* c, int lmin, int lmax, const int* noct, const int* nei_oct,

@@ -1,11 +1,16 @@
 // rt_kernels.hip -- gfx950 kernels of the resident-level radiation step.
 //
 // One level step (the work of advancerad + RadSolver's final update for one
-// level, rad_utils.c:1775-2006) is ONE kernel: a thread per cell reads its
-// own state and its six face neighbours straight from the level's SoA arrays
-// through the oct index tables (no stencil copy), forms the Lax-Friedrichs
-// M1 fluxes, updates, runs the chemistry sub-stepper in FP64 and writes the
-// next state; split cells write the mean of their children instead.  State is
+// level, rad_utils.c:1775-2006): a thread per cell reads its own state and its
+// neighbours' through the oct index tables of the level's SoA arrays (no
+// stencil copy; neighbours in the same tile through LDS), forms the
+// Lax-Friedrichs M1 fluxes, updates, runs the chemistry sub-stepper in FP64 and
+// writes the next state; split cells write the mean of their children instead.
+// One kernel (level_step_kernel, level_step_tiled, level_step_split, with the
+// straggler pass behind the tiled ones), or two where several groups' chemistry
+// would hold the transport's registers (transport_kernel, chemistry_kernel);
+// cell_step, with neighbours straight from memory, is the persistent kernel's
+// per-cell form.  State is
 // double-buffered (read A, write B), so the reference's rfieldnew copy
 // (clean_new_rad) disappears; coarse-fine refluxes go to small per-level
 // accumulators that the coarser level folds in on its next step.

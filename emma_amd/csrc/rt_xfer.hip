@@ -7,11 +7,10 @@
 // against 3.4 ms for their 193 MB over PCIe at the 57 GB/s that page-locked
 // memory reaches.  So the arrays cross in their device type, in chunks through
 // page-locked slots, and several host threads convert them (and take the page
-// faults) side by side while the next chunks are in flight: 5.6 ms (4.8 to
-// 6.0 ms for the way in, 22.5 ms before).  Up to one slot's
-// worth of doubles, where the nine copies' latency is what counts, one kernel
-// gathers all arrays, converted, straight into a slot (or scatters them from
-// it).
+// faults) side by side while the next chunks are in flight: 4.8 to 5.8 ms (5.5 ms
+// for the way in, 22.5 before).  Up to a MiB of doubles, where the nine copies'
+// latency is what counts, one kernel gathers all arrays, converted, straight into
+// a slot (or scatters them from it).
 #include <hip/hip_runtime.h>
 
 #include <sched.h>
@@ -230,7 +229,8 @@ hipError_t packed(hipStream_t s, const XferPart* parts, int np, size_t total) {
 // ---- chunks through slots
 // A chunk's copy as a kernel, 16 bytes a thread: the runtime's copies cost
 // about 35 us each on one stream whatever their size, kernels follow each
-// other within a few (128^3 cells with three groups back: 6.9 against 5.6 ms).
+// other within a few (128^3 cells with three groups back, 1 MiB chunks: 6.9
+// against 5.6 ms).
 __global__ __launch_bounds__(256) void copy_kernel(uint4* dst, const uint4* src, unsigned n) {
   const unsigned i = blockIdx.x * 256u + threadIdx.x;
   if (i < n) dst[i] = src[i];

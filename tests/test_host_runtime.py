@@ -172,21 +172,23 @@ def test_coarse_step_from_a_thread_on_another_device(m, rt):
 # ---------------------------------------------------------------- forked levels
 @modelled
 def test_levels_that_fork(m, rt):
-    """a level forks where its free tiles are worth it: large levels, and by family (two launches of the forked
-    level in a captured coarse step)"""
+    """a level forks where its free tiles are worth it: large levels, by family, and middling ones beside launches
+    that leave the chip idle (two launches of each forked level step in a captured coarse step)"""
     rng = np.random.default_rng(97)
     sampler = synth.lognormal_sampler(synth.gaussian_field(32, rng), 1.0)
     small, large = T.amr_tree(6, [40000, 3000], sampler, rng), T.amr_tree(7, [4000, 1500], sampler, rng)
+    deep = T.amr_tree(7, [80000, 20000, 3000, 400], sampler, rng)
     kernel = {(1, rt.FP64): "level_step_kernel", (3, rt.FP64): "transport_kernel"}
     for tree, G, precision, forks in ((small, 1, rt.MIXED, 0), (small, 3, rt.MIXED, 0), (small, 1, rt.FP64, 0),
                                       (large, 1, rt.MIXED, 0), (large, 3, rt.MIXED, 1), (large, 1, rt.FP64, 1),
-                                      (large, 3, rt.FP64, 1)):
+                                      (large, 3, rt.FP64, 1), (deep, 1, rt.MIXED, 0), (deep, 3, rt.MIXED, 1 + 2)):
         g = rt.RadGPU(_params(G, tree.lmin), precision)
         g.setup(_params(G, tree.lmin), tree, {})
         m.model_forget()
         g.coarse_step(1.0, 1)
         name = kernel.get((G, precision), "level_step_")
-        assert sum(name in k for k in m.launched()) == 7 + forks, (tree.lmin, G, precision, m.launched())
+        steps = 2 ** len(tree.levels) - 1
+        assert sum(name in k for k in m.launched()) == steps + forks, (tree.lmin, G, precision, m.launched())
         g.close()
 
 

@@ -59,10 +59,12 @@ def _same(x, y):
 
 
 def test_division_is_correctly_rounded(lib):
-    """operands of any sign within 2^-450 .. 2^450"""
+    """operands and quotients of any sign within 2^-900 .. 2^900"""
     rng = np.random.default_rng(1)
     n = 400000
-    a, b = (np.ldexp(rng.uniform(1, 2, n) * rng.choice([-1.0, 1.0], n), rng.integers(-450, 450, n)) for _ in range(2))
+    ka, kb = rng.integers(-899, 899, n), rng.integers(-899, 899, n)
+    kb = np.where(np.abs(ka - kb) < 898, kb, ka)
+    a, b = (np.ldexp(rng.uniform(1, 2, n) * rng.choice([-1.0, 1.0], n), k) for k in (ka, kb))
     near = np.nextafter(b, rng.choice([0.0, INF], n))  # quotients next to 1, and exact ones
     for x, y in ((a, b), (b, near), (b * 3, b), (b, b)):
         assert _same(_div(lib, x, y), x / y)
