@@ -167,7 +167,7 @@ int emma_rt_advance_stencil(emma_rt_ctx *ctx, void *stencil, int nread, int leve
    hipMalloc).  No counterpart in the reference.  A batch in ordinary memory is
    staged in a static device area of EMMA_RT_NOALLOC_STENCIL_BYTES per GPU (allocated with
    the library's code object, held until the process ends); the call allocates
-   nothing.  nread * sizeof(struct RGRID) beyond that size (e.g. 4128 records
+   no device or page-locked memory (a MiB of ordinary memory while it runs).  nread * sizeof(struct RGRID) beyond that size (e.g. 4128 records
    at NGRP=1, 1826 at NGRP=3, REAL=double) returns EMMA_RT_ERR_ARG.  real_bytes
    is sizeof(REAL).  Results equal emma_rt_advance_stencil's.  All calls on one
    GPU share its area: calls that overlap in time on one GPU (other host
