@@ -1136,9 +1136,11 @@ static int begin_call(emma_rt_ctx* c) {
   return EMMA_RT_OK;
 }
 
-// the call's last kernel (captured at the tail of a coarse step's graph)
+// the call's last kernel (captured at the tail of a coarse step's graph).  It is
+// one work-group and clears the list lengths this call used: their number grows
+// with the longest call there was.
 static hipError_t queue_call_end(emma_rt_ctx* c) {
-  return launch_call_end(c->d_status, c->counters ? c->d_counters : nullptr, c->d_defer_ctl, c->defer_slots, c->h_call,
+  return launch_call_end(c->d_status, c->counters ? c->d_counters : nullptr, c->d_defer_ctl, c->defer_seq, c->h_call,
                          c->stream);
 }
 

@@ -58,7 +58,7 @@ void (*meanwhile)() = nullptr;
 enum Key { kFailLaunch, kHostBytes, kDelayFlag, kCount };
 long keys[kCount] = {-1, -1, 0};
 std::atomic<int> pending{0};       // reports on their way
-long host_blocks = 0, host_bytes = 0, stream_waits = 0;
+long host_blocks = 0, host_bytes = 0, stream_waits = 0, cleared = 0;
 
 Block* block_of(const void* p, char** base) {
   auto it = blocks.upper_bound((char*)p);
@@ -130,6 +130,7 @@ void model_set(int key, long value) { keys[key] = value; }
 long model_host_blocks() { return host_blocks; }
 long model_host_bytes() { return host_bytes; }
 long model_stream_waits() { return stream_waits; }
+long model_cleared() { return cleared; }  // list lengths the last call's end cleared
 void model_device(int d) { device = d; }
 int model_current() { return device; }
 const char* model_launched() { return launched.c_str(); }
@@ -311,6 +312,7 @@ hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipSt
   if (name.find("copy_kernel") != std::string::npos) {
     memcpy(*(void**)args[0], *(void**)args[1], (size_t) * (unsigned*)args[2] * 16);
   } else if (name.find("call_end_kernel") != std::string::npos) {
+    cleared = *(int*)args[3];
     if (st->capture != 0)
       st->records.push_back(*(void**)args[4]);
     else
