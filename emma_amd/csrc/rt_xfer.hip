@@ -66,11 +66,16 @@ class Block {
   }
   ~Block() {
     if (p == nullptr) return;
-    std::vector<FreeBlock> gone;
+    FreeBlock gone[kKeepBlocks];
+    size_t n = 0;
     {
       std::lock_guard<std::mutex> lock(g_mu);
       if (g_users > 0 && bytes_ <= kKeepBytes) {
-        while (!g_free.empty() && (g_kept + bytes_ > kKeepBytes || g_free.size() == kKeepBlocks)) drop(gone, 0);
+        while (!g_free.empty() && (g_kept + bytes_ > kKeepBytes || g_free.size() == kKeepBlocks)) {
+          gone[n++] = g_free.front();
+          g_kept -= g_free.front().bytes;
+          g_free.erase(g_free.begin());
+        }
         if (g_free.size() < g_free.capacity()) {
           g_free.push_back({p, bytes_});
           g_kept += bytes_;
@@ -78,7 +83,7 @@ class Block {
         }
       }
     }
-    for (const FreeBlock& f : gone) (void)hipHostFree(f.p);
+    for (size_t i = 0; i < n; i++) (void)hipHostFree(gone[i].p);
     if (p != nullptr) (void)hipHostFree(p);
   }
   Block(const Block&) = delete;
@@ -88,11 +93,6 @@ class Block {
   size_t count = 0;   // units
 
  private:
-  static void drop(std::vector<FreeBlock>& gone, size_t i) {
-    gone.push_back(g_free[i]);
-    g_kept -= g_free[i].bytes;
-    g_free.erase(g_free.begin() + i);
-  }
   void take(size_t want) {
     {
       std::lock_guard<std::mutex> lock(g_mu);
