@@ -228,14 +228,18 @@ __global__ __launch_bounds__(64) void stencil_direct_kernel(char* base, StencilG
   R* sCell = lds;
   R* sNew = lds + S::kOcts * 32 * S::kLight;
   R* sFlux = sNew + S::kOcts * 8 * S::kRtype;
-  // several loads in flight per lane: a read over the bus takes microseconds
+  // several loads in flight per lane: a read over the bus takes microseconds.
+  // Past the end the last value again: behind a condition each load was waited
+  // for by itself in the FP32 kernels.  100 records with three FP32 groups 282 ->
+  // 215 us a call, 1501 392 -> 370; with 8 in flight 210 and 362, but then a full
+  // batch, which keeps the bus busy, takes longer (4096 records with three FP64
+  // groups 1067 -> 1094 us, 1081 with 6).
   auto fetch = [&](int count, R* to, auto&& from) {
-    constexpr int kFly = 8;
+    constexpr int kFly = 6;
     for (int i0 = lane; i0 < count; i0 += 64 * kFly) {
       R v[kFly];
 #pragma unroll
-      for (int u = 0; u < kFly; u++)
-        if (i0 + 64 * u < count) v[u] = *from(i0 + 64 * u);
+      for (int u = 0; u < kFly; u++) v[u] = *from(min(i0 + 64 * u, count - 1));
 #pragma unroll
       for (int u = 0; u < kFly; u++)
         if (i0 + 64 * u < count) to[i0 + 64 * u] = v[u];
