@@ -41,8 +41,9 @@ struct XferPart {
 constexpr int kMaxXferParts = 24;
 
 // Both wait for the work queued on the stream before and return with the copy
-// done.  Callable from several threads, whatever their current device; the staging memory is shared by all
-// callers, bounded, and released with the last xfer_release().
+// done.  Callable from several threads, whatever their current device; the
+// staging memory is shared by all callers, bounded (32 MiB), and all but 16 MiB
+// of it released with the last xfer_release().
 hipError_t xfer_to_host(int device, hipStream_t s, const XferPart* parts, int np);
 hipError_t xfer_to_device(int device, hipStream_t s, const XferPart* parts, int np);
 // a user of the staging memory comes (a context is made) and goes

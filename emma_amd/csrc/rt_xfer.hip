@@ -39,21 +39,40 @@ constexpr size_t kChunkBytes = 1u << 20, kLargeChunkBytes = 2u << 20, kLargeTota
 constexpr int kMaxThreads = 8;
 constexpr size_t kBytesPerThread = 4u << 20;  // host bytes that pay for starting a thread (0.02 to 2 ms)
 constexpr size_t kKeepBytes = 2 * kMaxThreads * kLargeChunkBytes;
+constexpr size_t kIdleBytes = 2 * kMaxThreads * kChunkBytes;
 constexpr size_t kKeepBlocks = 16;
 
 // The page-locked memory of a transfer: one block, two slots of a chunk for each
 // thread.  Freeing page-locked memory takes 0.28 ms a block whatever its size,
 // and allocating 32 MiB 2.2 ms in one block, 6 in sixteen: closing the last
 // context of a program after 64^3 cells and two finer levels, three FP64 groups,
-// takes 5.8 ms, 9.7 with sixteen slots of their own, 4.8 with none.
+// takes 5.8 ms, 9.7 with sixteen slots of their own, 4.8 with none.  The first
+// touch of fresh ones costs 0.37 ms a MiB, so that a program of many short-lived
+// contexts would pay more for its slots than they bring (32^3 cells, three FP64
+// groups, a context made, set, read and closed: 1.45 ms, 2.95 with a new block):
+// kIdleBytes stay with the process between contexts.
 struct FreeBlock {
   char* p;
   size_t bytes;
 };
 std::mutex g_mu;
-std::vector<FreeBlock> g_free;  // blocks nobody uses, kKeepBytes at most
+std::vector<FreeBlock> g_free;  // blocks nobody uses: kKeepBytes at most, kIdleBytes without a context
 size_t g_kept = 0;
 int g_users = 0;
+
+// blocks taken off the list under the lock, freed after it
+struct Gone {
+  FreeBlock b[kKeepBlocks];
+  size_t n = 0;
+  void take(size_t i) {
+    b[n++] = g_free[i];
+    g_kept -= g_free[i].bytes;
+    g_free.erase(g_free.begin() + i);
+  }
+  ~Gone() {
+    for (size_t i = 0; i < n; i++) (void)hipHostFree(b[i].p);
+  }
+};
 
 class Block {
  public:
@@ -66,24 +85,17 @@ class Block {
   }
   ~Block() {
     if (p == nullptr) return;
-    FreeBlock gone[kKeepBlocks];
-    size_t n = 0;
+    Gone gone;
     {
       std::lock_guard<std::mutex> lock(g_mu);
-      if (g_users > 0 && bytes_ <= kKeepBytes) {
-        while (!g_free.empty() && (g_kept + bytes_ > kKeepBytes || g_free.size() == kKeepBlocks)) {
-          gone[n++] = g_free.front();
-          g_kept -= g_free.front().bytes;
-          g_free.erase(g_free.begin());
-        }
-        if (g_free.size() < g_free.capacity()) {
-          g_free.push_back({p, bytes_});
-          g_kept += bytes_;
-          p = nullptr;
-        }
+      const size_t keep = g_users > 0 ? kKeepBytes : kIdleBytes;
+      if (bytes_ <= keep && g_free.capacity() >= kKeepBlocks) {
+        while (g_kept + bytes_ > keep || g_free.size() >= kKeepBlocks) gone.take(0);
+        g_free.push_back({p, bytes_});
+        g_kept += bytes_;
+        p = nullptr;
       }
     }
-    for (size_t i = 0; i < n; i++) (void)hipHostFree(gone[i].p);
     if (p != nullptr) (void)hipHostFree(p);
   }
   Block(const Block&) = delete;
@@ -387,15 +399,12 @@ void xfer_retain() {
 }
 
 void xfer_release() {
-  std::vector<FreeBlock> gone;
-  {
-    std::lock_guard<std::mutex> lock(g_mu);
-    if (--g_users == 0) {
-      gone.swap(g_free);
-      g_kept = 0;
-    }
-  }
-  for (const FreeBlock& f : gone) (void)hipHostFree(f.p);
+  Gone gone;
+  std::lock_guard<std::mutex> lock(g_mu);
+  if (--g_users > 0) return;
+  for (size_t i = g_free.size(); i-- > 0 && g_kept > kIdleBytes;)
+    if (g_free[i].bytes > kIdleBytes) gone.take(i);
+  while (g_kept > kIdleBytes) gone.take(0);
 }
 
 }  // namespace emma

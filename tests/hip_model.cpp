@@ -58,7 +58,7 @@ void (*meanwhile)() = nullptr;
 enum Key { kFailLaunch, kHostBytes, kDelayFlag, kCount };
 long keys[kCount] = {-1, -1, 0};
 std::atomic<int> pending{0};       // reports on their way
-long host_blocks = 0, host_bytes = 0, stream_waits = 0, cleared = 0;
+long host_blocks = 0, host_bytes = 0, host_allocs = 0, stream_waits = 0, cleared = 0;
 
 Block* block_of(const void* p, char** base) {
   auto it = blocks.upper_bound((char*)p);
@@ -77,6 +77,7 @@ hipError_t alloc(void** p, size_t n, unsigned flags, bool host) {
   blocks[(char*)*p] = {n, flags, host};
   if (host) {
     host_blocks++;
+    host_allocs++;
     host_bytes += n;
   }
   return hipSuccess;
@@ -129,6 +130,7 @@ extern "C" {
 void model_set(int key, long value) { keys[key] = value; }
 long model_host_blocks() { return host_blocks; }
 long model_host_bytes() { return host_bytes; }
+long model_host_allocs() { return host_allocs; }
 long model_stream_waits() { return stream_waits; }
 long model_cleared() { return cleared; }  // list lengths the last call's end cleared
 void model_device(int d) { device = d; }

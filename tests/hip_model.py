@@ -44,7 +44,7 @@ sys.path[:0] = [{HERE!r}, {ROOT!r}]
 m = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
 m.model_launched.restype = ctypes.c_char_p
 m.model_common_flags.restype = ctypes.c_uint
-m.model_host_bytes.restype = m.model_host_blocks.restype = ctypes.c_long
+m.model_host_bytes.restype = m.model_host_blocks.restype = m.model_host_allocs.restype = ctypes.c_long
 m.model_set.argtypes = [ctypes.c_int, ctypes.c_long]
 m.model_lock.argtypes = [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_uint]
 m.launched = lambda: m.model_launched().decode().split()
