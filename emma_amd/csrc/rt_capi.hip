@@ -1147,8 +1147,8 @@ static hipError_t queue_call_end(emma_rt_ctx* c) {
 // Wait for the call's record.  Its flag arrives with the record, some
 // microseconds before the runtime reports the stream idle.  The first kSpin
 // cover the small calls; then the core is offered to others between looks
-// (ranks that share it, the record's own rank among them), and past kPoll, in
-// long calls or a failed one, the runtime's own wait takes over.
+// (ranks that share it), and past kPoll, in long calls or a failed one, the
+// runtime's own wait takes over.
 static int wait_call(emma_rt_ctx* c) {
   using std::chrono::microseconds;
   constexpr microseconds kSpin(50), kPoll(2000);
@@ -2209,8 +2209,9 @@ extern "C" int emma_rt_destroy_pinned_stencil(void* stencil) {
 
 // the device address of page-locked host memory [h, h + bytes), null where the
 // range is not within one allocation of it (locked ends say nothing about what
-// lies between) or is locked for reading only; coherent: allocated with hipHostMallocCoherent, so that the
-// host reads a finished kernel's stores without a synchronisation
+// lies between) or is locked for reading only; coherent: allocated with
+// hipHostMallocCoherent, so that the host reads a finished kernel's stores
+// without a synchronisation
 static void* mapped_host(char* h, size_t bytes, bool* coherent) {
   hipPointerAttribute_t a;
   hipDeviceptr_t base = nullptr;

@@ -391,7 +391,15 @@ hipError_t xfer_to_device(int device, hipStream_t s, const XferPart* parts, int 
 
 void xfer_retain() {
   std::lock_guard<std::mutex> lock(g_mu);
-  g_users++;
+  if (g_users++ > 0) return;
+  // a device reset between contexts takes the blocks with it
+  for (size_t i = g_free.size(); i-- > 0;) {
+    unsigned flags = 0;
+    if (hipHostGetFlags(&flags, g_free[i].p) == hipSuccess) continue;
+    (void)hipGetLastError();
+    g_kept -= g_free[i].bytes;
+    g_free.erase(g_free.begin() + i);
+  }
   try {
     g_free.reserve(kKeepBlocks);
   } catch (...) {  // nothing is kept then

@@ -137,6 +137,11 @@ void model_device(int d) { device = d; }
 int model_current() { return device; }
 const char* model_launched() { return launched.c_str(); }
 void model_forget() { launched.clear(); }
+// what a device reset does: no block is known any more
+void model_reset() {
+  blocks.clear();
+  host_blocks = host_bytes = 0;
+}
 // called when a kernel of that name is launched: what another thread does meanwhile
 void model_during(const char* name, void (*f)()) {
   meanwhile_name = name;

@@ -279,6 +279,13 @@ def test_short_lived_contexts_share_their_blocks(m, rt):
         g.close()
         allocs.append(m.model_host_allocs())
     assert np.array_equal(np.diff(allocs), [1, 1, 1]), allocs  # the call record alone
+    m.model_reset()  # of the device: new blocks, and none of the old ones freed
+    g = rt.RadGPU(_params(3, 5), rt.FP64)
+    g.setup(_params(3, 5), tree, F)
+    assert m.model_host_allocs() == allocs[-1] + 2
+    for k in synth.Fields.NAMES:
+        assert np.array_equal(getattr(g.get(5), k), getattr(F[5], k)), k
+    g.close()
 
 
 @modelled
